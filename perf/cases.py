@@ -204,12 +204,10 @@ def _prepare_engine(case, seed):
             passes = [eng.upward_pass, eng.downward_pass]
         keep = (fmm, tree)
     q = torch.from_numpy(np.concatenate([p[1] for p in probs])).cuda()
-    back = np.empty(len(trg), np.int64)
-    back[trg] = np.arange(len(trg))  # sorted position of the user's i-th target
     width = 8 if case["kernel"] == "helmholtz" else 4
     values = torch.as_tensor(_Device(eng.values_device_ptr(), (len(trg), width)), device="cuda")
     return {"engine": eng, "passes": passes, "q": q, "src": torch.from_numpy(src.astype(np.int64)).cuda(),
-            "back": torch.from_numpy(back).cuda(), "values": values, "keep": keep, "single": case["precision"] != "fp64",
+            "trg": torch.from_numpy(trg.astype(np.int64)).cuda(), "values": values, "keep": keep, "single": case["precision"] != "fp64",
             "complex": width == 8}
 
 
@@ -220,9 +218,8 @@ def _run_engine(s):
     for step in s["passes"]:
         step()
     s["engine"].synchronize()
-    v = s["values"].index_select(0, s["back"])
-    if s["single"]:
-        v = v.float()
+    v = s["values"].float() if s["single"] else s["values"]
+    v = torch.empty_like(v).index_copy_(0, s["trg"], v)  # the tree's order -> the user's
     return torch.view_as_complex(v.view(-1, 4, 2)) if s["complex"] else v
 
 
