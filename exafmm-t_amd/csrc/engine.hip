@@ -110,9 +110,12 @@ struct xfmm_context {
   // ---- operators
   bool have_ops = false;
   int nlevels = 0, nm2l = 0;
+  // packed operands of the translation GEMMs (launch_gemm_pack), one slot of
+  // op_stride entries per operator level, in FP64 and, for the stages that
+  // run in FP32, in FP32
   DevBuf<double> uc2e_uT, uc2e_vT, dc2e_uT, dc2e_vT, m2mcat, l2lcat;
   // numerical rank of the upward / downward pseudo-inverse per operator level
-  // (uc2e_uT / dc2e_uT hold only the first r_up / r_dn columns, row stride r)
+  // (uc2e_uT / dc2e_uT hold only the first r_up / r_dn columns)
   std::vector<int> r_up, r_dn;
   DevBuf<float> uc2e_uT32, uc2e_vT32, dc2e_uT32, dc2e_vT32, m2mcat32, l2lcat32;  // f32_pinv / f32_trans
   DevBuf<double> m2l64;  // M2L operators in the expanded MFMA form, [L][nfreq][26][64][4]
@@ -147,7 +150,7 @@ struct xfmm_context {
   std::vector<int> blk_level_off;                         // [depth+2] block ranges per target level
   DevBuf<char> fft_in, fft_out;
   // buffers
-  DevBuf<double> up, dn, trg_value, check, tmp, gemm_scratch, near;
+  DevBuf<double> up, dn, trg_value, check, tmp, near;
   // near-coincident P2P pairs ([4] ints each) corrected in FP64 after an
   // FP32 near field
   DevBuf<int> close_pairs, close_off;
@@ -333,88 +336,99 @@ void check_ready(xfmm_context* c) {
   if (c->nm2l != 1 && c->nm2l < c->depth) throw ArgError{"xfmm: M2L operators cover fewer levels than the tree depth"};
 }
 
-// B operand of a translation GEMM: the FP32 copy for FP32 GEMMs, else the
-// FP64 operator; off = element offset.
-const void* gemm_op(bool f32, const xfmm_context* c, const DevBuf<double>& d, const DevBuf<float>& f, size_t off) {
-  (void)c;
-  if (f32) return f.ptr + off;
-  return d.ptr + off;
+// Entries between the packed operators of two levels: pseudo-inverse factors
+// (at most nsurf x nsurf) or the stacked / concatenated M2M / L2L matrices.
+// Complex operators are real 2 x 2 blocks [[Re, Im], [-Im, Re]] per entry, so
+// that a complex row-GEMM on interleaved (re, im) rows is one real GEMM with K
+// and N doubled.
+size_t pinv_stride(const xfmm_context* c, bool f32) {
+  return gemm_packed_size(f32, c->nsurf * c->vw, c->nsurf * c->vw);
+}
+size_t m2m_stride(const xfmm_context* c, bool f32) {
+  return gemm_packed_size(f32, 8 * c->nsurf * c->vw, c->nsurf * c->vw);
+}
+size_t l2l_stride(const xfmm_context* c, bool f32) {
+  return gemm_packed_size(f32, c->nsurf * c->vw, 8 * c->nsurf * c->vw);
 }
 
-// Doubles per nsurf x nsurf operator in GEMM form: complex operators are held
-// as real 2 x 2 blocks [[Re, Im], [-Im, Re]] per entry, so that a complex
-// row-GEMM on interleaved (re, im) rows is one real GEMM with K and N doubled
-// (on the FP64 matrix cores like the real kernels).
-size_t gemm_op_size(const xfmm_context* c) { return size_t(c->nsurf) * c->nsurf * c->vw * c->vw; }
+// B operand of a translation GEMM: the FP32 copy for FP32 GEMMs, else the
+// FP64 operator.
+const void* gemm_op(bool f32, const DevBuf<double>& d, const DevBuf<float>& f) {
+  if (f32) return f.ptr;
+  return d.ptr;
+}
+
+// The two products of a pseudo-inverse for the leaves of all levels, one
+// launch each: tmp = in U^T (only the first r singular directions carry a
+// nonzero S^+ entry: those r coefficients), out = leaf scale * tmp V^T.
+void pinv_products(xfmm_context* c, const std::vector<int>& rank, const double* in, const long* in_rows, bool f32,
+                   const void* u, const void* v, double* out) {
+  const int nv = c->nsurf * c->vw;
+  const size_t stride = pinv_stride(c, f32);
+  GemmGroup gu, gv;
+  for (int l = 0; l <= c->depth; l++) {
+    const int b = c->leaf_level_off[l], e = c->leaf_level_off[l + 1];
+    if (e <= b) continue;
+    const int L = c->op_level(l), r = rank[L] * c->vw;
+    GemmSeg sg;
+    sg.row0 = b;
+    sg.m = e - b;
+    sg.n = r;
+    sg.k = nv;
+    sg.boff = L * stride;
+    gu.seg[gu.nseg++] = sg;
+    sg.n = nv;
+    sg.k = r;
+    sg.alpha = c->leaf_scale(l);
+    gv.seg[gv.nseg++] = sg;
+  }
+  launch_gemm_rows(f32, gu, in, in_rows, u, c->tmp.ptr, c->leaf_slot_rows.ptr, 0, c->stream);
+  launch_gemm_rows(f32, gv, c->tmp.ptr, c->leaf_slot_rows.ptr, v, out, c->leaf_node_rows.ptr, 0, c->stream);
+}
 
 void op_P2M(xfmm_context* c) {
   // check potentials of every leaf, then up = alpha * UC2E_V (UC2E_U check)
   DevTree t = c->dev_tree();
   launch_eval_surface(c->kind, c->f32_surf, MODE_P2M, t, c->wavek(), c->w_leaf.ptr, c->n_leaf, c->check.ptr,
                       c->stream);
-  const size_t ns2 = gemm_op_size(c);
-  const int vw = c->vw;
-  for (int l = 0; l <= c->depth; l++) {
-    const int b = c->leaf_level_off[l], e = c->leaf_level_off[l + 1];
-    if (e <= b) continue;
-    const int L = c->op_level(l);
-    // only the first r singular directions carry a nonzero S^+ entry: the
-    // first product computes those r coefficients, the second sums over them
-    const int r = c->r_up[L];
-    launch_gemm_rows(c->f32_pinv, e - b, r * vw, c->nsurf * vw, c->check.ptr, c->leaf_slot_rows.ptr + b,
-                     gemm_op(c->f32_pinv, c, c->uc2e_uT, c->uc2e_uT32, L * ns2), c->tmp.ptr, c->leaf_slot_rows.ptr + b,
-                     1.0, 0, c->stream);
-    launch_gemm_rows(c->f32_pinv, e - b, c->nsurf * vw, r * vw, c->tmp.ptr, c->leaf_slot_rows.ptr + b,
-                     gemm_op(c->f32_pinv, c, c->uc2e_vT, c->uc2e_vT32, L * ns2), c->up.ptr, c->leaf_node_rows.ptr + b,
-                     c->leaf_scale(l), 0, c->stream);
-  }
+  pinv_products(c, c->r_up, c->check.ptr, c->leaf_slot_rows.ptr, c->f32_pinv, gemm_op(c->f32_pinv, c->uc2e_uT, c->uc2e_uT32),
+                gemm_op(c->f32_pinv, c->uc2e_vT, c->uc2e_vT32), c->up.ptr);
+}
+
+// One level of M2M / L2L: the non-leaves of level l.
+GemmGroup level_group(const xfmm_context* c, int l, int n, int k, size_t stride) {
+  GemmGroup G;
+  G.nseg = 1;
+  G.seg[0].row0 = c->nl_level_off[l];
+  G.seg[0].m = c->nl_level_off[l + 1] - c->nl_level_off[l];
+  G.seg[0].n = n * c->vw;
+  G.seg[0].k = k * c->vw;
+  G.seg[0].boff = c->op_level(l) * stride;
+  return G;
 }
 
 void op_M2M(xfmm_context* c) {
-  const size_t blk = 8 * gemm_op_size(c);
-  const int vw = c->vw;
-  for (int l = c->depth - 1; l >= 0; l--) {
-    const int b = c->nl_level_off[l], e = c->nl_level_off[l + 1];
-    if (e <= b) continue;
-    const int L = c->op_level(l);
-    // parent row = [child_0 .. child_7] (contiguous, K = 8 nsurf) x M2Mcat
-    launch_gemm_rows(c->trans32(), e - b, c->nsurf * vw, 8 * c->nsurf * vw, c->up.ptr, c->nl_child_rows.ptr + b,
-                     gemm_op(c->trans32(), c, c->m2mcat, c->m2mcat32, L * blk), c->up.ptr, c->nl_rows.ptr + b, 1.0, 1,
-                     c->stream, c->gemm_scratch.ptr, c->gemm_scratch.n);
-  }
+  const bool f32 = c->trans32();
+  // parent row = [child_0 .. child_7] (contiguous, K = 8 nsurf) x M2Mcat
+  for (int l = c->depth - 1; l >= 0; l--)
+    launch_gemm_rows(f32, level_group(c, l, c->nsurf, 8 * c->nsurf, m2m_stride(c, f32)), c->up.ptr,
+                     c->nl_child_rows.ptr, gemm_op(f32, c->m2mcat, c->m2mcat32), c->up.ptr, c->nl_rows.ptr, 1,
+                     c->stream);
 }
 
 void op_L2L(xfmm_context* c) {
-  const size_t blk = 8 * gemm_op_size(c);
-  const int vw = c->vw;
-  for (int l = 0; l < c->depth; l++) {
-    const int b = c->nl_level_off[l], e = c->nl_level_off[l + 1];
-    if (e <= b) continue;
-    const int L = c->op_level(l);
-    launch_gemm_rows(c->trans32(), e - b, 8 * c->nsurf * vw, c->nsurf * vw, c->dn.ptr, c->nl_rows.ptr + b,
-                     gemm_op(c->trans32(), c, c->l2lcat, c->l2lcat32, L * blk), c->dn.ptr, c->nl_child_rows.ptr + b,
-                     1.0, 1, c->stream, c->gemm_scratch.ptr, c->gemm_scratch.n);
-  }
+  const bool f32 = c->trans32();
+  for (int l = 0; l < c->depth; l++)
+    launch_gemm_rows(f32, level_group(c, l, 8 * c->nsurf, c->nsurf, l2l_stride(c, f32)), c->dn.ptr, c->nl_rows.ptr,
+                     gemm_op(f32, c->l2lcat, c->l2lcat32), c->dn.ptr, c->nl_child_rows.ptr, 1, c->stream);
 }
 
 // near_add (may be null): per-target values added to the L2P result (the
 // near field of a full evaluation); wait_near: they come from the second
 // stream, joined before the L2P kernel.
 void op_L2P(xfmm_context* c, const double* near_add, bool wait_near) {
-  const size_t ns2 = gemm_op_size(c);
-  const int vw = c->vw;
-  for (int l = 0; l <= c->depth; l++) {
-    const int b = c->leaf_level_off[l], e = c->leaf_level_off[l + 1];
-    if (e <= b) continue;
-    const int L = c->op_level(l);
-    const int r = c->r_dn[L];
-    launch_gemm_rows(c->f32_pinv, e - b, r * vw, c->nsurf * vw, c->dn.ptr, c->leaf_node_rows.ptr + b,
-                     gemm_op(c->f32_pinv, c, c->dc2e_uT, c->dc2e_uT32, L * ns2), c->tmp.ptr, c->leaf_slot_rows.ptr + b,
-                     1.0, 0, c->stream);
-    launch_gemm_rows(c->f32_pinv, e - b, c->nsurf * vw, r * vw, c->tmp.ptr, c->leaf_slot_rows.ptr + b,
-                     gemm_op(c->f32_pinv, c, c->dc2e_vT, c->dc2e_vT32, L * ns2), c->dn.ptr, c->leaf_node_rows.ptr + b,
-                     c->leaf_scale(l), 0, c->stream);
-  }
+  pinv_products(c, c->r_dn, c->dn.ptr, c->leaf_node_rows.ptr, c->f32_pinv, gemm_op(c->f32_pinv, c->dc2e_uT, c->dc2e_uT32),
+                gemm_op(c->f32_pinv, c->dc2e_vT, c->dc2e_vT32), c->dn.ptr);
   DevTree t = c->dev_tree();
   if (wait_near) HIPCHK(hipStreamWaitEvent(c->stream, c->ev[20], 0));
   t.near_add = near_add;
@@ -775,25 +789,44 @@ int xfmm_set_operators(xfmm_context* c, int nlevels, const double* uc2e_u, const
       }
     };
     std::vector<double> h, hx;
-    auto put = [&](DevBuf<double>& dst, const std::vector<int>* rk) {
-      if (!c->cplx) {
-        dst.upload(h, c->stream);
-        return;
+    DevBuf<double> rows;  // one operator in row-major form, all levels
+    // Uploads the K x N operators in src (levels at a stride of lev entries of
+    // kind T; with rk only the first r columns, with rrow the first r rows are
+    // used) and packs them into d (FP64) and / or f (FP32).
+    auto put = [&](std::vector<double>& src, int K, int N, const std::vector<int>* rk, const std::vector<int>* rrow,
+                   bool want64, bool want32, size_t s64, size_t s32, DevBuf<double>& d, DevBuf<float>& f) {
+      size_t lev = size_t(K) * N * vw;
+      const std::vector<double>* up = &src;
+      if (c->cplx) {
+        expand(src, K, rk, N, hx);
+        up = &hx;
+        lev *= 2;
       }
-      expand(h, ns, rk, ns, hx);
-      dst.upload(hx, c->stream);
-      HIPCHK(hipStreamSynchronize(c->stream));  // hx is reused
+      rows.upload(*up, c->stream);
+      d.release();
+      f.release();
+      if (want64) d.alloc(size_t(nlevels) * s64);
+      if (want32) f.alloc(size_t(nlevels) * s32);
+      for (int L = 0; L < nlevels; L++) {
+        const int k = (rrow ? (*rrow)[L] : K) * vw, n = (rk ? (*rk)[L] : N) * vw;
+        if (want64) launch_gemm_pack(false, k, n, rows.ptr + L * lev, d.ptr + L * s64, c->stream);
+        if (want32) launch_gemm_pack(true, k, n, rows.ptr + L * lev, f.ptr + L * s32, c->stream);
+      }
+      HIPCHK(hipStreamSynchronize(c->stream));  // the host and device copies are reused
+    };
+    auto put_pinv = [&](const std::vector<int>* rk, const std::vector<int>* rrow, DevBuf<double>& d, DevBuf<float>& f) {
+      put(h, ns, ns, rk, rrow, !c->f32_pinv, c->f32_pinv, pinv_stride(c, false), pinv_stride(c, true), d, f);
     };
     transpose_set(uc2e_u, h);
     compact(h, c->r_up);
-    put(c->uc2e_uT, &c->r_up);
+    put_pinv(&c->r_up, nullptr, c->uc2e_uT, c->uc2e_uT32);
     transpose_set(uc2e_v, h);
-    put(c->uc2e_vT, nullptr);
+    put_pinv(nullptr, &c->r_up, c->uc2e_vT, c->uc2e_vT32);
     transpose_set(dc2e_u, h);
     compact(h, c->r_dn);
-    put(c->dc2e_uT, &c->r_dn);
+    put_pinv(&c->r_dn, nullptr, c->dc2e_uT, c->dc2e_uT32);
     transpose_set(dc2e_v, h);
-    put(c->dc2e_vT, nullptr);
+    put_pinv(nullptr, &c->r_dn, c->dc2e_vT, c->dc2e_vT32);
     // M2Mcat[L]: (8 ns) x ns, row o*ns + k, col n = M2M[L][o][n][k]
     // L2Lcat[L]: ns x (8 ns), row k, col o*ns + n = L2L[L][o][n][k]
     std::vector<double> mm(size_t(nlevels) * 8 * ns2 * vw), ll(size_t(nlevels) * 8 * ns2 * vw);
@@ -806,31 +839,13 @@ int xfmm_set_operators(xfmm_context* c, int nlevels, const double* uc2e_u, const
               mm[((size_t(L) * 8 * ns2) + (size_t(o) * ns + k) * ns + n) * vw + w] = m2m[s];
               ll[((size_t(L) * 8 * ns2) + size_t(k) * 8 * ns + size_t(o) * ns + n) * vw + w] = l2l[s];
             }
-    if (c->cplx) {
-      // M2Mcat: (8 ns) x ns complex -> (16 ns) x (2 ns); L2Lcat: ns x (8 ns) -> (2 ns) x (16 ns)
-      expand(mm, 8 * ns, nullptr, ns, hx);
-      c->m2mcat.upload(hx, c->stream);
-      HIPCHK(hipStreamSynchronize(c->stream));
-      expand(ll, ns, nullptr, 8 * ns, hx);
-      c->l2lcat.upload(hx, c->stream);
-      HIPCHK(hipStreamSynchronize(c->stream));
-    } else {
-      c->m2mcat.upload(mm, c->stream);
-      c->l2lcat.upload(ll, c->stream);
-    }
-    // FP32 copies of the GEMM operators for the FP32 translation GEMMs
-    const std::pair<DevBuf<double>*, DevBuf<float>*> f32ops[] = {
-        {&c->uc2e_uT, &c->uc2e_uT32}, {&c->uc2e_vT, &c->uc2e_vT32}, {&c->dc2e_uT, &c->dc2e_uT32},
-        {&c->dc2e_vT, &c->dc2e_vT32}, {&c->m2mcat, &c->m2mcat32},   {&c->l2lcat, &c->l2lcat32}};
-    for (int i = 0; i < 6; i++) {
-      const auto& pr = f32ops[i];
-      if (i < 4 ? c->f32_pinv : c->f32_trans) {
-        pr.second->alloc(pr.first->n);
-        launch_to_float(pr.first->ptr, pr.second->ptr, pr.first->n, c->stream);
-      } else {
-        pr.second->release();
-      }
-    }
+    // (the mixed path keeps both: charges of one sign run M2M / L2L in FP64)
+    const bool t64 = !c->f32_trans || c->prec == XFMM_MIXED;
+    put(mm, 8 * ns, ns, nullptr, nullptr, t64, c->f32_trans, m2m_stride(c, false), m2m_stride(c, true), c->m2mcat,
+        c->m2mcat32);
+    put(ll, ns, 8 * ns, nullptr, nullptr, t64, c->f32_trans, l2l_stride(c, false), l2l_stride(c, true), c->l2lcat,
+        c->l2lcat32);
+    rows.release();
     const size_t msz = size_t(nm2l) * NM2L * c->nfreq * 64 * 2;
     // reference layout uploaded, then expanded on the device into the per-lane
     // MFMA operand form (twice the size) used by the Hadamard kernel
@@ -1176,16 +1191,6 @@ int xfmm_set_tree(xfmm_context* c, const xfmm_tree* t) {
     c->trg_value.alloc(std::max<size_t>(1, size_t(t->ntrgs) * 4 * c->vw));
     c->check.alloc(std::max<size_t>(1, leaf.size() * c->nsurf * c->vw));
     c->tmp.alloc(std::max<size_t>(1, leaf.size() * c->nsurf * c->vw));
-    {
-      size_t need = 0;  // split-K scratch of the per-level M2M / L2L GEMMs
-      for (int l = 0; l < D; l++) {
-        const int rows = c->nl_level_off[l + 1] - c->nl_level_off[l];
-        if (rows <= 0) continue;
-        need = std::max(need, gemm_scratch_doubles(rows, c->nsurf * c->vw, 8 * c->nsurf * c->vw));
-        need = std::max(need, gemm_scratch_doubles(rows, 8 * c->nsurf * c->vw, c->nsurf * c->vw));
-      }
-      c->gemm_scratch.alloc(need);
-    }
     c->q.alloc(std::max<size_t>(1, size_t(t->nsrcs) * c->vw));
     c->near.alloc(c->trg_value.n);
     launch_zero(c->q.ptr, c->q.n, st);

@@ -1,44 +1,38 @@
-// Row-gathered FP64 GEMM for the translation operators.
+// Row-gathered GEMMs for the translation operators.
 //
-//   C[crow[i] + n] (=|+=) alpha[i] * sum_k A[arow[i] + k] * B[k*N + n]
+//   C[crow[i] + n] (=|+=) alpha * sum_k A[arow[i] + k] * B[k][n]
 //
 // Used for the pseudo-inverse applications of P2M / L2P (reference
-// fmm_scale_invariant.h:189-193, 215-219: two gemv per leaf, batched here over
-// all leaves of a level), for M2M (fmm_scale_invariant.h:243-251: the 8 child
-// vectors of a parent are contiguous, so a level is one GEMM with
+// fmm_scale_invariant.h:189-193, 215-219: two gemv per leaf, here one launch
+// over the leaves of all levels), for M2M (fmm_scale_invariant.h:243-251: the
+// 8 child vectors of a parent are contiguous, so a level is one GEMM with
 // K = 8*nsurf against the stacked transposed M2M matrices) and for L2L
 // (fmm_scale_invariant.h:260-268: N = 8*nsurf against the concatenated
 // transposed L2L matrices, accumulating into the contiguous child vectors).
 //
-// All of them run on the matrix cores (k_gemm_rows_mfma64, split-K when the
-// output has too few tiles to fill the chip).  Complex operands (Helmholtz)
-// come as real GEMMs: interleaved (re, im) rows times the operator expanded
-// into real 2 x 2 blocks [[Re, Im], [-Im, Re]] (K and N doubled, built once
-// by the engine when the operators are set).
-#include <stdexcept>
+// All of them run on the matrix cores.  Complex operands (Helmholtz) come as
+// real GEMMs: interleaved (re, im) rows times the operator expanded into real
+// 2 x 2 blocks [[Re, Im], [-Im, Re]] (K and N doubled, built once by the
+// engine when the operators are set).
+#include <algorithm>
 
 #include "kernels.h"
 
 namespace xfmm {
 
-// MFMA path: BM x BN output tile per 256-thread workgroup, the 4 waves as
-// 2 x 2 sub-tiles of (BM/2) x (BN/2) (a grid of 16 x 16 MFMA tiles each), K
-// staged through LDS in steps of BK (16) with the next
-// step's global loads held in registers while the current step computes.
-// Tiles are ordered so that the column tiles of one BM-row band run on one
-// XCD (workgroup w goes to XCD w % 8), which then reads that band of A once
-// into its L2.  Optional split-K (grid.y): each split writes its partial
-// product to `partial` and k_gemm_reduce combines them in a fixed order.
-// Compute type of the MFMA path: FP64 (v_mfma_f64_16x16x4_f64, result
-// register q of lane group g = row g + 4q) or FP32 (v_mfma_f32_16x16x4_f32,
-// row 4g + q) for operators that tolerate it; A (the vectors) is FP64 in
-// memory and rounded while staged, B (the operator) is read in the compute
-// type, results are stored as FP64.
+// Compute types: FP64 (v_mfma_f64_16x16x4_f64, result register q of lane
+// group g = row g + 4q) or FP32 (v_mfma_f32_16x16x4_f32, row 4g + q) for
+// operators that tolerate it; A (the vectors) is FP64 in memory and rounded
+// as it is used, B (the operator) is read in the compute type, results are
+// stored as FP64.  KL = consecutive K entries of a lane per fragment (16
+// bytes of B), KB = 4 KL = K entries of a fragment.
 template <typename CT>
 struct GemmMfma;
 template <>
 struct GemmMfma<double> {
   typedef double v4 __attribute__((ext_vector_type(4)));
+  typedef double frag __attribute__((ext_vector_type(2)));
+  static constexpr int KL = 2, KB = 8;
   static __device__ __forceinline__ v4 mma(double a, double b, v4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
@@ -47,234 +41,287 @@ struct GemmMfma<double> {
 template <>
 struct GemmMfma<float> {
   typedef float v4 __attribute__((ext_vector_type(4)));
+  typedef float frag __attribute__((ext_vector_type(4)));
+  static constexpr int KL = 4, KB = 16;
   static __device__ __forceinline__ v4 mma(float a, float b, v4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ int row(int g, int q) { return 4 * g + q; }
 };
 
-// Without `partial` the kernel writes C itself: alpha scales the rows of A as
-// they are staged (exact: alpha is a power of two) and BETA adds C in the
-// epilogue.  BETA = false keeps the epilogue a plain store, so the
-// accumulators never leave the AGPRs before it (BETA = true costs occupancy
-// and is used only when no split-K scratch is available).
-template <int BM, int BN, int BK, bool BETA, typename CT>
-__global__ __launch_bounds__(256) void k_gemm_rows_mfma64(int m, int n, int k, int kper, int ncol,
-                                                         const double* __restrict__ A, const long* __restrict__ arow,
-                                                         const CT* __restrict__ B, double* __restrict__ C,
-                                                         const long* __restrict__ crow, double alpha,
-                                                         double* __restrict__ partial) {
-  constexpr int WM = BM / 2, WN = BN / 2, TA = WM / 16, TB = WN / 16;
-  constexpr int NQA = BM * BK / 256, NQB = BK * BN / 256;  // loader elements per thread
-  constexpr int ARS = 256 / BK, BKS = 256 / BN;            // loader row / k strides
-  static_assert(BM % 32 == 0 && BN % 32 == 0 && BN <= 256 && NQA >= 1 && NQB >= 1, "tile shape");
-  typedef typename GemmMfma<CT>::v4 d4;
-  __shared__ CT As[BK][BM + 2];
-  __shared__ CT Bs[BK][BN + 2];
-  __shared__ long arow_s[BM];
-  // XCD ordering when there are at least 8 row bands (grid padded to a
-  // multiple of 8 bands), plain row-major tile order otherwise
-  const int w = blockIdx.x;
-  const int nband = (m + BM - 1) / BM;
-  int row0, col0;
-  if (nband >= 8) {
-    const int x = w & 7, i = w >> 3;
-    row0 = ((i / ncol) * 8 + x) * BM;
-    col0 = (i % ncol) * BN;
-  } else {
-    row0 = (w / ncol) * BM;
-    col0 = (w % ncol) * BN;
+// Packed operators.  Lane (g, j) of a wave (g = lane / 16, j = lane % 16)
+// feeds step s < KL of K block kb with k = kb KB + KL g + s, for A and B
+// alike (the order of the K sum is free), so that its entries are
+// consecutive: one 16-byte load of B, one or two of A.  B is stored as
+// [column group of 64][kb][column tile of 16][lane][KL], zero beyond (K, N).
+static size_t packed_off(int nkb, int KL, int col, int kb, int lane) {
+  return ((size_t(col / 64) * nkb + kb) * 256 + size_t(col / 16 % 4) * 64 + lane) * KL;
+}
+
+size_t gemm_packed_size(bool f32, int k, int n) {
+  const int KB = f32 ? GemmMfma<float>::KB : GemmMfma<double>::KB;
+  const int KL = f32 ? GemmMfma<float>::KL : GemmMfma<double>::KL;
+  return packed_off((k + KB - 1) / KB, KL, (n + 63) / 64 * 64, 0, 0);
+}
+
+template <typename CT>
+__global__ void k_gemm_pack(int k, int n, const double* __restrict__ B, CT* __restrict__ out, size_t total) {
+  constexpr int KB = GemmMfma<CT>::KB, KL = GemmMfma<CT>::KL;
+  const int nkb = (k + KB - 1) / KB;
+  const size_t stride = size_t(gridDim.x) * blockDim.x;
+  for (size_t e = size_t(blockIdx.x) * blockDim.x + threadIdx.x; e < total; e += stride) {
+    const int s = int(e % KL), lane = int(e / KL % 64), ct = int(e / (KL * 64) % 4);
+    const size_t gk = e / (KL * 256);  // column group * nkb + kb
+    const int kk = int(gk % nkb) * KB + KL * (lane >> 4) + s;
+    const int cc = int(gk / nkb) * 64 + ct * 16 + (lane & 15);
+    out[e] = (kk < k && cc < n) ? CT(B[size_t(kk) * n + cc]) : CT(0);
   }
-  if (row0 >= m) return;  // padding bands of the XCD ordering (uniform per workgroup)
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+}
+
+void launch_gemm_pack(bool f32, int k, int n, const double* B, void* out, hipStream_t s) {
+  const size_t total = gemm_packed_size(f32, k, n);
+  if (total == 0) return;
+  const dim3 g(unsigned(std::min<size_t>((total + 255) / 256, 65536))), b(256);
+  if (f32) hipLaunchKernelGGL(k_gemm_pack<float>, g, b, 0, s, k, n, B, static_cast<float*>(out), total);
+  else hipLaunchKernelGGL(k_gemm_pack<double>, g, b, 0, s, k, n, B, static_cast<double*>(out), total);
+}
+
+// A wave computes a (16 TA) x (16 TB) tile of C; a workgroup is RW x CW such
+// tiles, each with KW waves that share its K range and add their sums through
+// LDS in a fixed order (in FP64).  Operands go straight from global memory
+// (L1 / L2) to registers, two K blocks ahead, with no LDS and no barrier in
+// the K loop: an FP64 MFMA takes 64 cycles for 8 flop per lane and byte of
+// operand, so a wave needs only ~6 bytes a cycle, and small tiles cost
+// little.  What bounds it: the FP64 matrix cores (52-60 of 78.6 TFLOP/s on the
+// large shapes) and, in FP32, the loads of A in FP64.  Against the previous
+// kernel (128 x 128 or 64 x 64 workgroup tiles staged through LDS, one launch per
+// level, split-K partial sums in memory): FP64 32768 x 488 x 224 172 -> 129 us, 4096 x 160 x
+// 296 64 -> 12, 4096 x 481 x 488 99 -> 39, 4096 x 488 x 3904 333 -> 256;
+// FP32 4096 x 488 x 3904 213 -> 157, 4096 x 3904 x 488 249 -> 217, 1 x 488 x 3904
+// 19 -> 9 us.
+// Tiles are numbered segment by segment, row band by row band; XCD x
+// (workgroup id % 8) takes a contiguous eighth of them, so that a band of A
+// is read into one L2.
+template <typename CT, int TA, int TB, int KW, int RW, int CW, bool BETA>
+__global__ __launch_bounds__(64 * KW * RW * CW, 2) void k_gemm_rows(GemmGroup G, const double* __restrict__ A,
+                                                                  const long* __restrict__ arow,
+                                                                  const CT* __restrict__ B, double* __restrict__ C,
+                                                                  const long* __restrict__ crow) {
+  typedef GemmMfma<CT> M;
+  typedef typename M::v4 v4;
+  typedef typename M::frag frag;
+  constexpr int KL = M::KL, KB = M::KB, PF = 2;
+  static_assert(TB == 1 || TB == 2 || TB == 4, "column tiles of a wave lie in one packed group");
+  static_assert(KW == 1 || RW * CW == 1, "waves that share a K range are one tile");
+  typedef double dv __attribute__((ext_vector_type(KL)));
+  const int per = (G.ntile + 7) / 8;
+  const int tile = int(blockIdx.x & 7) * per + int(blockIdx.x >> 3);
+  if (int(blockIdx.x >> 3) >= per || tile >= G.ntile) return;  // uniform per workgroup
+  int si = 0;
+  while (si + 1 < G.nseg && tile >= G.seg[si + 1].tile0) si++;
+  const GemmSeg sg = G.seg[si];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int j = lane & 15, g = lane >> 4;
-  const int wr = wv >> 1, wc = wv & 1;
-  const int kbeg = blockIdx.y * kper, kend = min(k, kbeg + kper);
-  for (int r = tid; r < BM; r += 256) arow_s[r] = (row0 + r < m) ? arow[row0 + r] : -1;
-  const bool direct = partial == nullptr;
-  const double scale = direct ? alpha : 1.0;
-  d4 acc[TA][TB];
+  const int ks = wv % KW, cw = wv / KW % CW, rw = wv / (KW * CW);
+  const int nct = (sg.n + 15) / 16, ncg = (nct + TB * CW - 1) / (TB * CW);
+  const int row0 = ((tile - sg.tile0) / ncg * RW + rw) * 16 * TA;
+  const int ct0 = ((tile - sg.tile0) % ncg * CW + cw) * TB;
+  const int nkb = (sg.k + KB - 1) / KB, kfull = sg.k / KB;  // kfull: blocks without a K remainder
+  const double* pa[TA];
+#pragma unroll
+  for (int a = 0; a < TA; a++) pa[a] = A + arow[sg.row0 + min(row0 + a * 16 + j, sg.m - 1)] + KL * g;
+  // (a wave past the last column tile or row has no work: its K range is empty)
+  const bool live = ct0 < nct && row0 < sg.m;
+  const int ctc = live ? ct0 : 0;
+  const CT* pb = B + sg.boff + (size_t(ctc / 4) * nkb * 256 + size_t(ctc % 4) * 64 + lane) * KL;
+  v4 acc[TA][TB];
 #pragma unroll
   for (int a = 0; a < TA; a++)
 #pragma unroll
-    for (int b = 0; b < TB; b++) acc[a][b] = d4{0, 0, 0, 0};
-  __syncthreads();
-  // loader mapping: A element e = tid + 256 q -> row e / BK, k e % BK;
-  // B element e -> k e / BN, column e % BN
-  const int akk = tid % BK, ar0 = tid / BK;
-  const int bkk = tid / BN, bc = tid % BN;
-  long arw[NQA];
+    for (int b = 0; b < TB; b++) acc[a][b] = v4{0, 0, 0, 0};
+  const int kper = (nkb + KW - 1) / KW;
+  const int kb0 = ks * kper, kb1 = live ? min(nkb, kb0 + kper) : kb0, kbf = min(kfull, kb1);
+  // FP32: sums of at most FOLD K blocks (128 products), added to their total
+  // one by one, so that rounding does not grow with K (a single chain of 488 or
+  // 976 gave 1.2 times the error of the evaluation)
+  constexpr int FOLD = 8;
+  constexpr bool FOLDS = sizeof(CT) == 4;
+  v4 tot[TA][TB];
+  auto fold = [&]() {
 #pragma unroll
-  for (int q = 0; q < NQA; q++) arw[q] = arow_s[ar0 + ARS * q];
-  const bool bcol_ok = col0 + bc < n;
-  double ra[NQA];
-  CT rb[NQB];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int q = 0; q < NQA; q++) ra[q] = (arw[q] >= 0 && k0 + akk < kend) ? A[arw[q] + k0 + akk] : 0.0;
-#pragma unroll
-    for (int q = 0; q < NQB; q++) {
-      const int kb = bkk + BKS * q;
-      rb[q] = (bcol_ok && k0 + kb < kend) ? B[size_t(k0 + kb) * n + col0 + bc] : CT(0);
-    }
-  };
-  if (kbeg < kend) fetch(kbeg);
-  for (int k0 = kbeg; k0 < kend; k0 += BK) {
-    // (the scale is applied here, when the loads have arrived anyway, so the
-    // prefetch of the next stage is not waited for before the MFMAs)
-#pragma unroll
-    for (int q = 0; q < NQA; q++) As[akk][ar0 + ARS * q] = CT(scale * ra[q]);
-#pragma unroll
-    for (int q = 0; q < NQB; q++) Bs[bkk + BKS * q][bc] = rb[q];
-    __syncthreads();
-    if (k0 + BK < kend) fetch(k0 + BK);
-#pragma unroll
-    for (int s = 0; s < BK / 4; s++) {
-      const int kk = 4 * s + g;
-      CT av[TA], bv[TB];
-#pragma unroll
-      for (int t = 0; t < TA; t++) av[t] = As[kk][wr * WM + t * 16 + j];
-#pragma unroll
-      for (int t = 0; t < TB; t++) bv[t] = Bs[kk][wc * WN + t * 16 + j];
-#pragma unroll
-      for (int a = 0; a < TA; a++)
-#pragma unroll
-        for (int b = 0; b < TB; b++) acc[a][b] = GemmMfma<CT>::mma(av[a], bv[b], acc[a][b]);
-    }
-    __syncthreads();
-  }
-  // result register q of lane (g, j): row GemmMfma::row(g, q), column j of
-  // the 16 x 16 tile
-#pragma unroll
-  for (int a = 0; a < TA; a++)
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int r = row0 + wr * WM + a * 16 + GemmMfma<CT>::row(g, q);
-      if (r >= m) continue;
+    for (int a = 0; a < TA; a++)
 #pragma unroll
       for (int b = 0; b < TB; b++) {
-        const int cc = col0 + wc * WN + b * 16 + j;
-        if (cc >= n) continue;
-        const double v = double(acc[a][b][q]);
-        if (!direct) partial[(size_t(blockIdx.y) * m + r) * n + cc] = v;
-        else if (BETA) C[crow[r] + cc] += v;
-        else C[crow[r] + cc] = v;
+        tot[a][b] += acc[a][b];
+        acc[a][b] = v4{0, 0, 0, 0};
       }
-      // one accumulator tile at a time through the VGPRs in the BETA epilogue
-      if (BETA) __builtin_amdgcn_sched_barrier(0);
+  };
+  if constexpr (FOLDS) {
+#pragma unroll
+    for (int a = 0; a < TA; a++)
+#pragma unroll
+      for (int b = 0; b < TB; b++) tot[a][b] = v4{0, 0, 0, 0};
+  }
+  dv fa[PF][TA];
+  frag fb[PF][TB];
+  // row offsets are even numbers of doubles: 16-byte aligned loads
+  auto load = [&](int kb, dv* xa, frag* xb) {
+#pragma unroll
+    for (int a = 0; a < TA; a++) {
+      const double2* p = reinterpret_cast<const double2*>(pa[a] + kb * KB);
+#pragma unroll
+      for (int s = 0; s < KL; s += 2) {
+        const double2 v = p[s / 2];
+        xa[a][s] = v.x;
+        xa[a][s + 1] = v.y;
+      }
     }
-}
-
-__global__ void k_to_float(const double* __restrict__ in, float* __restrict__ out, size_t n) {
-  const size_t stride = size_t(gridDim.x) * blockDim.x;
-  for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) out[i] = float(in[i]);
-}
-
-void launch_to_float(const double* in, float* out, size_t n, hipStream_t s) {
-  if (n == 0) return;
-  const unsigned blocks = unsigned(std::min<size_t>((n + 255) / 256, 65536));
-  hipLaunchKernelGGL(k_to_float, dim3(blocks), dim3(256), 0, s, in, out, n);
-}
-
-__global__ void k_gemm_reduce(int m, int n, int nsplit, const double* __restrict__ partial, double* __restrict__ C,
-                              const long* __restrict__ crow, double alpha, int beta) {
-  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= size_t(m) * n) return;
-  const int r = int(i / n), cc = int(i % n);
-  double s = 0;
-  for (int z = 0; z < nsplit; z++) s += partial[(size_t(z) * m + r) * n + cc];
-  const long cr = crow[r];
-  double v = alpha * s;
-  if (beta) v += C[cr + cc];
-  C[cr + cc] = v;
-}
-
-// Tile shape: 128 x 128 for large outputs, 64 x 64 for small levels (more
-// workgroups, shorter per-workgroup K loop).
-struct GemmTile {
-  int bm, bn;
-};
-static GemmTile gemm_tile(int m) { return m >= 2048 ? GemmTile{128, 128} : GemmTile{64, 64}; }
-
-// split-K factor: enough workgroups for every resident slot of the chip
-// (256 CUs x 2 workgroups of 128 x 128, x 4 of 64 x 64), each split keeping
-// at least 64 of K (4 LDS stages)
-static int gemm_split(int m, int n, int k) {
-  const GemmTile t = gemm_tile(m);
-  const int tiles = ((n + t.bn - 1) / t.bn) * ((m + t.bm - 1) / t.bm);
-  const int target = t.bm == 128 ? 512 : 1024;
-  int split = 1;
-  while (split < 64 && tiles * split < target && k / (split * 2) >= 64) split *= 2;
-  return split;
-}
-
-size_t gemm_scratch_doubles(int m, int n, int k) {
-  const int split = gemm_split(m, n, k);
-  return split > 1 ? size_t(split) * m * n : 0;
-}
-
-// K step (measured on 32768x488x488 and 4096x488x3904: FP32 with 32 needs
-// more registers and drops to 2 waves per SIMD, 5-7 % slower than 16)
-template <typename CT>
-constexpr int gemm_bk() { return 16; }
-
-template <int BM, int BN, bool BETA, typename CT>
-static void launch_mfma(int m, int n, int k, int split, const double* A, const long* arow, const CT* B, double* C,
-                        const long* crow, double alpha, double* partial, hipStream_t s) {
-  constexpr int BK = gemm_bk<CT>();
-  int kper = (k + split - 1) / split;
-  kper = (kper + BK - 1) / BK * BK;
-  const int ncol = (n + BN - 1) / BN;
-  const int nband = (m + BM - 1) / BM;
-  const int nb = nband >= 8 ? (nband + 7) / 8 * 8 : nband;
-  dim3 grid(unsigned(nb * ncol), split);
-  hipLaunchKernelGGL((k_gemm_rows_mfma64<BM, BN, BK, BETA, CT>), grid, dim3(256), 0, s, m, n, k, kper, ncol, A,
-                     arow, B, C, crow, alpha, partial);
-}
-
-template <int BM, int BN, typename CT>
-static void launch_tile(int m, int n, int k, int split, bool part, const double* A, const long* arow, const CT* B,
-                        double* C, const long* crow, double alpha, int beta, double* scratch, hipStream_t s) {
-  // (the 128 x 128 += epilogue is never built: it would cost occupancy;
-  // launch_real picks 128 x 128 only for split-K or plain stores)
-  if (part) {
-    launch_mfma<BM, BN, false, CT>(m, n, k, split, A, arow, B, C, crow, alpha, scratch, s);
-  } else if constexpr (BM != 128) {
-    if (beta) launch_mfma<BM, BN, true, CT>(m, n, k, 1, A, arow, B, C, crow, alpha, nullptr, s);
-    else launch_mfma<BM, BN, false, CT>(m, n, k, 1, A, arow, B, C, crow, alpha, nullptr, s);
+#pragma unroll
+    for (int b = 0; b < TB; b++) xb[b] = *reinterpret_cast<const frag*>(pb + (kb * 256 + b * 64) * KL);
+  };
+  auto mul = [&](const dv* xa, const frag* xb) {
+#pragma unroll
+    for (int s = 0; s < KL; s++)
+#pragma unroll
+      for (int a = 0; a < TA; a++) {
+        const CT av = CT(xa[a][s]);
+#pragma unroll
+        for (int b = 0; b < TB; b++) acc[a][b] = M::mma(av, xb[b][s], acc[a][b]);
+      }
+  };
+  if (kb0 < kbf) {
+#pragma unroll
+    for (int u = 0; u < PF; u++) load(min(kb0 + u, kbf - 1), fa[u], fb[u]);
+    int kb = kb0;
+    for (; kb + PF <= kbf; kb += PF) {
+#pragma unroll
+      for (int u = 0; u < PF; u++) {
+        mul(fa[u], fb[u]);
+        load(min(kb + u + PF, kbf - 1), fa[u], fb[u]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (FOLDS) {
+        if ((kb - kb0) % FOLD == FOLD - PF) fold();
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PF; u++)
+      if (kb + u < kbf) mul(fa[u], fb[u]);
+  }
+  if (kfull < kb1 && kfull >= kb0) {  // K remainder: A past the row's end is not read
+#pragma unroll
+    for (int a = 0; a < TA; a++)
+#pragma unroll
+      for (int s = 0; s < KL; s++) fa[0][a][s] = (kfull * KB + KL * g + s < sg.k) ? pa[a][kfull * KB + s] : 0.0;
+#pragma unroll
+    for (int b = 0; b < TB; b++) fb[0][b] = *reinterpret_cast<const frag*>(pb + (kfull * 256 + b * 64) * KL);
+    mul(fa[0], fb[0]);
+  }
+  if constexpr (FOLDS) {
+#pragma unroll
+    for (int a = 0; a < TA; a++)
+#pragma unroll
+      for (int b = 0; b < TB; b++) acc[a][b] += tot[a][b];
+  }
+  // result register q of lane (g, j): row M::row(g, q), column j of the tile
+  auto put = [&](int r, int cc, double v) {
+    double* c = C + crow[sg.row0 + r] + cc;
+    v *= sg.alpha;
+    *c = BETA ? *c + v : v;
+  };
+  if constexpr (KW == 1) {
+#pragma unroll
+    for (int a = 0; a < TA; a++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int r = row0 + a * 16 + M::row(g, q);
+        if (r >= sg.m) continue;
+#pragma unroll
+        for (int b = 0; b < TB; b++) {
+          const int cc = (ct0 + b) * 16 + j;
+          if (cc < sg.n) put(r, cc, double(acc[a][b][q]));
+        }
+      }
   } else {
-    if (beta) throw std::logic_error("launch_tile: accumulating 128 x 128 tile");
-    launch_mfma<BM, BN, false, CT>(m, n, k, 1, A, arow, B, C, crow, alpha, nullptr, s);
+    constexpr int NV = TA * TB * 4;
+    __shared__ CT red[KW][NV][64];
+#pragma unroll
+    for (int a = 0; a < TA; a++)
+#pragma unroll
+      for (int b = 0; b < TB; b++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) red[ks][(a * TB + b) * 4 + q][lane] = acc[a][b][q];
+    __syncthreads();
+    for (int e = ks; e < NV; e += KW) {
+      double v = 0;
+#pragma unroll
+      for (int z = 0; z < KW; z++) v += double(red[z][e][lane]);
+      const int r = row0 + e / 4 / TB * 16 + M::row(g, e & 3), cc = (ct0 + e / 4 % TB) * 16 + j;
+      if (r < sg.m && cc < sg.n) put(r, cc, v);
+    }
   }
 }
 
+template <typename CT, int TA, int TB, int KW, int RW, int CW>
+static void launch_tiles(GemmGroup G, const double* A, const long* arow, const CT* B, double* C, const long* crow,
+                         bool beta, hipStream_t s) {
+  G.ntile = 0;
+  for (int i = 0; i < G.nseg; i++) {
+    GemmSeg& sg = G.seg[i];
+    const int nct = (sg.n + 15) / 16;
+    sg.tile0 = G.ntile;
+    G.ntile += ((nct + TB * CW - 1) / (TB * CW)) * ((sg.m + 16 * TA * RW - 1) / (16 * TA * RW));
+  }
+  const dim3 grid(unsigned((G.ntile + 7) / 8 * 8)), block(64 * KW * RW * CW);
+  if (beta) hipLaunchKernelGGL((k_gemm_rows<CT, TA, TB, KW, RW, CW, true>), grid, block, 0, s, G, A, arow, B, C, crow);
+  else hipLaunchKernelGGL((k_gemm_rows<CT, TA, TB, KW, RW, CW, false>), grid, block, 0, s, G, A, arow, B, C, crow);
+}
+
+// Tile and K split by the number of 32 x 64 (w4) and 32 x 32 (w2) wave tiles
+// against the chip's 1024 SIMDs, and by the length of K (measured, us):
+//  w4 >= 768: 64 x 128 workgroups of four 32 x 64 tiles (FP64 4096 x 481 x
+//    488, w4 = 1024: 39, 32 x 64 with K over 4 waves 42, 32 x 32 over 4 42),
+//    but K over 4 waves when K is long (FP32 4096 x 488 x 3904, w4 = 1024:
+//    203 -> 157);
+//  w2 >= 128: 32 x 32 tiles with K over 4 waves (FP64 4096 x 160 x 296, w2 =
+//    640: 12, four waves without a split 14, 32 x 64 23), over 8 or 16
+//    when K is long (FP64 512 x 296 x 2368, w2 = 160: 28 with 4, 26 with 8; FP32
+//    512 x 488 x 3904 38, 37, 39 with 4, 8, 16: 16, whose FP32 sums are the shortest);
+//  else 16 x 16 tiles with K over 8 or 16 waves (FP32 64 x 488 x 3904: 19 and 20,
+//    32 x 32 over 8 34; FP64 512 x 160 x 296 5, 32 x 32 over 8 6).
 template <typename CT>
-static void launch_real(int m, int n, int k, const double* A, const long* arow, const CT* B, double* C,
-                        const long* crow, double alpha, int beta, hipStream_t s, double* scratch,
-                        size_t scratch_doubles) {
-  // an accumulating product without split-K uses the 64 x 64 tile, whose
-  // += epilogue keeps full occupancy
-  int split = gemm_split(m, n, k);
-  const bool part = scratch && split > 1 && size_t(split) * m * n <= scratch_doubles;
-  if (!part) split = 1;
-  if (gemm_tile(m).bm == 128 && (part || !beta))
-    launch_tile<128, 128, CT>(m, n, k, split, part, A, arow, B, C, crow, alpha, beta, scratch, s);
-  else
-    launch_tile<64, 64, CT>(m, n, k, split, part, A, arow, B, C, crow, alpha, beta, scratch, s);
-  if (part) {
-    const size_t tot = size_t(m) * n;
-    hipLaunchKernelGGL(k_gemm_reduce, dim3(unsigned((tot + 255) / 256)), dim3(256), 0, s, m, n, split, scratch, C,
-                       crow, alpha, beta);
+static void launch_group(const GemmGroup& G, const double* A, const long* arow, const CT* B, double* C,
+                         const long* crow, bool beta, hipStream_t s) {
+  constexpr int KLONG = sizeof(CT) == 4 ? 16 : 8;  // waves of a long K
+  long w4 = 0, w2 = 0;
+  int k = 0;
+  for (int i = 0; i < G.nseg; i++) {
+    const GemmSeg& sg = G.seg[i];
+    w4 += long((sg.m + 31) / 32) * ((sg.n + 63) / 64);
+    w2 += long((sg.m + 31) / 32) * ((sg.n + 31) / 32);
+    k = std::max(k, sg.k);
+  }
+  const bool klong = k >= 1024;
+  if (w4 >= 768) {
+    if (klong) launch_tiles<CT, 2, 4, 4, 1, 1>(G, A, arow, B, C, crow, beta, s);
+    else launch_tiles<CT, 2, 4, 1, 2, 2>(G, A, arow, B, C, crow, beta, s);
+  } else if (w2 >= 128) {
+    if (klong) launch_tiles<CT, 2, 2, KLONG, 1, 1>(G, A, arow, B, C, crow, beta, s);
+    else launch_tiles<CT, 2, 2, 4, 1, 1>(G, A, arow, B, C, crow, beta, s);
+  } else {
+    if (klong) launch_tiles<CT, 1, 1, 16, 1, 1>(G, A, arow, B, C, crow, beta, s);
+    else launch_tiles<CT, 1, 1, 8, 1, 1>(G, A, arow, B, C, crow, beta, s);
   }
 }
 
-void launch_gemm_rows(bool f32, int m, int n, int k, const double* A, const long* arow, const void* Bv, double* C,
-                      const long* crow, double alpha, int beta, hipStream_t s, double* scratch, size_t scratch_doubles) {
-  if (m <= 0 || n <= 0) return;
-  if (f32) launch_real<float>(m, n, k, A, arow, static_cast<const float*>(Bv), C, crow, alpha, beta, s, scratch,
-                              scratch_doubles);
-  else launch_real<double>(m, n, k, A, arow, static_cast<const double*>(Bv), C, crow, alpha, beta, s, scratch,
-                           scratch_doubles);
+void launch_gemm_rows(bool f32, const GemmGroup& G, const double* A, const long* arow, const void* B, double* C,
+                      const long* crow, int beta, hipStream_t s) {
+  GemmGroup H;
+  for (int i = 0; i < G.nseg; i++)
+    if (G.seg[i].m > 0 && G.seg[i].n > 0) H.seg[H.nseg++] = G.seg[i];
+  if (H.nseg == 0) return;
+  if (f32) launch_group<float>(H, A, arow, static_cast<const float*>(B), C, crow, beta != 0, s);
+  else launch_group<double>(H, A, arow, static_cast<const double*>(B), C, crow, beta != 0, s);
 }
 
 __global__ void k_zero(double* __restrict__ p, size_t n) {

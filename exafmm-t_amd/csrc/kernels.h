@@ -82,20 +82,31 @@ void launch_direct(int kind, bool mixed, bool cplx, Wavek k, const double* src, 
                    const double* trg, int nt, double* out, int gradient, double* scratch, int nsplit,
                    hipStream_t s);
 
-// C[crow[i]] (beta=0: =, beta=1: +=) alpha * A[arow[i]] x B for i < m.
-// A rows have K values, B is K x N row-major, C rows have N values (doubles;
-// arow/crow are row offsets in doubles, not rows); alpha is a power of two.
-// FP64 MFMA, or with f32 FP32 MFMA (operands rounded to FP32 while staged,
-// FP32 accumulation, FP64 results; B float); when the output has few tiles
-// the K range is split over workgroups, partial products go to `scratch` (at
-// least gemm_scratch_doubles(m, n, k) doubles) and are reduced in a fixed
-// order.  Complex GEMMs are called as real ones on the 2 x 2 block form.
-void launch_gemm_rows(bool f32, int m, int n, int k, const double* A, const long* arow, const void* B, double* C,
-                      const long* crow, double alpha, int beta, hipStream_t s, double* scratch = nullptr,
-                      size_t scratch_doubles = 0);
-// out[i] = float(in[i]) for i < n
-void launch_to_float(const double* in, float* out, size_t n, hipStream_t s);
-size_t gemm_scratch_doubles(int m, int n, int k);
+// C[crow[i]] (beta=0: =, beta=1: +=) alpha * A[arow[i]] x B for the rows of
+// every segment (row0 <= i < row0 + m): A rows have k values, B is k x n in the
+// packed form of launch_gemm_pack, starting boff entries into the array, C
+// rows have n values (doubles; arow/crow are even row offsets in doubles, not
+// rows); alpha is a power of two.  FP64 MFMA, or with f32 FP32 MFMA (operands
+// rounded to FP32, FP32 accumulation, FP64 results; B float).  All segments
+// (the levels of a tree) run in one launch.  Complex GEMMs are called as real
+// ones on the 2 x 2 block form.
+struct GemmSeg {
+  int row0 = 0, m = 0, n = 0, k = 0;
+  int tile0 = 0;  // first tile of the segment (set by the launcher)
+  size_t boff = 0;
+  double alpha = 1.0;
+};
+constexpr int GEMM_SEGS = 32;  // levels of a tree (depth < 30)
+struct GemmGroup {
+  int nseg = 0, ntile = 0;
+  GemmSeg seg[GEMM_SEGS];
+};
+void launch_gemm_rows(bool f32, const GemmGroup& G, const double* A, const long* arow, const void* B, double* C,
+                      const long* crow, int beta, hipStream_t s);
+// Packed MFMA operand form of a row-major k x n matrix B (out: float with
+// f32, else double), gemm_packed_size entries.
+size_t gemm_packed_size(bool f32, int k, int n);
+void launch_gemm_pack(bool f32, int k, int n, const double* B, void* out, hipStream_t s);
 
 // M2L stages.
 struct M2LDev {
