@@ -144,10 +144,13 @@ struct xfmm_context {
   DevBuf<long> nl_rows, nl_child_rows;                    // node*nsurf, child0*nsurf
   // M2L
   int n_m2l_src = 0, n_m2l_trg = 0, n_m2l_blk = 0;
-  DevBuf<int> m2l_src_node, m2l_trg_node, m2l_blk_trg, m2l_blk_uni, m2l_blk_nu;
+  DevBuf<int> m2l_src_node, m2l_trg_node, m2l_blk_trg, m2l_blk_uni, m2l_blk_nu, m2l_blk_lev;
   DevBuf<short> m2l_blk_loc;
   DevBuf<double> m2l_scale;
-  std::vector<int> blk_level_off;                         // [depth+2] block ranges per target level
+  // host side of the Hadamard blocks, rebuilt when their size changes
+  int had_ntrg = 0;                                       // targets per block they were built for
+  std::vector<int> h_m2l, h_m2l_trg, h_src_slot;          // [trg slot][26] source nodes; node of a target slot; slot of a source node
+  std::vector<int> h_lat;                                 // [nnodes][3] lattice position at the node's level
   DevBuf<char> fft_in, fft_out;
   // buffers
   DevBuf<double> up, dn, trg_value, check, tmp, near;
@@ -164,9 +167,10 @@ struct xfmm_context {
   // downward pass (xfmm_set_value_scale); empty = none
   DevBuf<double> vscale;
   // tuning (xfmm_set_tuning / xfmm_autotune)
-  int tune_kch = HAD_KCH;  // Hadamard frequencies per workgroup
-  int tune_groups = 2;     // split-FP16 Hadamard: 64-target blocks per workgroup
-  int tune_tiles = 1;      // split-FP16 Hadamard: 16-target tiles per wave
+  int tune_kch = 0;        // Hadamard frequencies per workgroup (0: chosen from the grid)
+  // split-FP16 Hadamard: 128-target groups per workgroup (1 or 2) and 16-target
+  // tiles per wave; 0: chosen from the number of targets
+  int tune_groups = 0, tune_tiles = 0;
   int tune_split = 32;     // real-kernel P2P / L2P: largest tail tile whose sources are split over lanes
 
   // ---- timing
@@ -231,6 +235,8 @@ struct xfmm_context {
     m.inv_dn = inv_dn.ptr;
     m.fft_in = fft_in.ptr;
     m.fft_out = fft_out.ptr;
+    m.nsrc = n_m2l_src;
+    m.ntrg = n_m2l_trg;
     m.amax = f16_had ? reinterpret_cast<unsigned*>(m2l_amax.ptr) : nullptr;
     return m;
   }
@@ -522,27 +528,130 @@ void launch_near(xfmm_context* c) {
   c->near_launched = true;
 }
 
-// hadamard_product of every operator level (after the forward transforms)
-void run_hadamards(xfmm_context* c, const M2LDev& m) {
-  const size_t opsz = size_t(NM2L) * c->nfreq * 64 * 4;
-  // one operator set (Laplace): a single launch over the blocks of all levels
-  const int nlaunch = (c->nm2l == 1) ? 1 : c->depth;
-  for (int l = 0; l < nlaunch; l++) {
-    const int b = (c->nm2l == 1) ? 0 : c->blk_level_off[l];
-    const int e = (c->nm2l == 1) ? c->n_m2l_blk : c->blk_level_off[l + 1];
-    if (e <= b) continue;
-    const int L = (c->nm2l == 1) ? 0 : l;
-    const void* ops = c->f32_m2l ? static_cast<const void*>(c->m2l32.ptr + L * opsz)
-                                              : static_cast<const void*>(c->m2l64.ptr + L * opsz);
-    HadBlocks hb;
-    hb.nblk = e - b;
-    hb.trg = c->m2l_blk_trg.ptr + size_t(b) * 64;
-    hb.uni = c->m2l_blk_uni.ptr + size_t(b) * HAD_UCAP;
-    hb.nunion = c->m2l_blk_nu.ptr + b;
-    hb.loc = c->m2l_blk_loc.ptr + size_t(b) * NM2L * 64;
-    launch_hadamard(m, ops, c->f16_had ? c->m2l_hscale.ptr + size_t(L) * c->nfreq : nullptr, hb, c->tune_kch,
-                    c->tune_groups, c->tune_tiles, c->stream);
+// Launch shape of the Hadamard.  Split FP16: blocks of 256 targets for 8 waves
+// of two tiles once there are 1024 targets (4680 targets at p = 10 1.08 ms, 128
+// targets for 8 waves of one tile 1.33), below that 128 targets, whose
+// workgroups are twice as many (584 targets at p = 8: 103 us, 114 with 256).  FP64 / FP32: 64
+// targets, two tiles per wave from 1024 targets on (1720 targets at p = 10
+// 1.73 ms, one tile 1.96; 584 targets at p = 8 451 and 384 us).
+int had_groups(const xfmm_context* c) {
+  if (c->tune_groups > 0) return std::min(c->tune_groups, 2);
+  return c->h_m2l_trg.size() >= 1024 ? 2 : 1;
+}
+int had_tiles(const xfmm_context* c) {
+  if (c->tune_tiles > 0) return c->tune_tiles;
+  if (c->f16_had) return had_groups(c) == 2 ? 2 : 1;
+  return c->h_m2l_trg.size() >= 1024 ? 2 : 1;
+}
+int had_block_targets(const xfmm_context* c) { return c->f16_had ? 128 * had_groups(c) : 64; }
+
+// Hadamard blocks of the uploaded tree (layout at HadBlocks): consecutive
+// targets of one operator level (all levels of a scale-invariant kernel), in
+// Hilbert order, at most had_block_targets of them and had_urows union rows per
+// colour.
+void build_had_blocks(xfmm_context* c) {
+  const int T = had_block_targets(c), ucap = had_ucap(T), urows = had_urows(T);
+  if (c->had_ntrg == T) return;
+  const int ntrg = int(c->h_m2l_trg.size());
+  std::vector<int> btrg, buni, bnu, blev;
+  std::vector<short> bloc;
+  std::vector<int> lidx(c->nnodes, -1);  // source node -> union slot in the current block
+  std::vector<int> cur_t, cur_u;
+  int rows[16] = {0};
+  auto colour = [&](int node) {
+    const int* q = &c->h_lat[3 * size_t(node)];
+    return (q[0] + 4 * q[1] + 8 * q[2]) & 15;
+  };
+  auto flush = [&]() {
+    if (cur_t.empty()) return;
+    const size_t bt = btrg.size(), bu = buni.size(), bl = bloc.size();
+    btrg.resize(bt + T, -1);
+    buni.resize(bu + ucap, -1);
+    bloc.resize(bl + size_t(NM2L) * T, short(-1));
+    int nu = 0;
+    for (int u : cur_u) {
+      buni[bu + lidx[u]] = c->h_src_slot[u];
+      nu = std::max(nu, lidx[u] + 1);
+    }
+    // lane placement: preferred position, else the first free one
+    std::vector<int> pos(cur_t.size(), -1), cubes;
+    std::vector<char> used(T, 0);
+    for (size_t jt = 0; jt < cur_t.size(); jt++) {
+      const int node = c->h_m2l_trg[cur_t[jt]];
+      const int* q = &c->h_lat[3 * size_t(node)];
+      // the cube's key: its position (10 bits of each coordinate tell the cubes of a block apart) and level
+      const int key = ((q[0] >> 2) & 511) | ((q[1] >> 2) & 511) << 9 | ((q[2] >> 2) & 511) << 18 | (c->h_level[node] & 15) << 27;
+      size_t k = std::find(cubes.begin(), cubes.end(), key) - cubes.begin();
+      if (k == cubes.size()) cubes.push_back(key);
+      if (int(64 * k) >= T) continue;
+      const int want = int(64 * k) + 16 * (((q[1] >> 1) & 1) + 2 * ((q[2] >> 1) & 1)) + (q[0] & 3) + 4 * (q[1] & 1) + 8 * (q[2] & 1);
+      if (!used[want]) { used[want] = 1; pos[jt] = want; }
+    }
+    int nextfree = 0;
+    for (size_t jt = 0; jt < cur_t.size(); jt++) {
+      if (pos[jt] < 0) {
+        while (used[nextfree]) nextfree++;
+        used[nextfree] = 1;
+        pos[jt] = nextfree;
+      }
+      btrg[bt + pos[jt]] = cur_t[jt];
+      for (int r = 0; r < NM2L; r++) {
+        const int sn = c->h_m2l[size_t(cur_t[jt]) * NM2L + r];
+        if (sn >= 0) bloc[bl + size_t(r) * T + pos[jt]] = short(lidx[sn]);
+      }
+    }
+    for (int u : cur_u) lidx[u] = -1;
+    for (int& r : rows) r = 0;
+    bnu.push_back(nu);
+    blev.push_back(c->kind == XFMM_LAPLACE ? 0 : c->h_level[c->h_m2l_trg[cur_t[0]]]);
+    cur_t.clear();
+    cur_u.clear();
+  };
+  for (int i = 0; i < ntrg; i++) {
+    int extra[16] = {0};
+    bool over = false;
+    const int* src = &c->h_m2l[size_t(i) * NM2L];
+    for (int r = 0; r < NM2L; r++) {
+      if (src[r] < 0 || lidx[src[r]] >= 0) continue;
+      // (a source repeated over r is counted twice: conservative)
+      const int col = colour(src[r]);
+      if (rows[col] + ++extra[col] > urows) over = true;
+    }
+    const bool other = c->kind != XFMM_LAPLACE && !cur_t.empty() &&
+                       c->h_level[c->h_m2l_trg[cur_t[0]]] != c->h_level[c->h_m2l_trg[i]];
+    if (int(cur_t.size()) == T || over || other) flush();
+    cur_t.push_back(i);
+    for (int r = 0; r < NM2L; r++) {
+      if (src[r] < 0 || lidx[src[r]] >= 0) continue;
+      const int col = colour(src[r]);
+      lidx[src[r]] = 16 * rows[col]++ + col;
+      cur_u.push_back(src[r]);
+    }
   }
+  flush();
+  HIPCHK(hipStreamSynchronize(c->stream));
+  c->n_m2l_blk = int(bnu.size());
+  c->m2l_blk_trg.upload(btrg, c->stream);
+  c->m2l_blk_uni.upload(buni, c->stream);
+  c->m2l_blk_nu.upload(bnu, c->stream);
+  c->m2l_blk_lev.upload(blev, c->stream);
+  c->m2l_blk_loc.upload(bloc, c->stream);
+  HIPCHK(hipStreamSynchronize(c->stream));
+  c->had_ntrg = T;
+}
+
+// hadamard_product of all levels (after the forward transforms)
+void run_hadamards(xfmm_context* c, const M2LDev& m) {
+  HadBlocks hb;
+  hb.nblk = c->n_m2l_blk;
+  hb.ntrg = c->had_ntrg;
+  hb.trg = c->m2l_blk_trg.ptr;
+  hb.uni = c->m2l_blk_uni.ptr;
+  hb.nunion = c->m2l_blk_nu.ptr;
+  hb.oplev = c->m2l_blk_lev.ptr;
+  hb.loc = c->m2l_blk_loc.ptr;
+  const void* ops = c->f32_m2l ? static_cast<const void*>(c->m2l32.ptr) : static_cast<const void*>(c->m2l64.ptr);
+  launch_hadamard(m, ops, c->f16_had ? c->m2l_hscale.ptr : nullptr, hb, c->tune_kch, had_tiles(c), c->stream);
 }
 
 void op_M2L(xfmm_context* c, bool timed) {
@@ -768,65 +877,40 @@ int xfmm_set_operators(xfmm_context* c, int nlevels, const double* uc2e_u, const
             for (int w = 0; w < vw; w++)
               d[(L * ns2 + size_t(k) * r[L] + n) * vw + w] = d[(L * ns2 + size_t(k) * ns + n) * vw + w];
     };
-    // complex operators: each level's K x N matrix (K rows of N complex
-    // entries, row stride N) -> real 2K x 2N with [[Re, Im], [-Im, Re]]
-    // blocks, levels at a stride of 4 ns^2 doubles (see gemm_op_size)
-    auto expand = [&](const std::vector<double>& d, int K, const std::vector<int>* rk, int N, std::vector<double>& out) {
-      const size_t src_level = size_t(K) * N * 2, dst_level = size_t(K) * N * 4;
-      out.assign(size_t(nlevels) * dst_level, 0.0);
-      for (int L = 0; L < nlevels; L++) {
-        const int n = rk ? (*rk)[L] : N;
-        const double* src = d.data() + size_t(L) * src_level;
-        double* dst = out.data() + size_t(L) * dst_level;
-        for (int k = 0; k < K; k++)
-          for (int j = 0; j < n; j++) {
-            const double re = src[(size_t(k) * n + j) * 2], im = src[(size_t(k) * n + j) * 2 + 1];
-            dst[size_t(2 * k) * (2 * n) + 2 * j] = re;
-            dst[size_t(2 * k) * (2 * n) + 2 * j + 1] = im;
-            dst[size_t(2 * k + 1) * (2 * n) + 2 * j] = -im;
-            dst[size_t(2 * k + 1) * (2 * n) + 2 * j + 1] = re;
-          }
-      }
-    };
-    std::vector<double> h, hx;
-    DevBuf<double> rows;  // one operator in row-major form, all levels
-    // Uploads the K x N operators in src (levels at a stride of lev entries of
+    DevBuf<double> rows;  // one operator in row-major form, all levels (reused in stream order)
+    rows.alloc(size_t(nlevels) * 8 * ns2 * vw);
+    std::vector<std::vector<double>> sent;  // uploaded host arrays, kept until the stream is waited for
+    // Uploads the K x N operators in src (levels at a stride of K N entries of
     // kind T; with rk only the first r columns, with rrow the first r rows are
     // used) and packs them into d (FP64) and / or f (FP32).
     auto put = [&](std::vector<double>& src, int K, int N, const std::vector<int>* rk, const std::vector<int>* rrow,
                    bool want64, bool want32, size_t s64, size_t s32, DevBuf<double>& d, DevBuf<float>& f) {
-      size_t lev = size_t(K) * N * vw;
-      const std::vector<double>* up = &src;
-      if (c->cplx) {
-        expand(src, K, rk, N, hx);
-        up = &hx;
-        lev *= 2;
-      }
-      rows.upload(*up, c->stream);
+      const size_t lev = size_t(K) * N * vw;
+      sent.emplace_back();
+      sent.back().swap(src);
+      HIPCHK(hipMemcpyAsync(rows.ptr, sent.back().data(), sent.back().size() * sizeof(double), hipMemcpyHostToDevice,
+                            c->stream));
       d.release();
       f.release();
       if (want64) d.alloc(size_t(nlevels) * s64);
       if (want32) f.alloc(size_t(nlevels) * s32);
       for (int L = 0; L < nlevels; L++) {
-        const int k = (rrow ? (*rrow)[L] : K) * vw, n = (rk ? (*rk)[L] : N) * vw;
-        if (want64) launch_gemm_pack(false, k, n, rows.ptr + L * lev, d.ptr + L * s64, c->stream);
-        if (want32) launch_gemm_pack(true, k, n, rows.ptr + L * lev, f.ptr + L * s32, c->stream);
+        const int k = rrow ? (*rrow)[L] : K, n = rk ? (*rk)[L] : N;
+        if (want64) launch_gemm_pack(false, c->cplx, k, n, rows.ptr + L * lev, d.ptr + L * s64, c->stream);
+        if (want32) launch_gemm_pack(true, c->cplx, k, n, rows.ptr + L * lev, f.ptr + L * s32, c->stream);
       }
-      HIPCHK(hipStreamSynchronize(c->stream));  // the host and device copies are reused
     };
-    auto put_pinv = [&](const std::vector<int>* rk, const std::vector<int>* rrow, DevBuf<double>& d, DevBuf<float>& f) {
+    std::vector<double> h;
+    auto put_pinv = [&](const double* op, const std::vector<int>* rk, const std::vector<int>* rrow, DevBuf<double>& d,
+                        DevBuf<float>& f) {
+      transpose_set(op, h);
+      if (rk) compact(h, *rk);
       put(h, ns, ns, rk, rrow, !c->f32_pinv, c->f32_pinv, pinv_stride(c, false), pinv_stride(c, true), d, f);
     };
-    transpose_set(uc2e_u, h);
-    compact(h, c->r_up);
-    put_pinv(&c->r_up, nullptr, c->uc2e_uT, c->uc2e_uT32);
-    transpose_set(uc2e_v, h);
-    put_pinv(nullptr, &c->r_up, c->uc2e_vT, c->uc2e_vT32);
-    transpose_set(dc2e_u, h);
-    compact(h, c->r_dn);
-    put_pinv(&c->r_dn, nullptr, c->dc2e_uT, c->dc2e_uT32);
-    transpose_set(dc2e_v, h);
-    put_pinv(nullptr, &c->r_dn, c->dc2e_vT, c->dc2e_vT32);
+    put_pinv(uc2e_u, &c->r_up, nullptr, c->uc2e_uT, c->uc2e_uT32);
+    put_pinv(uc2e_v, nullptr, &c->r_up, c->uc2e_vT, c->uc2e_vT32);
+    put_pinv(dc2e_u, &c->r_dn, nullptr, c->dc2e_uT, c->dc2e_uT32);
+    put_pinv(dc2e_v, nullptr, &c->r_dn, c->dc2e_vT, c->dc2e_vT32);
     // M2Mcat[L]: (8 ns) x ns, row o*ns + k, col n = M2M[L][o][n][k]
     // L2Lcat[L]: ns x (8 ns), row k, col o*ns + n = L2L[L][o][n][k]
     std::vector<double> mm(size_t(nlevels) * 8 * ns2 * vw), ll(size_t(nlevels) * 8 * ns2 * vw);
@@ -845,7 +929,6 @@ int xfmm_set_operators(xfmm_context* c, int nlevels, const double* uc2e_u, const
         c->m2mcat32);
     put(ll, ns, 8 * ns, nullptr, nullptr, t64, c->f32_trans, l2l_stride(c, false), l2l_stride(c, true), c->l2lcat,
         c->l2lcat32);
-    rows.release();
     const size_t msz = size_t(nm2l) * NM2L * c->nfreq * 64 * 2;
     // reference layout uploaded, then expanded on the device into the per-lane
     // MFMA operand form (twice the size) used by the Hadamard kernel
@@ -1074,113 +1157,27 @@ int xfmm_set_tree(xfmm_context* c, const xfmm_tree* t) {
         src_slot[i] = int(srcs.size());
         srcs.push_back(i);
       }
-    // blocks: consecutive targets of one level (Hilbert order), at most 64
-    // targets and HAD_UROWS union rows per colour each (slot and lane
-    // placement rules at HAD_UCAP)
-    auto lattice = [&](int node, int* ijk) {
-      const double h = 2.0 * t->r0 / double(1 << lev[node]);
-      for (int d = 0; d < 3; d++) {
-        const double v = std::floor((t->center[3 * size_t(node) + d] - (t->x0[d] - t->r0)) / h);
-        ijk[d] = int(std::max(0.0, v));
-      }
-    };
-    auto colour = [&](int node) {
-      int q[3];
-      lattice(node, q);
-      return (q[0] + 4 * q[1] + 8 * q[2]) & 15;
-    };
-    std::vector<int> src_colour(srcs.size());
-    for (size_t k = 0; k < srcs.size(); k++) src_colour[k] = colour(srcs[k]);
-    std::vector<int> btrg, buni, bnu;
-    std::vector<short> bloc;
-    c->blk_level_off.assign(D + 2, 0);
-    int nblk = 0;
-    std::vector<int> lidx(std::max<size_t>(1, srcs.size()), -1);  // src slot -> union slot in current block
-    std::vector<int> cur_t, cur_u;
-    int rows[16] = {0};
-    auto flush = [&]() {
-      if (cur_t.empty()) return;
-      const size_t bt = btrg.size(), bu = buni.size(), bl = bloc.size();
-      btrg.resize(bt + 64, -1);
-      buni.resize(bu + HAD_UCAP, -1);
-      bloc.resize(bl + size_t(NM2L) * 64, short(-1));
-      int nu = 0;
-      for (int u : cur_u) {
-        buni[bu + lidx[u]] = u;
-        nu = std::max(nu, lidx[u] + 1);
-      }
-      // lane placement: preferred position, else the first free one
-      std::vector<int> pos(cur_t.size(), -1);
-      bool used[64] = {false};
-      for (size_t jt = 0; jt < cur_t.size(); jt++) {
-        int q[3];
-        lattice(cur_t[jt], q);
-        const int want = 16 * (((q[1] >> 1) & 1) + 2 * ((q[2] >> 1) & 1)) + (q[0] & 3) + 4 * (q[1] & 1) + 8 * (q[2] & 1);
-        if (!used[want]) { used[want] = true; pos[jt] = want; }
-      }
-      int nextfree = 0;
-      for (size_t jt = 0; jt < cur_t.size(); jt++) {
-        if (pos[jt] >= 0) continue;
-        while (used[nextfree]) nextfree++;
-        used[nextfree] = true;
-        pos[jt] = nextfree;
-      }
-      for (size_t jt = 0; jt < cur_t.size(); jt++) {
-        const int node = cur_t[jt];
-        btrg[bt + pos[jt]] = trg_slot[node];
-        for (int r = 0; r < NM2L; r++) {
-          const int sn = t->m2l_source[size_t(node) * NM2L + r];
-          if (sn >= 0) bloc[bl + size_t(r) * 64 + pos[jt]] = short(lidx[src_slot[sn]]);
-        }
-      }
-      for (int u : cur_u) lidx[u] = -1;
-      for (int& r : rows) r = 0;
-      bnu.push_back(nu);
-      nblk++;
-      cur_t.clear();
-      cur_u.clear();
-    };
-    for (int l = 0; l <= D; l++) {
-      c->blk_level_off[l] = nblk;
-      for (int i = lo[l]; i < lo[l + 1]; i++) {
-        if (trg_slot[i] < 0) continue;
-        int extra[16] = {0};
-        bool over = false;
-        for (int r = 0; r < NM2L; r++) {
-          const int sn = t->m2l_source[size_t(i) * NM2L + r];
-          if (sn < 0 || lidx[src_slot[sn]] >= 0) continue;
-          // (a source repeated over r is counted twice: conservative)
-          const int col = src_colour[src_slot[sn]];
-          if (rows[col] + ++extra[col] > HAD_UROWS) over = true;
-        }
-        if (cur_t.size() == 64 || over) flush();
-        cur_t.push_back(i);
-        for (int r = 0; r < NM2L; r++) {
-          const int sn = t->m2l_source[size_t(i) * NM2L + r];
-          if (sn < 0) continue;
-          const int ss = src_slot[sn];
-          if (lidx[ss] < 0) {
-            const int col = src_colour[ss];
-            lidx[ss] = 16 * rows[col]++ + col;
-            cur_u.push_back(ss);
-          }
-        }
-      }
-      flush();
+    c->h_lat.resize(size_t(nn) * 3);
+    for (int i = 0; i < nn; i++) {
+      const double h = 2.0 * t->r0 / double(1 << lev[i]);
+      for (int d = 0; d < 3; d++)
+        c->h_lat[3 * size_t(i) + d] =
+            int(std::max(0.0, std::floor((t->center[3 * size_t(i) + d] - (t->x0[d] - t->r0)) / h)));
     }
-    c->blk_level_off[D + 1] = nblk;
+    c->h_m2l.resize(trgs.size() * NM2L);
+    for (size_t k = 0; k < trgs.size(); k++)
+      std::copy_n(t->m2l_source + size_t(trgs[k]) * NM2L, NM2L, c->h_m2l.begin() + k * NM2L);
+    c->h_m2l_trg = trgs;
+    c->h_src_slot = src_slot;
+    c->had_ntrg = 0;
+    build_had_blocks(c);
     c->n_m2l_src = int(srcs.size());
     c->n_m2l_trg = int(trgs.size());
-    c->n_m2l_blk = nblk;
     c->m2l_src_node.upload(srcs, st);
     c->m2l_trg_node.upload(trgs, st);
     c->m2l_scale.upload(scale, st);
-    c->m2l_blk_trg.upload(btrg, st);
-    c->m2l_blk_uni.upload(buni, st);
-    c->m2l_blk_nu.upload(bnu, st);
-    c->m2l_blk_loc.upload(bloc, st);
     const size_t rb = c->f32_m2l ? 4 : 8;
-    const size_t per = size_t(c->nfreq) * NCHILD * 2 * rb;
+    const size_t per = size_t((c->nfreq + SPEC_K - 1) / SPEC_K * SPEC_K) * NCHILD * 2 * rb;
     c->fft_in.alloc(per * std::max(1, c->n_m2l_src));
     c->fft_out.alloc(per * std::max(1, c->n_m2l_trg));
 
@@ -1485,6 +1482,7 @@ int xfmm_set_tuning(xfmm_context* c, int param, int value) {
     } else if (param == XFMM_TUNE_HAD_GROUPS) {
       require(value == 1 || value == 2 || value == 4, "xfmm_set_tuning: Hadamard groups must be 1, 2 or 4");
       c->tune_groups = value;
+      if (c->have_tree) build_had_blocks(c);
     } else if (param == XFMM_TUNE_HAD_TILES) {
       require(value == 1 || value == 2, "xfmm_set_tuning: Hadamard tiles per wave must be 1 or 2");
       c->tune_tiles = value;
@@ -1497,10 +1495,10 @@ int xfmm_set_tuning(xfmm_context* c, int param, int value) {
 
 int xfmm_get_tuning(const xfmm_context* c, int param, int* value) {
   if (!c || !value) return fail(nullptr, XFMM_ERR_ARG, "xfmm_get_tuning: null argument");
-  if (param == XFMM_TUNE_HAD_KCH) *value = c->tune_kch;
+  if (param == XFMM_TUNE_HAD_KCH) *value = c->tune_kch > 0 ? c->tune_kch : HAD_KCH;
   else if (param == XFMM_TUNE_P2P_SPLIT) *value = c->tune_split;
-  else if (param == XFMM_TUNE_HAD_GROUPS) *value = c->tune_groups;
-  else if (param == XFMM_TUNE_HAD_TILES) *value = c->tune_tiles;
+  else if (param == XFMM_TUNE_HAD_GROUPS) *value = had_groups(c);
+  else if (param == XFMM_TUNE_HAD_TILES) *value = had_tiles(c);
   else return fail(const_cast<xfmm_context*>(c), XFMM_ERR_ARG, "xfmm_get_tuning: unknown parameter");
   return XFMM_OK;
 }
@@ -1583,6 +1581,7 @@ int xfmm_autotune(xfmm_context* c, int reps, double* best_ms) {
           if (ngr > 1) {
             c->tune_groups = (gi & 1) ? 2 : 1;
             c->tune_tiles = (gi & 2) ? 2 : 1;
+            build_had_blocks(c);
           }
           const double ms = time_it([&] { run_hadamards(c, m); });
           if (ms < bt) {
@@ -1595,6 +1594,7 @@ int xfmm_autotune(xfmm_context* c, int reps, double* best_ms) {
       c->tune_kch = best;
       c->tune_groups = bestg;
       c->tune_tiles = bestt;
+      build_had_blocks(c);
       ms_kch = bt;
     }
     launch_zero(c->near.ptr, c->near.n, c->stream);

@@ -64,7 +64,9 @@ size_t gemm_packed_size(bool f32, int k, int n) {
   return packed_off((k + KB - 1) / KB, KL, (n + 63) / 64 * 64, 0, 0);
 }
 
-template <typename CT>
+// k, n: sizes of the real form; CPLX: B holds k / 2 x n / 2 complex entries,
+// each the real block [[Re, Im], [-Im, Re]].
+template <typename CT, bool CPLX>
 __global__ void k_gemm_pack(int k, int n, const double* __restrict__ B, CT* __restrict__ out, size_t total) {
   constexpr int KB = GemmMfma<CT>::KB, KL = GemmMfma<CT>::KL;
   const int nkb = (k + KB - 1) / KB;
@@ -74,16 +76,27 @@ __global__ void k_gemm_pack(int k, int n, const double* __restrict__ B, CT* __re
     const size_t gk = e / (KL * 256);  // column group * nkb + kb
     const int kk = int(gk % nkb) * KB + KL * (lane >> 4) + s;
     const int cc = int(gk / nkb) * 64 + ct * 16 + (lane & 15);
-    out[e] = (kk < k && cc < n) ? CT(B[size_t(kk) * n + cc]) : CT(0);
+    double v = 0;
+    if (kk < k && cc < n) {
+      if constexpr (CPLX) {
+        const double* z = B + (size_t(kk / 2) * (n / 2) + cc / 2) * 2;
+        v = ((kk ^ cc) & 1) == 0 ? z[0] : (kk & 1) ? -z[1] : z[1];
+      } else {
+        v = B[size_t(kk) * n + cc];
+      }
+    }
+    out[e] = CT(v);
   }
 }
 
-void launch_gemm_pack(bool f32, int k, int n, const double* B, void* out, hipStream_t s) {
+void launch_gemm_pack(bool f32, bool cplx, int k, int n, const double* B, void* out, hipStream_t s) {
+  if (cplx) k *= 2, n *= 2;
   const size_t total = gemm_packed_size(f32, k, n);
   if (total == 0) return;
   const dim3 g(unsigned(std::min<size_t>((total + 255) / 256, 65536))), b(256);
-  if (f32) hipLaunchKernelGGL(k_gemm_pack<float>, g, b, 0, s, k, n, B, static_cast<float*>(out), total);
-  else hipLaunchKernelGGL(k_gemm_pack<double>, g, b, 0, s, k, n, B, static_cast<double*>(out), total);
+  auto go = [&](auto kern, auto* o) { hipLaunchKernelGGL(kern, g, b, 0, s, k, n, B, o, total); };
+  if (f32) cplx ? go(k_gemm_pack<float, true>, static_cast<float*>(out)) : go(k_gemm_pack<float, false>, static_cast<float*>(out));
+  else cplx ? go(k_gemm_pack<double, true>, static_cast<double*>(out)) : go(k_gemm_pack<double, false>, static_cast<double*>(out));
 }
 
 // A wave computes a (16 TA) x (16 TB) tile of C; a workgroup is RW x CW such

@@ -104,9 +104,10 @@ struct GemmGroup {
 void launch_gemm_rows(bool f32, const GemmGroup& G, const double* A, const long* arow, const void* B, double* C,
                       const long* crow, int beta, hipStream_t s);
 // Packed MFMA operand form of a row-major k x n matrix B (out: float with
-// f32, else double), gemm_packed_size entries.
+// f32, else double), gemm_packed_size entries; with cplx B has k x n complex
+// entries and the packed form is that of its 2k x 2n real blocks.
 size_t gemm_packed_size(bool f32, int k, int n);
-void launch_gemm_pack(bool f32, int k, int n, const double* B, void* out, hipStream_t s);
+void launch_gemm_pack(bool f32, bool cplx, int k, int n, const double* B, void* out, hipStream_t s);
 
 // M2L stages.
 struct M2LDev {
@@ -117,44 +118,58 @@ struct M2LDev {
   const int* map_up = nullptr;       // [nsurf] local index x + p (y + p z) in the [0,p)^3 input cube
   const int* map_dn = nullptr;       // [nsurf] local index in the [p,2p)^3 output cube (offset p removed)
   const int* inv_dn = nullptr;       // [p^3] inverse of map_dn: surface index of a cube point, or -1
-  void* fft_in = nullptr;            // [nsrc_slots][nfreq][8] complex
-  void* fft_out = nullptr;           // [ntrg_slots][nfreq][8] complex
+  // Spectra: [frequency / SPEC_K][slot][SPEC_K][8 children] complex.  The
+  // Hadamard product walks frequencies with a few hundred slots at a time:
+  // in this order those lie in one region of a few MB (with a slot's whole
+  // spectrum contiguous, 280 KB at p = 10, every slot is another page and DRAM
+  // row).
+  void* fft_in = nullptr;            // nsrc slots
+  void* fft_out = nullptr;           // ntrg slots
+  int nsrc = 0, ntrg = 0;
   unsigned* amax = nullptr;          // split-FP16 Hadamard: largest |spectrum value| (float bits), else null
 };
+
+constexpr int SPEC_K = 16;
+// spectrum values (of 8 children each) before frequency k of a slot
+__host__ __device__ __forceinline__ size_t spec_off(int nslots, int slot, int k) {
+  return (size_t(k / SPEC_K) * nslots + slot) * SPEC_K + k % SPEC_K;
+}
 
 // fft_up_equiv: one (source slot, child) per work item; src_node[slot] gives
 // the node whose 8 children are transformed.
 void launch_fft_up(const M2LDev& m, const DevTree& t, const int* src_node, int nslots, hipStream_t s);
-// hadamard_product over blocks of <= 64 M2L targets of one operator level.
-// Block b: trg[b][64] target slots (-1 = padding), uni[b][HAD_UCAP] source
-// slots of the union of the block's sources (nunion[b] used), loc[b][26][64]
-// local union index of the source of target t for relative position r (-1 =
-// none).
+// hadamard_product over blocks of <= ntrg M2L targets of one operator level.
+// Block b: trg[b][ntrg] target slots (-1 = padding), uni[b][ucap] source
+// slots of the union of the block's sources (slots below nunion[b] used; ucap
+// = had_ucap(ntrg)), loc[b][26][ntrg] local union index of the source of target
+// t for relative position r (-1 = none), oplev[b] operator level.
 // Union slots of a block: slot = 16 row + colour, colour = (x + 4 y + 8 z) mod 16
-// of the source's lattice position at its level, at most HAD_UROWS rows.
+// of the source's lattice position at its level.
 // Targets sit at lane (x mod 4) + 4 (y mod 2) + 8 (z mod 2) of tile
-// (y / 2 mod 2) + 2 (z / 2 mod 2) where that is free, so that the 16 sources a
-// wave gathers for one relative position fall on 16 different colours (LDS
-// banks).
-constexpr int HAD_UROWS = 18;
-constexpr int HAD_UCAP = 16 * HAD_UROWS;  // union slots per block (LDS staging)
-constexpr int HAD_KCH = 16;    // default frequencies per workgroup (tunable per context)
+// (y / 2 mod 2) + 2 (z / 2 mod 2) + 4 (number of their 4 x 4 x 4 cube in the
+// block) where that is free, so that the 16 sources a wave gathers for one
+// relative position fall on 16 different colours (LDS banks).
+// The cap holds the sources of a full block of cubes in the uniform tree: 6^3
+// (64 targets), 6 x 6 x 10 (128) and 6 x 10 x 10 (256), with room for uneven
+// colours.
+constexpr int had_urows(int ntrg) { return ntrg <= 64 ? 18 : ntrg <= 128 ? 26 : 40; }
+constexpr int had_ucap(int ntrg) { return 16 * had_urows(ntrg); }
+constexpr int HAD_KCH = 16;    // largest default of the frequencies per workgroup (tunable per context)
 struct HadBlocks {
-  int nblk = 0;
+  int nblk = 0, ntrg = 64;
   const int* trg = nullptr;
   const int* uni = nullptr;
   const int* nunion = nullptr;
+  const int* oplev = nullptr;
   const short* loc = nullptr;
 };
-// m2l_opsx: operators of the level in the expanded MFMA form of launch_m2l_expand
+// m2l_opsx: operators of all levels in the expanded MFMA form of launch_m2l_expand
 // hscale != null (mixed, with m.amax set): split-FP16 operators of
 // launch_m2l_expand with their per-frequency scales, spectra scaled by *m.amax
-// kch: frequencies per workgroup (<= 0: HAD_KCH); groups: 64-target blocks
-// per workgroup of the split-FP16 kernel (1, 2 or 4; they share the staged
-// operators of a frequency); tiles: 16-target tiles per wave of that kernel
-// (1 or 2; a wave's tiles share the operator operands it reads)
+// kch: frequencies per workgroup (<= 0: chosen from the grid); tiles: 16-target
+// tiles per wave (1 or 2; a wave's tiles share the operator operands it reads)
 void launch_hadamard(const M2LDev& m, const void* m2l_opsx, const float* hscale, const HadBlocks& hb, int kch,
-                     int groups, int tiles, hipStream_t s);
+                     int tiles, hipStream_t s);
 // Expand nlev operator levels from the reference layout [L][26][nfreq][64]
 // complex into the per-lane MFMA A-operand form [L][nfreq][26][64 lanes][4]
 // (float for the mixed path, else double), frequencies in the order of the

@@ -29,6 +29,7 @@ namespace xfmm {
 template <typename R>
 struct C2 { R x, y; };
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 
 template <typename R>
 __device__ __forceinline__ C2<R> cmul(C2<R> a, C2<R> b) {
@@ -117,13 +118,13 @@ __global__ __launch_bounds__(256) void k_fft_up(M2LDev m, DevTree t, const int* 
   }
   __syncthreads();
   // z pass straight to global: f = kx + nh*(ky + n1*kz)
-  C2<R>* out = reinterpret_cast<C2<R>*>(m.fft_in) + size_t(slot) * m.nfreq * NCHILD;
+  C2<R>* out = reinterpret_cast<C2<R>*>(m.fft_in);
   float mx = 0.f;
   for (int f = threadIdx.x; f < m.nfreq; f += blockDim.x) {
     const int kx = f % nh, ky = (f / nh) % n1, kz = f / (nh * n1);
     C2<R> acc{0, 0};
     for (int z = 0; z < p; z++) cfma(acc, B[(z * n1 + ky) * nh + kx], w[(kz * z) % n1]);
-    out[size_t(f) * NCHILD + c] = acc;
+    out[spec_off(m.nsrc, slot, f) * NCHILD + c] = acc;
     mx = fmaxf(mx, fmaxf(fabsf(float(acc.x)), fabsf(float(acc.y))));
   }
   if (m.amax) wave_amax(mx, m.amax);
@@ -144,14 +145,14 @@ __global__ __launch_bounds__(256) void k_ifft_dn(M2LDev m, DevTree t, const int*
   R* g = reinterpret_cast<R*>(Bp);                 // p^3 output cube (x2 complex), reuses Bp
   make_twiddles(w, n1, +1);
   __syncthreads();
-  const C2<R>* in = reinterpret_cast<const C2<R>*>(m.fft_out) + size_t(slot) * m.nfreq * NCHILD;
+  const C2<R>* in = reinterpret_cast<const C2<R>*>(m.fft_out);
   // inverse z pass for z' = p + zz
   for (int e = threadIdx.x; e < p * n1 * nh; e += blockDim.x) {
     const int kx = e % nh, ky = (e / nh) % n1, zz = e / (nh * n1);
     const int z = p + zz;
     C2<R> acc{0, 0};
     for (int kz = 0; kz < n1; kz++)
-      cfma(acc, in[size_t(kx + nh * (ky + n1 * kz)) * NCHILD + c], w[(kz * z) % n1]);
+      cfma(acc, in[spec_off(m.ntrg, slot, kx + nh * (ky + n1 * kz)) * NCHILD + c], w[(kz * z) % n1]);
     Bp[e] = acc;
   }
   __syncthreads();
@@ -255,10 +256,11 @@ static void node_dispatch(int p, F&& f) {
 // j2 in {g, g+4} (g = lane/16, j1 = lane%8); the B fragment needs the input
 // children g and g+4 of the lane's target source.
 //
-// Workgroup = one block of <= 64 M2L targets (4 waves x 16-target tiles) and
-// a chunk of kch frequencies (HAD_KCH unless tuned).  The union of the block's M2L sources (<= HAD_UCAP) is
-// staged in LDS one frequency at a time, so each source vector is read from
-// HBM once per block and reused by every target of the block that needs it.
+// Workgroup = one block of M2L targets (64, 128 or 256, in tiles of 16) and a
+// chunk of kch frequencies.  The union of the block's M2L sources (at most
+// had_ucap) is staged in LDS one frequency at a time, so each source vector is
+// read from HBM once per block and reused by every target of the block that
+// needs it.
 // Grid order is XCD aware: the workgroups of one frequency chunk run on the
 // same XCD, so that chunk's operator slice is fetched into one L2 once and
 // reused by all target blocks.
@@ -423,30 +425,27 @@ void launch_m2l_expand(const M2LDev& m, int nlev, const void* M, void* X, float*
                        static_cast<const double*>(M), static_cast<double*>(X));
 }
 
-// Per block of <= 64 target slots and a chunk of kch frequencies.  For
-// each frequency the block stages in LDS the spectra of its source union,
-// arranged so that every lane fetches its B operands for one relative
-// position with one 16-byte read: [g][union slot] = {Re c_g, Im c_g,
-// Re c_(g+4), Im c_(g+4)}, and the 26 operators in the expanded form above
-// (one 16-byte read per lane and relative position).  All staging moves
-// 16-byte vectors (no LDS bank conflicts on the stores), and the next
-// frequency's data is loaded into registers while the current one computes.
-// Each wave owns 16 targets; per
-// relative position the complex 8x8 product is one real 16x16x16 product
-// (four 16x16x4 MFMAs) whose rows are (Re or Im, target child) in HadRow
-// order.  A lane's union index for each relative position is fixed
-// for the block and held in registers; an absent source points at a zero
-// slot, so the 26 relative positions run without branches.
-template <typename R>
-__global__ __launch_bounds__(256) void k_hadamard(M2LDev m, const R* __restrict__ opsx, HadBlocks hb, int nchunk, int kch) {
+// k_hadamard (FP64, or FP32 spectra without the FP16 split): a workgroup of NW
+// waves owns a block of 16 NW TPW targets and kch frequencies.  Per frequency
+// the spectra of the block's source union are staged in LDS, arranged so that
+// every lane fetches its B operands for one relative position with one read:
+// [g][union slot] = {Re c_g, Im c_g, Re c_(g+4), Im c_(g+4)}; the next
+// frequency's spectra are loaded into registers while the current one
+// computes.  The operators come straight from global memory (L2), PFA
+// relative positions ahead, and are applied to the wave's TPW tiles of 16
+// targets; per relative position and tile the complex 8x8 product is one real
+// 16x16x16 product (four 16x16x4 MFMAs) whose rows are (Re or Im, target
+// child) in HadRow order.  A lane's union index for each relative position is
+// fixed for the block and held in registers; an absent source points at a zero
+// slot, and a position that no target of the wave has is left out.
+template <typename R, int NW, int TPW>
+__global__ __launch_bounds__(64 * NW) void k_hadamard(M2LDev m, const R* __restrict__ opsx, HadBlocks hb, int nchunk,
+                                                      int kch) {
   typedef typename MfmaT<R>::v4 v4;
   typedef typename Quad<R>::t q4;
-  constexpr int US = HAD_UCAP + 1;
-  // FP64 reads its operators straight from global memory (L1 / L2): staged,
-  // they would not leave room for a second workgroup per CU
-  constexpr bool STAGE_M = std::is_same<R, float>::value;
-  __shared__ q4 Us[4 * US];                   // [g][union slot]; slot HAD_UCAP stays zero
-  __shared__ q4 Ms[STAGE_M ? NM2L * 64 : 1];  // [r][lane]: A operands of the frequency
+  constexpr int NT = 64 * NW, T = 16 * NW * TPW, UCAP = had_ucap(T), US = UCAP + 1;
+  constexpr int PFA = 4;
+  __shared__ q4 Us[4 * US];  // [g][union slot]; slot UCAP stays zero
   // XCD-aware (chunk, block) mapping: XCD x = w % 8 owns chunks x, x+8, ...
   const int w = blockIdx.x;
   const int x = w & 7, i = w >> 3;
@@ -455,91 +454,95 @@ __global__ __launch_bounds__(256) void k_hadamard(M2LDev m, const R* __restrict_
   if (chunk >= nchunk) return;
   const int kbeg = chunk * kch, kend = min(m.nfreq, kbeg + kch);
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 15, g = lane >> 4;
   const int nu = hb.nunion[b];
-  if (tid < 4) Us[tid * US + HAD_UCAP] = q4{0, 0, 0, 0};
-  int uoff[NM2L];
+  if (tid < 4) Us[tid * US + UCAP] = q4{0, 0, 0, 0};
+  // tile t of this wave: targets (NW t + wave) 16 + j of the block
+  int uoff[TPW][NM2L], trg[TPW];
+  unsigned have = 0;  // relative positions that some target of the wave has
 #pragma unroll
-  for (int r = 0; r < NM2L; r++) {
-    const int u = hb.loc[(size_t(b) * NM2L + r) * 64 + wave * 16 + j];
-    uoff[r] = g * US + (u >= 0 ? u : HAD_UCAP);
+  for (int t = 0; t < TPW; t++) {
+    const int tt = (NW * t + wave) * 16 + j;
+#pragma unroll
+    for (int r = 0; r < NM2L; r++) {
+      const int u = hb.loc[(size_t(b) * NM2L + r) * T + tt];
+      uoff[t][r] = g * US + (u >= 0 ? u : UCAP);
+      have |= __any(u >= 0) ? 1u << r : 0u;
+    }
+    trg[t] = hb.trg[size_t(b) * T + tt];
   }
+  have = __builtin_amdgcn_readfirstlane(have);
   const C2<R>* fin = reinterpret_cast<const C2<R>*>(m.fft_in);
   C2<R>* fout = reinterpret_cast<C2<R>*>(m.fft_out);
-  const q4* X = reinterpret_cast<const q4*>(opsx);
-  // staging: element e = tid + 256 q (q < 4) is slot e / 4, pair g' = e % 4
-  // (children g' and g' + 4)
-  constexpr int NU_Q = (HAD_UCAP * 4 + 255) / 256;
+  const q4* X = reinterpret_cast<const q4*>(opsx) + size_t(hb.oplev[b]) * m.nfreq * NM2L * 64;
+  // staging: element e = tid + NT q is slot e / 4, pair g' = e % 4 (children
+  // g' and g' + 4)
+  constexpr int NU_Q = (UCAP * 4 + NT - 1) / NT;
   const int gp = tid & 3;
   int usrc[NU_Q];
 #pragma unroll
   for (int q = 0; q < NU_Q; q++) {
-    const int e = tid + 256 * q;
-    usrc[q] = (e < nu * 4) ? hb.uni[size_t(b) * HAD_UCAP + (e >> 2)] : -1;
+    const int e = tid + NT * q;
+    usrc[q] = (e < nu * 4) ? hb.uni[size_t(b) * UCAP + (e >> 2)] : -1;
   }
-  constexpr int NM_Q = (NM2L * 64 + 255) / 256;
   C2<R> ra[NU_Q], rb[NU_Q];
-  q4 rm[NM_Q];
   auto fetch = [&](int k) {
 #pragma unroll
     for (int q = 0; q < NU_Q; q++)
       if (usrc[q] >= 0) {
-        const C2<R>* f = fin + (size_t(usrc[q]) * m.nfreq + k) * NCHILD;
+        const C2<R>* f = fin + spec_off(m.nsrc, usrc[q], k) * NCHILD;
         ra[q] = f[gp];
         rb[q] = f[gp + 4];
       }
-    if constexpr (STAGE_M) {
-      const q4* xk = X + size_t(k) * NM2L * 64;
-#pragma unroll
-      for (int q = 0; q < NM_Q; q++)
-        if (tid + 256 * q < NM2L * 64) rm[q] = xk[tid + 256 * q];
-    }
   };
-  const bool im_out = j >= 8;
-  (void)im_out;
-  const int trg = hb.trg[size_t(b) * 64 + wave * 16 + j];
   fetch(kbeg);
   for (int k = kbeg; k < kend; k++) {
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < NU_Q; q++)
-      if (usrc[q] >= 0) Us[gp * US + ((tid + 256 * q) >> 2)] = q4{ra[q].x, ra[q].y, rb[q].x, rb[q].y};
-    if constexpr (STAGE_M) {
-#pragma unroll
-      for (int q = 0; q < NM_Q; q++)
-        if (tid + 256 * q < NM2L * 64) Ms[tid + 256 * q] = rm[q];
-    }
+      if (usrc[q] >= 0) Us[gp * US + ((tid + NT * q) >> 2)] = q4{ra[q].x, ra[q].y, rb[q].x, rb[q].y};
     __syncthreads();
     if (k + 1 < kend) fetch(k + 1);
-    // two accumulators (even / odd r); operands of r + 1 read while r computes
-    v4 acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
-    const q4* Ma = STAGE_M ? Ms : X + size_t(k) * NM2L * 64;
-    q4 mm = Ma[lane];
-    q4 vv = Us[uoff[0]];
+    v4 acc[TPW];
 #pragma unroll
-    for (int r = 0; r < NM2L; r++) {
-      q4 mn = mm, vn = vv;
-      if (r + 1 < NM2L) {
-        mn = Ma[(r + 1) * 64 + lane];
-        vn = Us[uoff[r + 1]];
+    for (int t = 0; t < TPW; t++) acc[t] = v4{0, 0, 0, 0};
+    const q4* Ma = X + size_t(k) * NM2L * 64 + lane;
+    auto mul = [&](int r, const q4& a) {
+#pragma unroll
+      for (int t = 0; t < TPW; t++) {
+        const q4 vv = Us[uoff[t][r]];
+        acc[t] = MfmaT<R>::mma(a.x, vv.x, acc[t]);
+        acc[t] = MfmaT<R>::mma(a.y, vv.z, acc[t]);
+        acc[t] = MfmaT<R>::mma(a.z, vv.y, acc[t]);
+        acc[t] = MfmaT<R>::mma(a.w, vv.w, acc[t]);
       }
-      v4& acc = (r & 1) ? acc1 : acc0;
-      acc = MfmaT<R>::mma(mm.x, vv.x, acc);
-      acc = MfmaT<R>::mma(mm.y, vv.z, acc);
-      acc = MfmaT<R>::mma(mm.z, vv.y, acc);
-      acc = MfmaT<R>::mma(mm.w, vv.w, acc);
-      mm = mn;
-      vv = vn;
+    };
+    if (have == (1u << NM2L) - 1) {
+      q4 ring[PFA];
+#pragma unroll
+      for (int r = 0; r < PFA; r++) ring[r] = Ma[r * 64];
+#pragma unroll
+      for (int r = 0; r < NM2L; r++) {
+        const q4 a = ring[r % PFA];
+        if (r + PFA < NM2L) ring[r % PFA] = Ma[(r + PFA) * 64];
+        mul(r, a);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < NM2L; r++)
+        if (have >> r & 1) mul(r, Ma[r * 64]);
     }
-    const v4 acc = acc0 + acc1;
     // result: lane (g, j) register q holds row MfmaT::row(g, q) of target j,
     // registers (0, 1) and (2, 3) the (Re, Im) of one child each (HadRow)
-    if (trg >= 0) {
-      C2<R>* o = fout + (size_t(trg) * m.nfreq + k) * NCHILD;
-      o[HadRow<R>::child(MfmaT<R>::row(g, 0))] = C2<R>{acc[0], acc[1]};
-      o[HadRow<R>::child(MfmaT<R>::row(g, 2))] = C2<R>{acc[2], acc[3]};
-    }
+#pragma unroll
+    for (int t = 0; t < TPW; t++)
+      if (trg[t] >= 0) {
+        C2<R>* o = fout + spec_off(m.ntrg, trg[t], k) * NCHILD;
+        o[HadRow<R>::child(MfmaT<R>::row(g, 0))] = C2<R>{acc[t][0], acc[t][1]};
+        o[HadRow<R>::child(MfmaT<R>::row(g, 2))] = C2<R>{acc[t][2], acc[t][3]};
+      }
   }
 }
 
@@ -555,130 +558,229 @@ __global__ __launch_bounds__(256) void k_hadamard(M2LDev m, const R* __restrict_
 // take source children 0..3 / 4..7 of position 2 pm, groups 2, 3 those of
 // 2 pm + 1 (A layout of k_m2l_expand_h); the B operand of a lane is the
 // matching 4 children (re, im) of its target's source, staged in LDS as
-// [term][h][union slot] 16-byte vectors.  Blocks, union staging, grid order
-// and result layout are those of k_hadamard.
-template <int GPB, int TPW>
-__global__ __launch_bounds__(256 * GPB / TPW) void k_hadamard_h(M2LDev m, const h8* __restrict__ X,
-                                                                const float* __restrict__ hscale, HadBlocks hb,
-                                                                int nchunk, int kch) {
+// [term][h][union slot] 16-byte vectors.  Blocks, grid order and result
+// layout are those of k_hadamard, except that the operators of a frequency
+// are staged in LDS too and that two LDS buffers alternate: while a frequency
+// computes, the next one's operands arrive in registers, are split and go to
+// the other buffer, with one barrier per frequency.
+// What bounds it (N = 2M, p = 10: 4680 targets, 4400 frequencies; the 2.7 GB of
+// spectra and operators take 0.55 ms at the rate of a large copy): staging
+// (loads, split, LDS stores, results: 0.95 ms alone) beside the matrix
+// products with their LDS reads (0.87 ms alone).  Measured there: blocks of
+// 64 targets, one LDS buffer, two blocks per workgroup 1.37 ms; 256
+// targets, two buffers, 16 waves of a tile 1.49; half of the waves staging
+// before they compute 1.38; frequency pairs as whole 128-byte lines
+// 1.35, 8 waves of two tiles 1.19; operands read a position pair ahead 1.08 ms.
+template <int NW, int TPW>
+__global__ __launch_bounds__(64 * NW) void k_hadamard_h(M2LDev m, const h8* __restrict__ opsx,
+                                                        const float* __restrict__ hscale, HadBlocks hb, int nchunk,
+                                                        int kch) {
   typedef float v4 __attribute__((ext_vector_type(4)));
-  constexpr int US = HAD_UCAP + 1;
-  constexpr int NP = NM2L / 2;
-  static_assert(TPW == 1 || TPW == 2, "tiles per wave");
-  constexpr int TPB = 256 / TPW;    // threads per target block: 4 / TPW waves of TPW 16-target tiles
-  constexpr int NT = TPB * GPB;
-  __shared__ h8 Us[GPB][4 * US];    // per target block: [term][h][union slot]; slot HAD_UCAP stays zero
-  __shared__ h8 Ms[NP * 2 * 64];    // [pair][term][lane], shared by the GPB target blocks
-  const int nbg = (hb.nblk + GPB - 1) / GPB;
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  constexpr int NT = 64 * NW, T = 16 * NW * TPW, UCAP = had_ucap(T), US = UCAP + 1;
+  constexpr int NP = NM2L / 2, MS = NP * 2 * 64;
+  constexpr int BUF = 4 * US + MS;  // one buffer: [term][h][union slot], then [pair][term][lane]
+  extern __shared__ h8 had_smem[];  // slot UCAP of each [term][h] stays zero
   const int w = blockIdx.x;
   const int x = w & 7, i = w >> 3;
-  const int chunk = (i / nbg) * 8 + x;
+  const int chunk = (i / hb.nblk) * 8 + x;
+  const int b = i % hb.nblk;
   if (chunk >= nchunk) return;
   const int kbeg = chunk * kch, kend = min(m.nfreq, kbeg + kch);
-  const int tid = threadIdx.x, sub = tid / TPB, st = tid % TPB;
-  const int lane = tid & 63, wave = st >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 15, g = lane >> 4;
-  const int b = (i % nbg) * GPB + sub;
-  const bool live = b < hb.nblk;  // the last workgroup may hold fewer than GPB target blocks
-  const int nu = live ? hb.nunion[b] : 0;
-  h8* U = Us[sub];
-  if (st < 4) U[st * US + HAD_UCAP] = h8{0, 0, 0, 0, 0, 0, 0, 0};
-  // tile t of this wave: targets (TPW wave + t) 16 + j of the block
-  int uoff[TPW][NP];
-  int trg[TPW];
+  const int nu = hb.nunion[b];
+  if (tid < 8) had_smem[(tid >> 2) * BUF + (tid & 3) * US + UCAP] = h8{0, 0, 0, 0, 0, 0, 0, 0};
+  // tile t of this wave: targets (NW t + wave) 16 + j of the block
+  int uoff[TPW][NP], trg[TPW];
+  unsigned have = 0;  // pairs of relative positions that some target of the wave has
 #pragma unroll
   for (int t = 0; t < TPW; t++) {
-    const int tt = (TPW * wave + t) * 16 + j;
+    const int tt = (NW * t + wave) * 16 + j;
 #pragma unroll
     for (int pm = 0; pm < NP; pm++) {
-      const int u = live ? hb.loc[(size_t(b) * NM2L + 2 * pm + (g >> 1)) * 64 + tt] : -1;
-      uoff[t][pm] = (g & 1) * US + (u >= 0 ? u : HAD_UCAP);
+      const int u = hb.loc[(size_t(b) * NM2L + 2 * pm + (g >> 1)) * T + tt];
+      uoff[t][pm] = (g & 1) * US + (u >= 0 ? u : UCAP);
+      have |= __any(u >= 0) ? 1u << pm : 0u;
     }
-    trg[t] = live ? hb.trg[size_t(b) * 64 + tt] : -1;
+    trg[t] = hb.trg[size_t(b) * T + tt];
   }
+  have = __builtin_amdgcn_readfirstlane(have);
+  // (with few positions missing the pipelined loop over all of them is faster)
+  const bool most = __popc(have) > 8;
   // spectrum scale: largest |value| of this evaluation's spectra -> [2^14, 2^15)
   const float amax = __uint_as_float(*m.amax);
   int ex = 0;
   frexpf(amax, &ex);
   if (!(amax <= 3.0e38f)) ex = 15;
   const float sb = ldexpf(1.f, 15 - ex), isb = ldexpf(1.f, ex - 15);
-  typedef float f4 __attribute__((ext_vector_type(4)));
   const f4* fin = reinterpret_cast<const f4*>(m.fft_in);  // [slot][k][2 halves of 4 children]
   C2<float>* fout = reinterpret_cast<C2<float>*>(m.fft_out);
-  // staging of a target block's union by its TPB threads: element
-  // e = st + TPB q is union slot e / 2, children 4 (e % 2) .. + 3
-  constexpr int NU_Q = (HAD_UCAP * 2 + TPB - 1) / TPB;
-  const int hh = st & 1;
+  const int lev = hb.oplev[b];
+  const h8* X = opsx + size_t(lev) * m.nfreq * MS;
+  const float* hs = hscale + size_t(lev) * m.nfreq;
+  // Frequencies are taken in pairs (k even): a pair of a slot is one 128-byte
+  // line of the spectra, loaded and stored whole.  LDS buffer 0 holds the even
+  // one, buffer 1 the odd one.
+  // Staging of the union: element e = tid + NT q is union slot e / 4, children
+  // 2 (e % 4) and 2 (e % 4) + 1.
+  constexpr int NU_Q = (UCAP * 4 + NT - 1) / NT;
+  constexpr int NM_Q = (MS + NT - 1) / NT;
+  const int qq = tid & 3;
   int usrc[NU_Q];
 #pragma unroll
   for (int q = 0; q < NU_Q; q++) {
-    const int e = st + TPB * q;
-    usrc[q] = (e < nu * 2) ? hb.uni[size_t(b) * HAD_UCAP + (e >> 1)] : -1;
+    const int e = tid + NT * q;
+    usrc[q] = (e < nu * 4) ? hb.uni[size_t(b) * UCAP + (e >> 2)] : -1;
   }
-  // the operators of a frequency, staged once for the GPB target blocks
-  constexpr int NM_Q = (NP * 2 * 64 + NT - 1) / NT;
-  f4 ra[NU_Q], rb[NU_Q];
+  f4 ru[2][NU_Q];
   h8 rm[NM_Q];
-  auto fetch = [&](int k) {
+  auto fetch_u = [&](int k) {
 #pragma unroll
     for (int q = 0; q < NU_Q; q++)
       if (usrc[q] >= 0) {
-        const f4* f = fin + ((size_t(usrc[q]) * m.nfreq + k) * 2 + hh) * 2;
-        ra[q] = f[0];
-        rb[q] = f[1];
+        const f4* f = fin + spec_off(m.nsrc, usrc[q], k) * 4 + qq;
+        ru[0][q] = f[0];
+        ru[1][q] = f[4];
       }
-    const h8* xk = X + size_t(k) * NP * 2 * 64;
+  };
+  auto fetch_m = [&](int k) {
+    const h8* xk = X + size_t(k) * MS;
 #pragma unroll
     for (int q = 0; q < NM_Q; q++)
-      if (tid + NT * q < NP * 2 * 64) rm[q] = xk[tid + NT * q];
+      if (tid + NT * q < MS) rm[q] = xk[tid + NT * q];
   };
-  fetch(kbeg);
-  for (int k = kbeg; k < kend; k++) {
-    __syncthreads();
+  auto stage = [&](h8* U, const f4* r) {
+#pragma unroll
+    for (int q = 0; q < NM_Q; q++)
+      if (tid + NT * q < MS) U[4 * US + tid + NT * q] = rm[q];
 #pragma unroll
     for (int q = 0; q < NU_Q; q++)
       if (usrc[q] >= 0) {
-        h8 hi, lo;
+        h4 hi, lo;
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-          const float v = sb * (e < 4 ? ra[q][e] : rb[q][e - 4]);
+        for (int e = 0; e < 4; e++) {
+          const float v = sb * r[q][e];
           const _Float16 h = _Float16(v);
           hi[e] = h;
           lo[e] = _Float16(v - float(h));
         }
-        const int slot = (st + TPB * q) >> 1;
-        U[hh * US + slot] = hi;
-        U[2 * US + hh * US + slot] = lo;
+        h4* V = reinterpret_cast<h4*>(U + (qq >> 1) * US + ((tid + NT * q) >> 2)) + (qq & 1);
+        V[0] = hi;
+        V[4 * US] = lo;
       }
-#pragma unroll
-    for (int q = 0; q < NM_Q; q++)
-      if (tid + NT * q < NP * 2 * 64) Ms[tid + NT * q] = rm[q];
-    __syncthreads();
-    if (k + 1 < kend) fetch(k + 1);
+  };
+  v4 res[TPW];
+  auto compute = [&](int k, const h8* U) {
+    const h8* Ms = U + 4 * US;
     v4 ahh[TPW], ahl[TPW], alh[TPW];
 #pragma unroll
     for (int t = 0; t < TPW; t++) ahh[t] = ahl[t] = alh[t] = v4{0, 0, 0, 0};
-#pragma unroll
-    for (int pm = 0; pm < NP; pm++) {
-      // the operator pair is read once and applied to the wave's TPW tiles
-      const h8 ah = Ms[(2 * pm) * 64 + lane], al = Ms[(2 * pm + 1) * 64 + lane];
+    // the operator pair is read once and applied to the wave's TPW tiles
+    struct Ops {
+      h8 ah, al, bh[TPW], bl[TPW];
+    };
+    auto read = [&](int pm, Ops& o) {
+      o.ah = Ms[(2 * pm) * 64 + lane];
+      o.al = Ms[(2 * pm + 1) * 64 + lane];
 #pragma unroll
       for (int t = 0; t < TPW; t++) {
-        const h8 bh = U[uoff[t][pm]], bl = U[2 * US + uoff[t][pm]];
-        ahh[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh, ahh[t], 0, 0, 0);
-        ahl[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl, ahl[t], 0, 0, 0);
-        alh[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh, alh[t], 0, 0, 0);
+        o.bh[t] = U[uoff[t][pm]];
+        o.bl[t] = U[2 * US + uoff[t][pm]];
       }
+    };
+    auto mul = [&](const Ops& o) {
+#pragma unroll
+      for (int t = 0; t < TPW; t++) ahh[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.ah, o.bh[t], ahh[t], 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < TPW; t++) ahl[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.ah, o.bl[t], ahl[t], 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < TPW; t++) alh[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.al, o.bh[t], alh[t], 0, 0, 0);
+    };
+    if (most) {
+      // the operands of the next position pair are read while this one multiplies
+      Ops o[2];
+      read(0, o[0]);
+#pragma unroll
+      for (int pm = 0; pm < NP; pm++) {
+        if (pm + 1 < NP) read(pm + 1, o[(pm + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        mul(o[pm & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      Ops o;
+#pragma unroll
+      for (int pm = 0; pm < NP; pm++)
+        if (have >> pm & 1) {
+          read(pm, o);
+          mul(o);
+        }
     }
-    const float sc = hscale[k] * isb;
+    const float sc = hs[k] * isb;
     // lane (g, j) register q holds row 4 g + q of target j: (Re, Im) of
-    // children 2g and 2g + 1, one 16-byte store
+    // children 2g and 2g + 1
+#pragma unroll
+    for (int t = 0; t < TPW; t++) res[t] = (ahh[t] + (ahl[t] + alh[t])) * sc;
+  };
+  // the lane j ^ 8 of the same group of 16
+  auto swap8 = [](int v) { return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, false); };
+  // Half of the waves of each SIMD stage the next frequency before they
+  // compute, half after it, so that the conversions and LDS stores of one half
+  // run beside the matrix products of the other.
+  const bool early = (wave >> 2 & 1) != 0;
+  h8* const U0 = had_smem;
+  h8* const U1 = had_smem + BUF;
+  fetch_u(kbeg);
+  fetch_m(kbeg);
+  stage(U0, ru[0]);
+  fetch_m(kbeg + 1);
+  __syncthreads();
+  for (int k = kbeg; k < kend; k += 2) {
+    const bool more = k + 2 < kend;
+    auto odd = [&]() {  // the odd frequency of this pair; the loads of the next pair
+      stage(U1, ru[1]);
+      if (more) {
+        fetch_u(k + 2);
+        fetch_m(k + 2);
+      }
+    };
+    if (early) odd();
+    compute(k, U0);
+    v4 even[TPW];
+#pragma unroll
+    for (int t = 0; t < TPW; t++) even[t] = res[t];
+    if (!early) odd();
+    __syncthreads();
+    auto next = [&]() {
+      if (more) {
+        stage(U0, ru[0]);
+        fetch_m(k + 3);
+      }
+    };
+    if (early) next();
+    compute(k + 1, U1);
+    // whole lines: lanes j < 8 store the even, lanes j >= 8 the odd frequency,
+    // of targets 0..7 and then of targets 8..15 of the tile
 #pragma unroll
     for (int t = 0; t < TPW; t++) {
-      const v4 acc = (ahh[t] + (ahl[t] + alh[t])) * sc;
-      if (trg[t] >= 0)
-        *reinterpret_cast<v4*>(fout + (size_t(trg[t]) * m.nfreq + k) * NCHILD + 2 * g) = acc;
+      const int other = swap8(trg[t]);
+      v4 x, y;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const float se = __int_as_float(swap8(__float_as_int(even[t][q])));
+        const float so = __int_as_float(swap8(__float_as_int(res[t][q])));
+        x[q] = j < 8 ? even[t][q] : so;
+        y[q] = j < 8 ? se : res[t][q];
+      }
+      const int tx = j < 8 ? trg[t] : other, ty = j < 8 ? other : trg[t];
+      const int kk = k + (j >> 3);
+      if (tx >= 0) *reinterpret_cast<v4*>(fout + spec_off(m.ntrg, tx, kk) * NCHILD + 2 * g) = x;
+      if (ty >= 0) *reinterpret_cast<v4*>(fout + spec_off(m.ntrg, ty, kk) * NCHILD + 2 * g) = y;
     }
+    if (!early) next();
+    __syncthreads();
   }
 }
 
@@ -804,7 +906,7 @@ __global__ __launch_bounds__(256) void k_fft_up_mfma(M2LDev m, DevTree t, const 
       wf[mt][ks] = (f < n1 && k < KK) ? R(dft_entry(f * v, n1, -1, RowMap<R>::ra(j), k & 1)) : R(0);
     }
   __syncthreads();
-  C2<RS>* out = reinterpret_cast<C2<RS>*>(m.fft_in) + size_t(slot) * m.nfreq * NCHILD;
+  C2<RS>* out = reinterpret_cast<C2<RS>*>(m.fft_in);
   float mx = 0.f;
   for (int kx = 0; kx < NKX; kx++) {
     // x: Ay[(y, re/im)][(z, c)] = sum_x gx[c][z][y][x] exp(-2 pi i kx x / n1),
@@ -884,7 +986,7 @@ __global__ __launch_bounds__(256) void k_fft_up_mfma(M2LDev m, DevTree t, const 
           const int kz = mt * 8 + RowMap<R>::fd(g, 2 * h);
           if (kz < n1) {
             const C2<RS> v{RS(acc[2 * h]), RS(acc[2 * h + 1])};
-            out[size_t(kx * n1 * n1 + ky + n1 * kz) * NCHILD + c] = v;
+            out[spec_off(m.nsrc, slot, kx * n1 * n1 + ky + n1 * kz) * NCHILD + c] = v;
             mx = fmaxf(mx, fmaxf(fabsf(float(v.x)), fabsf(float(v.y))));
           }
         }
@@ -956,7 +1058,7 @@ __global__ __launch_bounds__(256) void k_ifft_dn_mfma(M2LDev m, DevTree t, const
     for (int x = 0; x < 2; x++)
 #pragma unroll
       for (int v = 0; v < VW; v++) gs[r][x][v] = R(0);
-  const C2<RS>* in = reinterpret_cast<const C2<RS>*>(m.fft_out) + size_t(slot) * m.nfreq * NCHILD;
+  const C2<RS>* in = reinterpret_cast<const C2<RS>*>(m.fft_out);
   // z-pass input fragments of this wave's tiles, loaded one slab ahead
   RS bz[NTZW][KS];
   auto fetch = [&](int kx) {
@@ -967,7 +1069,7 @@ __global__ __launch_bounds__(256) void k_ifft_dn_mfma(M2LDev m, DevTree t, const
 #pragma unroll
       for (int kp = 0; kp < KS / 2; kp++) {
         C2<RS> v{RS(0), RS(0)};
-        if (nt < NTZ && kp * 4 + g < n1) v = in[size_t(kx * n1 * n1 + ky + n1 * (kp * 4 + g)) * NCHILD + c];
+        if (nt < NTZ && kp * 4 + g < n1) v = in[spec_off(m.ntrg, slot, kx * n1 * n1 + ky + n1 * (kp * 4 + g)) * NCHILD + c];
         bz[s][2 * kp] = v.x;
         bz[s][2 * kp + 1] = v.y;
       }
@@ -1195,36 +1297,55 @@ void launch_ifft_dn(const M2LDev& m, const DevTree& t, const int* trg_node, cons
   }
 }
 
+// Frequencies per workgroup when not tuned: an even number up to HAD_KCH, such
+// that the workgroups fill the chip's slots (`resident` per CU) with the least
+// waste; a workgroup's start (index loads, first staging) costs about as
+// much as two frequencies.
+static int had_kch(const M2LDev& m, const HadBlocks& hb, int kch, int resident) {
+  if (kch >= 1) return kch;
+  int best = 2;
+  long cost = -1;
+  for (int k = 2; k <= HAD_KCH; k += 2) {
+    const long wgs = long((m.nfreq + k - 1) / k) * hb.nblk, rounds = (wgs + 256 * resident - 1) / (256 * resident);
+    const long c = rounds * (k + 2);
+    if (cost < 0 || c <= cost) {
+      cost = c;
+      best = k;
+    }
+  }
+  return best;
+}
+
 void launch_hadamard(const M2LDev& m, const void* m2l_opsx, const float* hscale, const HadBlocks& hb, int kch,
-                     int groups, int tiles, hipStream_t s) {
+                     int tiles, hipStream_t s) {
   if (hb.nblk <= 0) return;
-  if (kch < 1) kch = HAD_KCH;
+  const bool split = m.mixed && hscale && m.amax;
+  kch = had_kch(m, hb, kch, split ? 1 : 3);
+  if (split) kch = (kch + 1) / 2 * 2;  // whole pairs of frequencies (nfreq is even)
   const int nchunk = (m.nfreq + kch - 1) / kch;
-  const int nchunk8 = (nchunk + 7) / 8 * 8;
-  dim3 grid(unsigned(nchunk8) * unsigned(hb.nblk));
-  if (m.mixed && hscale && m.amax) {
-    auto go = [&](auto kern, int gp, int tpw) {
-      dim3 gg(unsigned(nchunk8) * unsigned((hb.nblk + gp - 1) / gp));
-      hipLaunchKernelGGL(kern, gg, dim3(256 * gp / tpw), 0, s, m, static_cast<const h8*>(m2l_opsx), hscale, hb,
-                         nchunk, kch);
+  dim3 grid(unsigned((nchunk + 7) / 8 * 8) * unsigned(hb.nblk));
+  if (split) {
+    auto go = [&](auto kern, int nw) {
+      const size_t lds = 2 * (4 * size_t(had_ucap(hb.ntrg) + 1) + (NM2L / 2) * 2 * 64) * sizeof(h8);
+      allow_lds(kern, lds);
+      hipLaunchKernelGGL(kern, grid, dim3(64 * nw), lds, s, m, static_cast<const h8*>(m2l_opsx), hscale, hb, nchunk,
+                         kch);
     };
-    if (tiles >= 2) {
-      if (groups >= 4) go(k_hadamard_h<4, 2>, 4, 2);
-      else if (groups == 2) go(k_hadamard_h<2, 2>, 2, 2);
-      else go(k_hadamard_h<1, 2>, 1, 2);
+    if (hb.ntrg == 128) {
+      if (tiles >= 2) go(k_hadamard_h<4, 2>, 4);
+      else go(k_hadamard_h<8, 1>, 8);
     } else {
-      if (groups >= 4) go(k_hadamard_h<4, 1>, 4, 1);
-      else if (groups == 2) go(k_hadamard_h<2, 1>, 2, 1);
-      else go(k_hadamard_h<1, 1>, 1, 1);
+      if (tiles >= 2) go(k_hadamard_h<8, 2>, 8);
+      else go(k_hadamard_h<16, 1>, 16);
     }
     return;
   }
-  else if (m.mixed)
-    hipLaunchKernelGGL((k_hadamard<float>), grid, dim3(256), 0, s, m, static_cast<const float*>(m2l_opsx), hb, nchunk,
-                       kch);
-  else
-    hipLaunchKernelGGL((k_hadamard<double>), grid, dim3(256), 0, s, m, static_cast<const double*>(m2l_opsx), hb,
-                       nchunk, kch);
+  auto go = [&](auto kern, int nw, auto ops) {
+    hipLaunchKernelGGL(kern, grid, dim3(64 * nw), 0, s, m, ops, hb, nchunk, kch);
+  };
+  if (m.mixed) go(k_hadamard<float, 4, 1>, 4, static_cast<const float*>(m2l_opsx));
+  else if (tiles >= 2) go(k_hadamard<double, 2, 2>, 2, static_cast<const double*>(m2l_opsx));
+  else go(k_hadamard<double, 4, 1>, 4, static_cast<const double*>(m2l_opsx));
 }
 
 }  // namespace xfmm

@@ -176,17 +176,20 @@ int xfmm_set_value_scale(xfmm_context* ctx, const double* scale);
 /* Launch-shape parameters of one context (no counterpart in the reference,
  * whose loops have fixed blocking; none of them changes which pairs are
  * summed):
- *   XFMM_TUNE_HAD_KCH    frequencies per Hadamard workgroup, 1..256 (default 16)
+ *   XFMM_TUNE_HAD_KCH    frequencies per Hadamard workgroup, 1..256 (default:
+ *                        chosen from the size of the problem, at most 16; the
+ *                        split-FP16 kernel rounds it up to an even number)
  *   XFMM_TUNE_P2P_SPLIT  real kernels: P2P / L2P tail tiles of at most this many
  *                        targets (0..32) split each target's sources over
  *                        several lanes (default 32; the partial sums then add
  *                        in another order)
- *   XFMM_TUNE_HAD_GROUPS split-FP16 Hadamard (mixed / FLOAT): 64-target blocks
- *                        per workgroup, 1, 2 or 4, which share the operators
- *                        staged in LDS for a frequency (default 2)
- *   XFMM_TUNE_HAD_TILES  split-FP16 Hadamard: 16-target tiles per wave, 1 or 2;
- *                        a wave applies each operator operand it reads from
- *                        LDS to all of its tiles (default 1)
+ *   XFMM_TUNE_HAD_GROUPS split-FP16 Hadamard (mixed / FLOAT): 128-target groups
+ *                        per workgroup, 1 or 2 (4 is taken as 2), which share
+ *                        the operators and the union of sources staged in LDS
+ *                        for a frequency (default: 2 from 1024 targets on)
+ *   XFMM_TUNE_HAD_TILES  16-target tiles per wave, 1 or 2; a wave applies each
+ *                        operator operand it reads to all of its tiles
+ *                        (default: from the number of targets)
  * Setting one drops a captured graph. */
 enum { XFMM_TUNE_HAD_KCH = 0, XFMM_TUNE_P2P_SPLIT = 1, XFMM_TUNE_HAD_GROUPS = 2, XFMM_TUNE_HAD_TILES = 3 };
 int xfmm_set_tuning(xfmm_context* ctx, int param, int value);
