@@ -840,15 +840,6 @@ int xfmm_set_operators(xfmm_context* c, int nlevels, const double* uc2e_u, const
     if (c->kind == XFMM_LAPLACE) require(nlevels == 1 && nm2l == 1, "xfmm_set_operators: Laplace operators are scale invariant (nlevels = nm2l = 1)");
     const int ns = c->nsurf, vw = c->vw;
     const size_t ns2 = size_t(ns) * ns;
-    // transposes for row-GEMM: out_row = in_row x op^T
-    auto transpose_set = [&](const double* src, std::vector<double>& dst) {
-      dst.resize(size_t(nlevels) * ns2 * vw);
-      for (int L = 0; L < nlevels; L++)
-        for (int i = 0; i < ns; i++)
-          for (int j = 0; j < ns; j++)
-            for (int w = 0; w < vw; w++)
-              dst[(L * ns2 + size_t(j) * ns + i) * vw + w] = src[(L * ns2 + size_t(i) * ns + j) * vw + w];
-    };
     // Rank of C2E_V = V S^+ per level: 1 + its last column that is not
     // exactly zero (S^+ holds 0 for the truncated singular values, which
     // come last).  The products with the columns past it are exact zeros, so
@@ -869,65 +860,39 @@ int xfmm_set_operators(xfmm_context* c, int nlevels, const double* uc2e_u, const
     };
     rank_of(uc2e_v, c->r_up);
     rank_of(dc2e_v, c->r_dn);
-    // keep the first r columns of each level's transposed C2E_U, row stride r
-    auto compact = [&](std::vector<double>& d, const std::vector<int>& r) {
-      for (int L = 0; L < nlevels; L++)
-        for (int k = 0; k < ns; k++)
-          for (int n = 0; n < r[L]; n++)
-            for (int w = 0; w < vw; w++)
-              d[(L * ns2 + size_t(k) * r[L] + n) * vw + w] = d[(L * ns2 + size_t(k) * ns + n) * vw + w];
-    };
-    DevBuf<double> rows;  // one operator in row-major form, all levels (reused in stream order)
-    rows.alloc(size_t(nlevels) * 8 * ns2 * vw);
-    std::vector<std::vector<double>> sent;  // uploaded host arrays, kept until the stream is waited for
-    // Uploads the K x N operators in src (levels at a stride of K N entries of
-    // kind T; with rk only the first r columns, with rrow the first r rows are
-    // used) and packs them into d (FP64) and / or f (FP32).
-    auto put = [&](std::vector<double>& src, int K, int N, const std::vector<int>* rk, const std::vector<int>* rrow,
+    // Each operator is uploaded as it is and packed for out_row = in_row x op^T
+    // by the device: C2E_U^T (its first r columns), C2E_V^T (its first r rows),
+    // M2Mcat (8 ns x ns, row o ns + k, column n = M2M[o][n][k]) and L2Lcat (ns x
+    // 8 ns, row k, column o ns + n = L2L[o][n][k]), in FP64 and / or FP32.
+    DevBuf<double> raw;  // reused in stream order
+    raw.alloc(size_t(nlevels) * 8 * ns2 * vw);
+    auto put = [&](const double* src, int mats, int K, int N, const std::vector<int>* rk, const std::vector<int>* rrow,
                    bool want64, bool want32, size_t s64, size_t s32, DevBuf<double>& d, DevBuf<float>& f) {
-      const size_t lev = size_t(K) * N * vw;
-      sent.emplace_back();
-      sent.back().swap(src);
-      HIPCHK(hipMemcpyAsync(rows.ptr, sent.back().data(), sent.back().size() * sizeof(double), hipMemcpyHostToDevice,
-                            c->stream));
+      const size_t lev = size_t(mats) * ns2 * vw;
+      HIPCHK(hipMemcpyAsync(raw.ptr, src, size_t(nlevels) * lev * sizeof(double), hipMemcpyHostToDevice, c->stream));
       d.release();
       f.release();
       if (want64) d.alloc(size_t(nlevels) * s64);
       if (want32) f.alloc(size_t(nlevels) * s32);
       for (int L = 0; L < nlevels; L++) {
         const int k = rrow ? (*rrow)[L] : K, n = rk ? (*rk)[L] : N;
-        if (want64) launch_gemm_pack(false, c->cplx, k, n, rows.ptr + L * lev, d.ptr + L * s64, c->stream);
-        if (want32) launch_gemm_pack(true, c->cplx, k, n, rows.ptr + L * lev, f.ptr + L * s32, c->stream);
+        if (want64) launch_gemm_pack(false, c->cplx, ns, k, n, raw.ptr + L * lev, d.ptr + L * s64, c->stream);
+        if (want32) launch_gemm_pack(true, c->cplx, ns, k, n, raw.ptr + L * lev, f.ptr + L * s32, c->stream);
       }
     };
-    std::vector<double> h;
     auto put_pinv = [&](const double* op, const std::vector<int>* rk, const std::vector<int>* rrow, DevBuf<double>& d,
                         DevBuf<float>& f) {
-      transpose_set(op, h);
-      if (rk) compact(h, *rk);
-      put(h, ns, ns, rk, rrow, !c->f32_pinv, c->f32_pinv, pinv_stride(c, false), pinv_stride(c, true), d, f);
+      put(op, 1, ns, ns, rk, rrow, !c->f32_pinv, c->f32_pinv, pinv_stride(c, false), pinv_stride(c, true), d, f);
     };
     put_pinv(uc2e_u, &c->r_up, nullptr, c->uc2e_uT, c->uc2e_uT32);
     put_pinv(uc2e_v, nullptr, &c->r_up, c->uc2e_vT, c->uc2e_vT32);
     put_pinv(dc2e_u, &c->r_dn, nullptr, c->dc2e_uT, c->dc2e_uT32);
     put_pinv(dc2e_v, nullptr, &c->r_dn, c->dc2e_vT, c->dc2e_vT32);
-    // M2Mcat[L]: (8 ns) x ns, row o*ns + k, col n = M2M[L][o][n][k]
-    // L2Lcat[L]: ns x (8 ns), row k, col o*ns + n = L2L[L][o][n][k]
-    std::vector<double> mm(size_t(nlevels) * 8 * ns2 * vw), ll(size_t(nlevels) * 8 * ns2 * vw);
-    for (int L = 0; L < nlevels; L++)
-      for (int o = 0; o < 8; o++)
-        for (int n = 0; n < ns; n++)
-          for (int k = 0; k < ns; k++)
-            for (int w = 0; w < vw; w++) {
-              const size_t s = ((size_t(L) * 8 + o) * ns2 + size_t(n) * ns + k) * vw + w;
-              mm[((size_t(L) * 8 * ns2) + (size_t(o) * ns + k) * ns + n) * vw + w] = m2m[s];
-              ll[((size_t(L) * 8 * ns2) + size_t(k) * 8 * ns + size_t(o) * ns + n) * vw + w] = l2l[s];
-            }
     // (the mixed path keeps both: charges of one sign run M2M / L2L in FP64)
     const bool t64 = !c->f32_trans || c->prec == XFMM_MIXED;
-    put(mm, 8 * ns, ns, nullptr, nullptr, t64, c->f32_trans, m2m_stride(c, false), m2m_stride(c, true), c->m2mcat,
+    put(m2m, 8, 8 * ns, ns, nullptr, nullptr, t64, c->f32_trans, m2m_stride(c, false), m2m_stride(c, true), c->m2mcat,
         c->m2mcat32);
-    put(ll, ns, 8 * ns, nullptr, nullptr, t64, c->f32_trans, l2l_stride(c, false), l2l_stride(c, true), c->l2lcat,
+    put(l2l, 8, ns, 8 * ns, nullptr, nullptr, t64, c->f32_trans, l2l_stride(c, false), l2l_stride(c, true), c->l2lcat,
         c->l2lcat32);
     const size_t msz = size_t(nm2l) * NM2L * c->nfreq * 64 * 2;
     // reference layout uploaded, then expanded on the device into the per-lane

@@ -64,11 +64,13 @@ size_t gemm_packed_size(bool f32, int k, int n) {
   return packed_off((k + KB - 1) / KB, KL, (n + 63) / 64 * 64, 0, 0);
 }
 
-// k, n: sizes of the real form; CPLX: B holds k / 2 x n / 2 complex entries,
-// each the real block [[Re, Im], [-Im, Re]].
+// k, n: sizes of the real form; CPLX: the matrix has k / 2 x n / 2 complex
+// entries, each the real block [[Re, Im], [-Im, Re]].  Entry (r, c) of the
+// matrix is src[r / ns ns + c][r % ns], rows of ns entries: the transpose of
+// one ns x ns matrix, or of 8 of them stacked by rows (M2M) or columns (L2L).
 template <typename CT, bool CPLX>
-__global__ void k_gemm_pack(int k, int n, const double* __restrict__ B, CT* __restrict__ out, size_t total) {
-  constexpr int KB = GemmMfma<CT>::KB, KL = GemmMfma<CT>::KL;
+__global__ void k_gemm_pack(int ns, int k, int n, const double* __restrict__ src, CT* __restrict__ out, size_t total) {
+  constexpr int KB = GemmMfma<CT>::KB, KL = GemmMfma<CT>::KL, V = CPLX ? 2 : 1;
   const int nkb = (k + KB - 1) / KB;
   const size_t stride = size_t(gridDim.x) * blockDim.x;
   for (size_t e = size_t(blockIdx.x) * blockDim.x + threadIdx.x; e < total; e += stride) {
@@ -78,23 +80,21 @@ __global__ void k_gemm_pack(int k, int n, const double* __restrict__ B, CT* __re
     const int cc = int(gk / nkb) * 64 + ct * 16 + (lane & 15);
     double v = 0;
     if (kk < k && cc < n) {
-      if constexpr (CPLX) {
-        const double* z = B + (size_t(kk / 2) * (n / 2) + cc / 2) * 2;
-        v = ((kk ^ cc) & 1) == 0 ? z[0] : (kk & 1) ? -z[1] : z[1];
-      } else {
-        v = B[size_t(kk) * n + cc];
-      }
+      const int r = kk / V;
+      const double* z = src + ((size_t(r / ns) * ns + cc / V) * ns + r % ns) * V;
+      if constexpr (CPLX) v = ((kk ^ cc) & 1) == 0 ? z[0] : (kk & 1) ? -z[1] : z[1];
+      else v = z[0];
     }
     out[e] = CT(v);
   }
 }
 
-void launch_gemm_pack(bool f32, bool cplx, int k, int n, const double* B, void* out, hipStream_t s) {
+void launch_gemm_pack(bool f32, bool cplx, int ns, int k, int n, const double* src, void* out, hipStream_t s) {
   if (cplx) k *= 2, n *= 2;
   const size_t total = gemm_packed_size(f32, k, n);
   if (total == 0) return;
   const dim3 g(unsigned(std::min<size_t>((total + 255) / 256, 65536))), b(256);
-  auto go = [&](auto kern, auto* o) { hipLaunchKernelGGL(kern, g, b, 0, s, k, n, B, o, total); };
+  auto go = [&](auto kern, auto* o) { hipLaunchKernelGGL(kern, g, b, 0, s, ns, k, n, src, o, total); };
   if (f32) cplx ? go(k_gemm_pack<float, true>, static_cast<float*>(out)) : go(k_gemm_pack<float, false>, static_cast<float*>(out));
   else cplx ? go(k_gemm_pack<double, true>, static_cast<double*>(out)) : go(k_gemm_pack<double, false>, static_cast<double*>(out));
 }

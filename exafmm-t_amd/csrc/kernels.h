@@ -103,11 +103,13 @@ struct GemmGroup {
 };
 void launch_gemm_rows(bool f32, const GemmGroup& G, const double* A, const long* arow, const void* B, double* C,
                       const long* crow, int beta, hipStream_t s);
-// Packed MFMA operand form of a row-major k x n matrix B (out: float with
-// f32, else double), gemm_packed_size entries; with cplx B has k x n complex
-// entries and the packed form is that of its 2k x 2n real blocks.
+// Packed MFMA operand form of a k x n matrix (out: float with f32, else
+// double), gemm_packed_size entries, from operators in the layout of
+// xfmm_set_operators: entry (r, c) is src[r / ns ns + c][r % ns], rows of ns
+// entries.  With cplx the entries are complex and the packed form is that of
+// the 2k x 2n real blocks.
 size_t gemm_packed_size(bool f32, int k, int n);
-void launch_gemm_pack(bool f32, bool cplx, int k, int n, const double* B, void* out, hipStream_t s);
+void launch_gemm_pack(bool f32, bool cplx, int ns, int k, int n, const double* src, void* out, hipStream_t s);
 
 // M2L stages.
 struct M2LDev {
