@@ -134,10 +134,10 @@ struct xfmm_context {
   DevBuf<int> level, child0, src_begin, src_count, trg_begin, trg_count;
   DevBuf<int> p2p_off, p2p_src, m2p_off, m2p_src, p2l_off, p2l_src;
   // work lists
-  DevBuf<int> w_p2p, w_m2p, w_p2l, w_l2p_eval, w_leaf;  // w_leaf: P2M/L2P conversion leaves, sorted by level
-  int n_p2p = 0, n_m2p = 0, n_p2l = 0, n_l2p_eval = 0, n_leaf = 0;
-  DevBuf<int> t_p2p, t_l2p;  // (leaf, 64-target tile) pairs of w_p2p / w_l2p_eval
-  int nt_p2p = 0, nt_l2p = 0;
+  DevBuf<int> w_p2p, w_p2l, w_leaf;  // w_leaf: P2M/L2P conversion leaves, sorted by level
+  int n_p2p = 0, n_p2l = 0, n_leaf = 0;
+  DevBuf<int> t_p2p, t_m2p, t_l2p;  // (leaf, 64-target tile) pairs of the leaves with P2P / M2P lists / targets
+  int nt_p2p = 0, nt_m2p = 0, nt_l2p = 0;
   std::vector<int> leaf_level_off;                        // [depth+2] ranges in w_leaf
   DevBuf<long> leaf_slot_rows, leaf_node_rows;            // i*nsurf, node*nsurf
   std::vector<int> nl_level_off;                          // [depth+2] ranges of the non-leaf list
@@ -171,7 +171,7 @@ struct xfmm_context {
   // split-FP16 Hadamard: 128-target groups per workgroup (1 or 2) and 16-target
   // tiles per wave; 0: chosen from the number of targets
   int tune_groups = 0, tune_tiles = 0;
-  int tune_split = 32;     // real-kernel P2P / L2P: largest tail tile whose sources are split over lanes
+  int tune_split = 32;     // P2P / M2P / L2P: largest tail tile whose sources are split over lanes
 
   // ---- timing
   hipEvent_t ev[24] = {};
@@ -438,8 +438,7 @@ void op_L2P(xfmm_context* c, const double* near_add, bool wait_near) {
   DevTree t = c->dev_tree();
   if (wait_near) HIPCHK(hipStreamWaitEvent(c->stream, c->ev[20], 0));
   t.near_add = near_add;
-  launch_eval_targets(c->kind, c->f32_far, MODE_L2P, t, c->wavek(), c->w_l2p_eval.ptr, c->n_l2p_eval, c->t_l2p.ptr,
-                      c->nt_l2p, c->stream);
+  launch_eval_targets(c->kind, c->f32_far, MODE_L2P, t, c->wavek(), c->t_l2p.ptr, c->nt_l2p, c->stream);
 }
 
 void op_P2L(xfmm_context* c) {
@@ -450,7 +449,7 @@ void op_P2L(xfmm_context* c) {
 
 void op_M2P(xfmm_context* c) {
   DevTree t = c->dev_tree();
-  launch_eval_targets(c->kind, c->f32_far, MODE_M2P, t, c->wavek(), c->w_m2p.ptr, c->n_m2p, nullptr, 0, c->stream);
+  launch_eval_targets(c->kind, c->f32_far, MODE_M2P, t, c->wavek(), c->t_m2p.ptr, c->nt_m2p, c->stream);
 }
 
 // The near-coincident pairs of the P2P lists (FP32 near field only), found
@@ -502,8 +501,7 @@ void find_close_pairs(xfmm_context* c) {
 
 void op_P2P(xfmm_context* c) {
   DevTree t = c->dev_tree();
-  launch_eval_targets(c->kind, c->f32_p2p, MODE_P2P, t, c->wavek(), c->w_p2p.ptr, c->n_p2p, c->t_p2p.ptr,
-                      c->nt_p2p, c->stream);
+  launch_eval_targets(c->kind, c->f32_p2p, MODE_P2P, t, c->wavek(), c->t_p2p.ptr, c->nt_p2p, c->stream);
 }
 
 void record(xfmm_context* c, int i) {
@@ -520,8 +518,7 @@ void launch_near(xfmm_context* c) {
   if (!c->capturing) HIPCHK(hipEventRecord(c->ev[21], c->stream2));
   DevTree t = c->dev_tree();
   t.trg_value = c->near.ptr;
-  launch_eval_targets(c->kind, c->f32_p2p, MODE_P2P, t, c->wavek(), c->w_p2p.ptr, c->n_p2p, c->t_p2p.ptr,
-                      c->nt_p2p, c->stream2);
+  launch_eval_targets(c->kind, c->f32_p2p, MODE_P2P, t, c->wavek(), c->t_p2p.ptr, c->nt_p2p, c->stream2);
   if (!c->capturing) HIPCHK(hipEventRecord(c->ev[22], c->stream2));
   HIPCHK(hipEventRecord(c->ev[20], c->stream2));
   c->near_pending = true;
@@ -1010,7 +1007,7 @@ int xfmm_set_tree(xfmm_context* c, const xfmm_tree* t) {
           for (int d = 0; d < 3; d++) rel[3 * size_t(k) + d] = t->src_coord[3 * size_t(k) + d] - t->center[3 * i + d];
       }
       c->src_rel.upload(rel, st);
-      c->src_pack.alloc(std::max<size_t>(1, size_t(t->nsrcs) * 4));
+      c->src_pack.alloc(std::max<size_t>(1, size_t(t->nsrcs) * (c->cplx ? 5 : 4)));
       // L2P equivalent surface per level, relative to the box centre
       const std::vector<double> us = unit_surface(c->p);
       std::vector<double> tab(size_t(D + 1) * c->nsurf * 4, 0.0);
@@ -1064,22 +1061,20 @@ int xfmm_set_tree(xfmm_context* c, const xfmm_tree* t) {
         }
       return v;
     };
-    const std::vector<int> tp2p = tiles(wp2p), tl2p = tiles(wl2p);
+    const std::vector<int> tp2p = tiles(wp2p), tm2p = tiles(wm2p), tl2p = tiles(wl2p);
     c->t_p2p.upload(tp2p, st);
+    c->t_m2p.upload(tm2p, st);
+    c->nt_m2p = int(tm2p.size() / 2);
     c->t_l2p.upload(tl2p, st);
     c->nt_p2p = int(tp2p.size() / 2);
     c->nt_l2p = int(tl2p.size() / 2);
     c->w_p2p.upload(wp2p, st);
-    c->w_m2p.upload(wm2p, st);
     c->w_p2l.upload(wp2l, st);
-    c->w_l2p_eval.upload(wl2p, st);
     c->w_leaf.upload(leaf, st);
     c->leaf_slot_rows.upload(lsr, st);
     c->leaf_node_rows.upload(lnr, st);
     c->n_p2p = int(wp2p.size());
-    c->n_m2p = int(wm2p.size());
     c->n_p2l = int(wp2l.size());
-    c->n_l2p_eval = int(wl2p.size());
     c->n_leaf = int(leaf.size());
     // non-leaves by level (level-major order already)
     std::vector<long> nr, ncr;
@@ -1274,8 +1269,7 @@ int xfmm_downward_pass(xfmm_context* c) {
       DevTree t = c->dev_tree();
       t.trg_value = c->near.ptr;
       launch_zero(c->near.ptr, c->near.n, c->stream);
-      launch_eval_targets(c->kind, c->f32_p2p, MODE_P2P, t, c->wavek(), c->w_p2p.ptr, c->n_p2p, c->t_p2p.ptr,
-                      c->nt_p2p, c->stream);
+      launch_eval_targets(c->kind, c->f32_p2p, MODE_P2P, t, c->wavek(), c->t_p2p.ptr, c->nt_p2p, c->stream);
     }
     record(c, 6);
     op_M2L(c, true);
@@ -1516,10 +1510,8 @@ int xfmm_autotune(xfmm_context* c, int reps, double* best_ms) {
         const double ms = time_it([&] {
           DevTree t = c->dev_tree();
           t.trg_value = c->near.ptr;
-          launch_eval_targets(c->kind, c->f32_p2p, MODE_P2P, t, c->wavek(), c->w_p2p.ptr, c->n_p2p, c->t_p2p.ptr,
-                              c->nt_p2p, c->stream);
-          launch_eval_targets(c->kind, c->f32_far, MODE_L2P, t, c->wavek(), c->w_l2p_eval.ptr, c->n_l2p_eval,
-                              c->t_l2p.ptr, c->nt_l2p, c->stream);
+          launch_eval_targets(c->kind, c->f32_p2p, MODE_P2P, t, c->wavek(), c->t_p2p.ptr, c->nt_p2p, c->stream);
+          launch_eval_targets(c->kind, c->f32_far, MODE_L2P, t, c->wavek(), c->t_l2p.ptr, c->nt_l2p, c->stream);
         });
         if (ms < bt) {
           bt = ms;

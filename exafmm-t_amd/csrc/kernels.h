@@ -32,13 +32,13 @@ struct DevTree {
   const double* src_rel = nullptr;    // [nsrcs][3] source positions relative to their leaf centre
   const double* surf_tab = nullptr;   // [depth + 1][nsurf][4] L2P equivalent surface (radius 2.95 r_l), (x, y, z, 0) relative to the centre
   const float* surf_tab32 = nullptr;  // the same in FP32 (FP32 L2P)
-  void* src_pack = nullptr;           // [nsrcs] (x, y, z, q) relative to the leaf centre, in the P2P type
+  void* src_pack = nullptr;           // [nsrcs] (x, y, z, q[, Im q]) relative to the leaf centre, in the P2P type
   double* up = nullptr;               // T[nnodes][nsurf]
   double* dn = nullptr;               // T[nnodes][nsurf]
   double* trg_value = nullptr;        // T[ntrgs][4]
   const double* near_add = nullptr;   // L2P only (may be null): [ntrgs][4] values that the L2P kernels add to
                                       // each target's result after their own sum (the evaluation's near field)
-  int p2p_split = 32;                 // real-kernel P2P / L2P: tail tiles of <= p2p_split targets (<= 32) split their sources over lanes
+  int p2p_split = 32;                 // P2P / M2P / L2P: tail tiles of <= p2p_split targets (<= 32) split their sources over lanes
   const int* close = nullptr;         // near-coincident P2P pairs, [4] ints (target, source, target leaf, source leaf), sorted by target
   const int* close_off = nullptr;     // [nclose + 1]: pairs of the k-th target with any are close[close_off[k] .. close_off[k + 1])
   const double* close_coef = nullptr; // [pairs][4 or 8]: FP64 minus FP32 value of each pair per unit charge
@@ -61,14 +61,13 @@ void launch_close_find(const DevTree& t, const int* work, int nwork, int* out, i
 void launch_close_coef(int kind, const DevTree& t, Wavek k, int npairs, double* coef, hipStream_t s);
 enum SurfaceMode { MODE_P2M = 0, MODE_P2L = 1 };
 
-// Particle targets of the leaves in work[0..nwork): P2P (sources: leaf
-// particles of the P2P list), M2P (sources: upward equivalent surfaces of the
-// M2P list, alpha 1.05), L2P (source: the leaf's own downward equivalent
-// surface, alpha 2.95).  Adds grad/potential into trg_value.  tiles[2 i],
-// tiles[2 i + 1] (i < ntiles) = (leaf, tile of 64 targets) of the same
-// leaves: the P2P and L2P kernels of the real kernels take one tile per wave.
-void launch_eval_targets(int kind, bool f32, int mode, const DevTree& t, Wavek k, const int* work, int nwork,
-                         const int* tiles, int ntiles, hipStream_t s);
+// Particle targets: P2P (sources: leaf particles of the P2P list), M2P (sources:
+// upward equivalent surfaces of the M2P list, alpha 1.05), L2P (source: the
+// leaf's own downward equivalent surface, alpha 2.95).  Adds grad/potential
+// into trg_value.  tiles[2 i], tiles[2 i + 1] (i < ntiles) = (leaf, tile of 64
+// targets).
+void launch_eval_targets(int kind, bool f32, int mode, const DevTree& t, Wavek k, const int* tiles, int ntiles,
+                         hipStream_t s);
 
 // Surface targets: P2M writes the upward check potential of each work leaf to
 // check[slot] (slot = position in work); P2L adds the potential of the P2L list

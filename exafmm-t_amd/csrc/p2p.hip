@@ -9,13 +9,16 @@
 //   Helmholtz helmholtz.h:186-207:          phi += q e^{ikr}/r,    grad += (1/r^2 - ik/r) phi_ij d
 // Pairs with r = 0 contribute nothing (laplace.h:57, `invr &= r2 > zero`).
 //
-// Layout: one wave (64 lanes) per target leaf / node; lane = one target (in
-// chunks of 64); sources are staged through LDS in tiles of 64 and read as
-// wave-uniform broadcasts.  Coordinates are made relative to the target leaf
+// Layout: particle targets in tiles of 64 per leaf, a target per lane, sources
+// read as wave-uniform vectors; surface targets with a wave per node, sources
+// staged through LDS in tiles of 64.  Coordinates are made relative to a leaf
 // centre in FP64 before any FP32 conversion, so the mixed path keeps
-// |d| accuracy at the scale of the leaf.  In the FP32 path each tile is
-// summed in plain FP32 and tiles are combined with compensated (Kahan)
-// summation.
+// |d| accuracy at the scale of the leaf.  In the FP32 path each tile of 64
+// sources is summed in plain FP32 and tiles are combined with compensated
+// (Kahan) summation.
+#include <algorithm>
+#include <type_traits>
+
 #include "kernels.h"
 
 namespace xfmm {
@@ -160,340 +163,314 @@ __device__ __forceinline__ R close_rmin2(const DevTree& t, int leaf) {
   return R(0);
 }
 
-// ------------------------------------------------------------------ P2P
+// ---------------------------------------------- particle targets: P2P, M2P, L2P
 //
-// Near field of the real kernels with the sources read as wave-uniform
-// 16/32-byte vectors (scalar loads, no LDS and no barriers): each source is
-// packed once per evaluation as (x, y, z, q) relative to its leaf centre; a
-// target is moved into the frame of the source leaf with one subtraction per
-// source leaf (the offset of the two centres is formed in FP64).  Pairs are
-// summed per source leaf in chunks of 64 (plain sums, FP32 chunks combined
-// with Kahan summation, as in the tiled kernel).
+// One workgroup of W waves per (leaf, tile of TILE targets), work[2 b] = leaf,
+// work[2 b + 1] = tile.  A full tile has a target per lane and reads its
+// sources as wave-uniform vectors (scalar loads from constant address space,
+// no LDS and no barriers); a tail tile of nt <= t.p2p_split (<= TILE / 2)
+// targets gives each target TILE / nt lanes (target lane % nt, phase lane /
+// nt) that take every (TILE / nt)-th source.  The W waves share the sources;
+// the partial sums of a target are added in FP64 through LDS in a fixed order.
+// Pairs are summed in chunks of 64 sources (plain sums, FP32 chunks combined
+// with Kahan summation).
+// W (particle_waves): a wave per tile leaves a small tree's chip idle and its
+// longest tile is the time.  Near field, a wave per tile and W waves: Laplace
+// FP64, 64 leaves of 47 targets 119 and 29 us (16); Yukawa FP64, 1300
+// leaves of 15 193 and 73 (4); Helmholtz FP64, 512 leaves of 59 881 (a wave per
+// leaf) and 276 (4).
+template <int KIND>
+constexpr int nval() { return kcplx<KIND>() ? 8 : 4; }  // values per target
+
+// The tile of this workgroup and the target of this lane.
 template <typename R>
-struct P4;
-template <>
-struct P4<float> {
-  typedef float4 t;
-};
-template <>
-struct P4<double> {
-  typedef double4 t;
-};
-
-template <typename R>
-__global__ void k_pack_sources(int n, const double* __restrict__ rel, const double* __restrict__ q,
-                               typename P4<R>::t* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  typename P4<R>::t v;
-  v.x = R(rel[3 * size_t(i)]);
-  v.y = R(rel[3 * size_t(i) + 1]);
-  v.z = R(rel[3 * size_t(i) + 2]);
-  v.w = R(q[i]);
-  out[i] = v;
-}
-
-// Tail of a leaf with nt <= t.p2p_split (<= TILE / 2) targets: k = TILE / nt lanes per target,
-// lane (target lane % nt, phase lane / nt) takes every k-th source from its
-// phase on (vector loads); the k partial sums of a target are added in FP64
-// through LDS by split_reduce.
-// add (may be null): NA values per target added after the sum (the
-// near field that an L2P adds to its result, see DevTree::near_add).
-template <typename R, int NA>
-__device__ __forceinline__ void split_reduce(const R* acc, const R* comp, int nt, int k, double* out,
-                                             const double* add = nullptr) {
-  __shared__ double red[TILE][NA];
-  const int lane = threadIdx.x;
-#pragma unroll
-  for (int a = 0; a < NA; a++) red[lane][a] = double(acc[a]) - double(comp[a]);
-  __syncthreads();
-  if (lane < nt) {
-#pragma unroll
-    for (int a = 0; a < NA; a++) {
-      double v = 0;
-      for (int ph = 0; ph < k; ph++) v += red[lane + ph * nt][a];
-      if (add) out[a] = (out[a] + v * FOUR_PI_INV) + add[a];
-      else out[a] += v * FOUR_PI_INV;
-    }
-  }
-}
-
-// Near field of the real kernels (fmm_base.h:82-94): one wave per (leaf,
-// tile of TILE targets), work[2 b] = leaf, work[2 b + 1] = tile.  A full tile
-// has a target per lane and reads the packed sources (relative to their leaf
-// centre) with scalar loads (constant address space); a tail tile of at most
-// t.p2p_split (<= TILE / 2) targets splits the sources of each target over
-// several lanes.
-template <int KIND, typename R>
-__global__ __launch_bounds__(64) void k_p2p_smem(DevTree t, Wavek wk, const int* __restrict__ work) {
-  constexpr int NA = 4;
-  // constant address space: the packed sources are read-only for the whole
-  // launch, and wave-uniform loads from it become scalar loads
-  typedef const R __attribute__((address_space(4))) * CR;
-  typedef typename P4<R>::t V;
-  const CR src = (CR)(t.src_pack);
-  const V* srcv = static_cast<const V*>(t.src_pack);
-  const int leaf = work[2 * blockIdx.x], t0 = TILE * work[2 * blockIdx.x + 1];
-  const int lane = threadIdx.x;
-  const double cx = t.center[3 * leaf], cy = t.center[3 * leaf + 1], cz = t.center[3 * leaf + 2];
-  const int tb = t.trg_begin[leaf], nt = min(TILE, t.trg_count[leaf] - t0);
-  const R kr = R(wk.re), ki = R(wk.im);
-  const int g0 = t.p2p_off[leaf], g1 = t.p2p_off[leaf + 1];
-  const bool split = nt <= t.p2p_split;
-  const int k = split ? TILE / nt : 1;
-  const int ti = split ? lane % nt : lane, ph = split ? lane / nt : 0;
-  const bool act = split ? ph < k : ti < nt;
-  const R rmin2 = close_rmin2<R>(t, leaf);
-  R tx = 0, ty = 0, tz = 0;
-  if (ti < nt) {
-    const double* x = t.trg + 3 * size_t(tb + t0 + ti);
-    tx = R(x[0] - cx);
-    ty = R(x[1] - cy);
-    tz = R(x[2] - cz);
-  }
-  R acc[NA], comp[NA];
-#pragma unroll
-  for (int a = 0; a < NA; a++) { acc[a] = 0; comp[a] = 0; }
-  for (int g = g0; g < g1; g++) {
-    const int snode = t.p2p_src[g];
-    const int sb = t.src_begin[snode], ns = t.src_count[snode];
-    // target in the frame of the source leaf
-    const R ux = tx - R(t.center[3 * snode] - cx);
-    const R uy = ty - R(t.center[3 * snode + 1] - cy);
-    const R uz = tz - R(t.center[3 * snode + 2] - cz);
-    const bool self = snode == leaf;
-    if (split) {
-      R part[NA] = {0, 0, 0, 0};
-      if (act) {
-        if (self)
-          for (int j = ph; j < ns; j += k) {
-            const V v = srcv[sb + j];
-            pair_grad<KIND, R, RSQ_MASK>(v.x - ux, v.y - uy, v.z - uz, v.w, R(0), kr, ki, part, rmin2);
-          }
-        else
-          for (int j = ph; j < ns; j += k) {
-            const V v = srcv[sb + j];
-            pair_grad<KIND, R, RSQ_SEP>(v.x - ux, v.y - uy, v.z - uz, v.w, R(0), kr, ki, part);
-          }
-      }
-      fold_tile<R, NA>(acc, comp, part);
-      continue;
-    }
-    for (int s0 = 0; s0 < ns; s0 += TILE) {
-      const int m = min(TILE, ns - s0);
-      const CR S = src + 4 * size_t(sb + s0);
-      R part[NA] = {0, 0, 0, 0};
-      int j = 0;
-      if (self) {
-        for (; j + 4 <= m; j += 4) {
-#pragma unroll
-          for (int u = 0; u < 4; u++) {
-            const CR v = S + 4 * (j + u);
-            pair_grad<KIND, R, RSQ_MASK>(v[0] - ux, v[1] - uy, v[2] - uz, v[3], R(0), kr, ki, part, rmin2);
-          }
-        }
-        for (; j < m; j++) {
-          const CR v = S + 4 * j;
-          pair_grad<KIND, R, RSQ_MASK>(v[0] - ux, v[1] - uy, v[2] - uz, v[3], R(0), kr, ki, part, rmin2);
-        }
-      } else {
-        for (; j + 4 <= m; j += 4) {
-#pragma unroll
-          for (int u = 0; u < 4; u++) {
-            const CR v = S + 4 * (j + u);
-            pair_grad<KIND, R, RSQ_SEP>(v[0] - ux, v[1] - uy, v[2] - uz, v[3], R(0), kr, ki, part);
-          }
-        }
-        for (; j < m; j++) {
-          const CR v = S + 4 * j;
-          pair_grad<KIND, R, RSQ_SEP>(v[0] - ux, v[1] - uy, v[2] - uz, v[3], R(0), kr, ki, part);
-        }
-      }
-      fold_tile<R, NA>(acc, comp, part);
-    }
-  }
-  double* o = t.trg_value + size_t(tb + t0) * 4;
-  if (split) {
-    split_reduce<R, NA>(acc, comp, nt, k, o + 4 * size_t(lane < nt ? lane : 0));
-  } else if (act) {
-#pragma unroll
-    for (int a = 0; a < NA; a++) o[4 * lane + a] += (double(acc[a]) - double(comp[a])) * FOUR_PI_INV;
-  }
-}
-
-// L2P of the real kernels (fmm_scale_invariant.h:198-230, fmm.h:188-218):
-// one wave per (leaf, tile of TILE targets), work as for k_p2p_smem.  The
-// sources, the leaf's equivalent surface points (per-level table, relative
-// to the centre) and its local equivalent densities, are the same for every
-// lane of a full tile and are read with scalar loads, four per unrolled
-// step; a tail tile of at most TILE / 2 targets splits them over lanes.
-template <int KIND, typename R>
-__global__ __launch_bounds__(64) void k_l2p_smem(DevTree t, Wavek wk, const int* __restrict__ work) {
-  constexpr int NA = 4;
-  typedef const double __attribute__((address_space(4))) * CD;
-  // surface points in the arithmetic type (no per-source conversions)
-  typedef const R __attribute__((address_space(4))) * CRT;
-  const int leaf = work[2 * blockIdx.x], t0 = TILE * work[2 * blockIdx.x + 1];
-  const int lane = threadIdx.x;
-  const double cx = t.center[3 * leaf], cy = t.center[3 * leaf + 1], cz = t.center[3 * leaf + 2];
-  const int tb = t.trg_begin[leaf], nt = min(TILE, t.trg_count[leaf] - t0), ns = t.nsurf;
-  const R kr = R(wk.re), ki = R(wk.im);
-  const size_t tab0 = size_t(t.level[leaf]) * ns;
-  const R* tabr;
-  if constexpr (sizeof(R) == 4) tabr = reinterpret_cast<const R*>(t.surf_tab32);
-  else tabr = reinterpret_cast<const R*>(t.surf_tab);
-  const CRT sp = (CRT)(tabr) + tab0 * 4;
-  const CD eq = (CD)(t.dn) + size_t(leaf) * ns;
-  const bool split = nt <= t.p2p_split;
-  const int k = split ? TILE / nt : 1;
-  const int ti = split ? lane % nt : lane, ph = split ? lane / nt : 0;
-  const bool act = split ? ph < k : ti < nt;
-  R tx = 0, ty = 0, tz = 0;
-  if (ti < nt) {
-    const double* x = t.trg + 3 * size_t(tb + t0 + ti);
-    tx = R(x[0] - cx);
-    ty = R(x[1] - cy);
-    tz = R(x[2] - cz);
-  }
-  R acc[NA], comp[NA];
-#pragma unroll
-  for (int a = 0; a < NA; a++) { acc[a] = 0; comp[a] = 0; }
-  double* o = t.trg_value + size_t(tb + t0) * 4;
-  if (split) {
-    const double4* tab = reinterpret_cast<const double4*>(t.surf_tab) + tab0;
-    const double* eqv = t.dn + size_t(leaf) * ns;
-    for (int s0 = 0; s0 < ns; s0 += TILE * k) {
-      R part[NA] = {0, 0, 0, 0};
-      const int e = min(ns, s0 + TILE * k);
-      if (act)
-        for (int j = s0 + ph; j < e; j += k) {
-          const double4 v = tab[j];
-          pair_grad<KIND, R, RSQ_SEP>(R(v.x) - tx, R(v.y) - ty, R(v.z) - tz, R(eqv[j]), R(0), kr, ki, part);
-        }
-      fold_tile<R, NA>(acc, comp, part);
-    }
-    const size_t ol = 4 * size_t(lane < nt ? lane : 0);
-    split_reduce<R, NA>(acc, comp, nt, k, o + ol, t.near_add ? t.near_add + size_t(tb + t0) * 4 + ol : nullptr);
-    return;
-  }
-  for (int s0 = 0; s0 < ns; s0 += TILE) {
-    const int m = min(TILE, ns - s0);
-    R part[NA] = {0, 0, 0, 0};
-    int j = 0;
-    for (; j + 4 <= m; j += 4) {
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const CRT v = sp + 4 * (s0 + j + u);
-        pair_grad<KIND, R, RSQ_SEP>(v[0] - tx, v[1] - ty, v[2] - tz, R(eq[s0 + j + u]), R(0), kr, ki, part);
-      }
-    }
-    for (; j < m; j++) {
-      const CRT v = sp + 4 * (s0 + j);
-      pair_grad<KIND, R, RSQ_SEP>(v[0] - tx, v[1] - ty, v[2] - tz, R(eq[s0 + j]), R(0), kr, ki, part);
-    }
-    fold_tile<R, NA>(acc, comp, part);
-  }
-  if (act) {
-    const double* add = t.near_add ? t.near_add + size_t(tb + t0) * 4 + 4 * lane : nullptr;
-#pragma unroll
-    for (int a = 0; a < NA; a++) {
-      const double v = (double(acc[a]) - double(comp[a])) * FOUR_PI_INV;
-      if (add) o[4 * lane + a] = (o[4 * lane + a] + v) + add[a];
-      else o[4 * lane + a] += v;
-    }
-  }
-}
-
-template <int KIND, typename R, int MODE>
-__global__ __launch_bounds__(64) void k_eval_targets(DevTree t, Wavek wk, const int* __restrict__ work) {
-  constexpr bool C = kcplx<KIND>();
-  constexpr int NA = C ? 8 : 4;
-  __shared__ R sx[TILE], sy[TILE], sz[TILE], sq[TILE], sqi[TILE];
-  const int leaf = work[blockIdx.x];
-  const int lane = threadIdx.x;
-  const double cx = t.center[3 * leaf], cy = t.center[3 * leaf + 1], cz = t.center[3 * leaf + 2];
-  const int tb = t.trg_begin[leaf], nt = t.trg_count[leaf];
-  const R kr = R(wk.re), ki = R(wk.im);
-  const int vw = t.vw;
-  int g0 = 0, g1 = 1;
-  if (MODE == MODE_P2P) { g0 = t.p2p_off[leaf]; g1 = t.p2p_off[leaf + 1]; }
-  if (MODE == MODE_M2P) { g0 = t.m2p_off[leaf]; g1 = t.m2p_off[leaf + 1]; }
-  for (int t0 = 0; t0 < nt; t0 += TILE) {
-    const int ti = t0 + lane;
-    const bool act = ti < nt;
-    R tx = 0, ty = 0, tz = 0;
-    if (act) {
+struct Tile {
+  int leaf, tb, nt, k, ti, ph, wave;
+  bool split, act;
+  double cx, cy, cz;
+  R tx, ty, tz;  // target relative to its leaf centre
+  __device__ __forceinline__ Tile(const DevTree& t, const int* work) {
+    leaf = work[2 * blockIdx.x];
+    const int t0 = TILE * work[2 * blockIdx.x + 1];
+    const int lane = threadIdx.x & 63;
+    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    cx = t.center[3 * leaf];
+    cy = t.center[3 * leaf + 1];
+    cz = t.center[3 * leaf + 2];
+    tb = t.trg_begin[leaf] + t0;
+    nt = min(TILE, t.trg_count[leaf] - t0);
+    split = nt <= t.p2p_split;
+    k = split ? TILE / nt : 1;
+    ti = split ? lane % nt : lane;
+    ph = split ? lane / nt : 0;
+    act = split ? ph < k : ti < nt;
+    tx = ty = tz = 0;
+    if (ti < nt) {
       const double* x = t.trg + 3 * size_t(tb + ti);
       tx = R(x[0] - cx);
       ty = R(x[1] - cy);
       tz = R(x[2] - cz);
     }
-    R acc[NA], comp[NA];
+  }
+};
+
+// trg_value (+ near_add) of the tile's targets += the sums of its lanes and
+// waves / 4 pi.
+template <int NA, int W, typename R>
+__device__ __forceinline__ void put_tile(const DevTree& t, const Tile<R>& T, const R* acc, const R* comp,
+                                         const double* near_add) {
+  auto add = [&](int i, const double* v) {
+    double* o = t.trg_value + size_t(T.tb + i) * NA;
+    const double* n = near_add ? near_add + size_t(T.tb + i) * NA : nullptr;
 #pragma unroll
-    for (int a = 0; a < NA; a++) { acc[a] = 0; comp[a] = 0; }
-    for (int g = g0; g < g1; g++) {
-      int snode, ns, sb = 0;
-      double b = 0, ox = 0, oy = 0, oz = 0;
-      const double* eq = nullptr;
-      if (MODE == MODE_P2P) {
-        snode = t.p2p_src[g];
-        sb = t.src_begin[snode];
-        ns = t.src_count[snode];
-      } else {
-        snode = (MODE == MODE_M2P) ? t.m2p_src[g] : leaf;
-        ns = t.nsurf;
-        b = ((MODE == MODE_M2P) ? 1.05 : 2.95) * t.r0 * ldexp(1.0, -t.level[snode]);
-        ox = t.center[3 * snode] - cx;
-        oy = t.center[3 * snode + 1] - cy;
-        oz = t.center[3 * snode + 2] - cz;
-        eq = ((MODE == MODE_M2P) ? t.up : t.dn) + size_t(snode) * t.nsurf * vw;
-      }
-      for (int s0 = 0; s0 < ns; s0 += TILE) {
-        const int m = min(TILE, ns - s0);
-        __syncthreads();
-        if (lane < m) {
-          const int si = s0 + lane;
-          if (MODE == MODE_P2P) {
-            const double* x = t.src + 3 * size_t(sb + si);
-            sx[lane] = R(x[0] - cx);
-            sy[lane] = R(x[1] - cy);
-            sz[lane] = R(x[2] - cz);
-            const double* qq = t.q + size_t(sb + si) * vw;
-            sq[lane] = R(qq[0]);
-            if (C) sqi[lane] = R(qq[1]);
-          } else {
-            sx[lane] = R(ox + t.unit_surf[3 * si] * b);
-            sy[lane] = R(oy + t.unit_surf[3 * si + 1] * b);
-            sz[lane] = R(oz + t.unit_surf[3 * si + 2] * b);
-            sq[lane] = R(eq[size_t(si) * vw]);
-            if (C) sqi[lane] = R(eq[size_t(si) * vw + 1]);
-          }
-        }
-        __syncthreads();
-        R part[NA];
+    for (int a = 0; a < NA; a++) o[a] = n ? (o[a] + v[a] * FOUR_PI_INV) + n[a] : o[a] + v[a] * FOUR_PI_INV;
+  };
+  if (W == 1 && !T.split) {
+    if (T.act) {
+      double v[NA];
 #pragma unroll
-        for (int a = 0; a < NA; a++) part[a] = 0;
-        // only a leaf with itself can pair coinciding points; equivalent
-        // surfaces never touch the targets
-        if (MODE == MODE_P2P && snode == leaf)
-          tile_sum<KIND, R, RSQ_MASK, true>(m, sx, sy, sz, sq, sqi, tx, ty, tz, kr, ki, part,
-                                            close_rmin2<R>(t, leaf));
-        else
-          tile_sum<KIND, R, RSQ_SEP, true>(m, sx, sy, sz, sq, sqi, tx, ty, tz, kr, ki, part);
-        fold_tile<R, NA>(acc, comp, part);
-      }
+      for (int a = 0; a < NA; a++) v[a] = double(acc[a]) - double(comp[a]);
+      add(T.ti, v);
     }
-    if (act) {
-      double* o = t.trg_value + size_t(tb + ti) * 4 * vw;
-      const double* add = (MODE == MODE_L2P && t.near_add) ? t.near_add + size_t(tb + ti) * 4 * vw : nullptr;
+    return;
+  }
+  __shared__ double red[W][NA][TILE];
+  const int lane = threadIdx.x & 63;
 #pragma unroll
-      for (int a = 0; a < NA; a++) {
-        const double v = (double(acc[a]) - double(comp[a])) * FOUR_PI_INV;
-        if (add) o[a] = (o[a] + v) + add[a];
-        else o[a] += v;
-      }
+  for (int a = 0; a < NA; a++) red[T.wave][a][lane] = double(acc[a]) - double(comp[a]);
+  __syncthreads();
+  if (int(threadIdx.x) < T.nt) {
+    double v[NA];
+#pragma unroll
+    for (int a = 0; a < NA; a++) {
+      v[a] = 0;
+      for (int w = 0; w < W; w++)
+        for (int ph = 0; ph < T.k; ph++) v[a] += red[w][a][threadIdx.x + ph * T.nt];
+    }
+    add(threadIdx.x, v);
+  }
+}
+
+// Readers of a list of sources: get(u, v) puts x, y, z, q (and Im q, else 0) of
+// source u from the current one on into v, skip(n) moves on by n sources.
+// P, E: pointers to positions (stride PS) and densities (stride ES); with ES = 0
+// the densities follow the position.
+template <typename R, int NQ, int PS, int ES, typename P, typename E>
+struct Sources {
+  P p;
+  E e;
+  __device__ __forceinline__ Sources(P p_, E e_) : p(p_), e(e_) {}
+  __device__ __forceinline__ void skip(int n) {
+    p += size_t(PS) * n;
+    if constexpr (ES > 0) e += size_t(ES) * n;
+  }
+  __device__ __forceinline__ void get(int u, R* v) const {
+#pragma unroll
+    for (int d = 0; d < 3; d++) v[d] = p[PS * u + d];
+#pragma unroll
+    for (int d = 0; d < 2; d++) {
+      if constexpr (ES > 0) v[3 + d] = d < NQ ? R(e[ES * u + (d < NQ ? d : 0)]) : R(0);
+      else v[3 + d] = d < NQ ? p[PS * u + (d < NQ ? 3 + d : 0)] : R(0);
     }
   }
+};
+
+// Sum of n sources of a full tile in chunks of TILE, four pairs per loop trip.
+template <int KIND, typename R, int RM, typename SRC>
+__device__ __forceinline__ void sum_uniform(int n, SRC src, R ux, R uy, R uz, R kr, R ki, R* acc, R* comp, R rmin2) {
+  constexpr int NA = nval<KIND>();
+  for (int s0 = 0; s0 < n; s0 += TILE) {
+    const int m = min(TILE, n - s0);
+    R part[NA] = {0};
+    int j = 0;
+    for (; j + 4 <= m; j += 4) {
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        R v[5];
+        src.get(u, v);
+        pair_grad<KIND, R, RM>(v[0] - ux, v[1] - uy, v[2] - uz, v[3], v[4], kr, ki, part, rmin2);
+      }
+      src.skip(4);
+    }
+    for (; j < m; j++) {
+      R v[5];
+      src.get(0, v);
+      pair_grad<KIND, R, RM>(v[0] - ux, v[1] - uy, v[2] - uz, v[3], v[4], kr, ki, part, rmin2);
+      src.skip(1);
+    }
+    fold_tile<R, NA>(acc, comp, part);
+  }
+}
+// The same for a split tile: this lane's sources ph, ph + k, ..., in chunks of
+// TILE per lane; the loads of four pairs are issued together (one at a time
+// their latency is the time).
+template <int KIND, typename R, int RM, typename SRC>
+__device__ __forceinline__ void sum_split(int n, const Tile<R>& T, SRC src, R ux, R uy, R uz, R kr, R ki, R* acc,
+                                          R* comp, R rmin2) {
+  constexpr int NA = nval<KIND>();
+  src.skip(T.ph);
+  for (int s0 = 0; s0 < n; s0 += TILE * T.k) {
+    const int e = min(n, s0 + TILE * T.k);
+    R part[NA] = {0};
+    if (T.act) {
+      int j = s0 + T.ph;
+      for (; j + 3 * T.k < e; j += 4 * T.k) {
+        R v[4][5];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          src.get(0, v[u]);
+          src.skip(T.k);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          pair_grad<KIND, R, RM>(v[u][0] - ux, v[u][1] - uy, v[u][2] - uz, v[u][3], v[u][4], kr, ki, part, rmin2);
+      }
+      for (; j < e; j += T.k) {
+        R v[5];
+        src.get(0, v);
+        src.skip(T.k);
+        pair_grad<KIND, R, RM>(v[0] - ux, v[1] - uy, v[2] - uz, v[3], v[4], kr, ki, part, rmin2);
+      }
+    }
+    fold_tile<R, NA>(acc, comp, part);
+  }
+}
+
+// Near field (fmm_base.h:82-94).  Each source is packed once per evaluation as
+// (x, y, z, q[, Im q]) relative to its leaf centre; a target is moved into the
+// frame of the source leaf with one subtraction per source leaf (the offset
+// of the two centres is formed in FP64).
+template <int KIND>
+constexpr int npack() { return kcplx<KIND>() ? 5 : 4; }
+
+template <typename R, int NP>
+__global__ void k_pack_sources(int n, const double* __restrict__ rel, const double* __restrict__ q,
+                               R* __restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  R v[NP];
+#pragma unroll
+  for (int d = 0; d < 3; d++) v[d] = R(rel[3 * size_t(i) + d]);
+#pragma unroll
+  for (int d = 3; d < NP; d++) v[d] = R(q[size_t(i) * (NP - 3) + d - 3]);
+#pragma unroll
+  for (int d = 0; d < NP; d++) out[size_t(i) * NP + d] = v[d];
+}
+
+template <int KIND, typename R, int W>
+__global__ __launch_bounds__(64 * W) void k_p2p_smem(DevTree t, Wavek wk, const int* __restrict__ work) {
+  constexpr int NA = nval<KIND>(), NP = npack<KIND>();
+  // constant address space: the packed sources are read-only for the whole
+  // launch, and wave-uniform loads from it become scalar loads
+  typedef const R __attribute__((address_space(4))) * CR;
+  const R* pack = static_cast<const R*>(t.src_pack);
+  const Tile<R> T(t, work);
+  const R kr = R(wk.re), ki = R(wk.im);
+  const R rmin2 = close_rmin2<R>(t, T.leaf);
+  R acc[NA], comp[NA];
+#pragma unroll
+  for (int a = 0; a < NA; a++) { acc[a] = 0; comp[a] = 0; }
+  for (int g = t.p2p_off[T.leaf] + T.wave; g < t.p2p_off[T.leaf + 1]; g += W) {
+    const int snode = t.p2p_src[g];
+    const int sb = t.src_begin[snode], ns = t.src_count[snode];
+    // target in the frame of the source leaf
+    const R ux = T.tx - R(t.center[3 * snode] - T.cx);
+    const R uy = T.ty - R(t.center[3 * snode + 1] - T.cy);
+    const R uz = T.tz - R(t.center[3 * snode + 2] - T.cz);
+    const R* S = pack + size_t(NP) * sb;
+    const Sources<R, NP - 3, NP, 0, const R*, int> vec(S, 0);
+    const Sources<R, NP - 3, NP, 0, CR, int> uni((CR)(S), 0);
+    // only a leaf with itself can pair coinciding points
+    if (snode == T.leaf) {
+      if (T.split) sum_split<KIND, R, RSQ_MASK>(ns, T, vec, ux, uy, uz, kr, ki, acc, comp, rmin2);
+      else sum_uniform<KIND, R, RSQ_MASK>(ns, uni, ux, uy, uz, kr, ki, acc, comp, rmin2);
+    } else {
+      if (T.split) sum_split<KIND, R, RSQ_SEP>(ns, T, vec, ux, uy, uz, kr, ki, acc, comp, R(0));
+      else sum_uniform<KIND, R, RSQ_SEP>(ns, uni, ux, uy, uz, kr, ki, acc, comp, R(0));
+    }
+  }
+  put_tile<NA, W>(t, T, acc, comp, nullptr);
+}
+
+// L2P (fmm_scale_invariant.h:198-230, fmm.h:188-218).  The sources are the points
+// of the leaf's own downward equivalent surface (alpha 2.95), from a per-level
+// table relative to the box centre, with the leaf's densities: the same for
+// every lane of a full tile.  The W waves share the points.
+template <int KIND, typename R, int W>
+__global__ __launch_bounds__(64 * W) void k_l2p_smem(DevTree t, Wavek wk, const int* __restrict__ work) {
+  constexpr int NA = nval<KIND>();
+  constexpr bool C = kcplx<KIND>();
+  typedef const double __attribute__((address_space(4))) * CD;
+  // surface points in the arithmetic type (no per-source conversions)
+  typedef const R __attribute__((address_space(4))) * CR;
+  const Tile<R> T(t, work);
+  const R kr = R(wk.re), ki = R(wk.im);
+  const int ns = t.nsurf;
+  const R* tab;
+  if constexpr (sizeof(R) == 4) tab = t.surf_tab32;
+  else tab = t.surf_tab;
+  tab += size_t(t.level[T.leaf]) * ns * 4;
+  const double* eq = t.dn + size_t(T.leaf) * ns * (C ? 2 : 1);
+  R acc[NA], comp[NA];
+#pragma unroll
+  for (int a = 0; a < NA; a++) { acc[a] = 0; comp[a] = 0; }
+  const int per = ((ns + W - 1) / W + 3) / 4 * 4, j0 = min(ns, T.wave * per), n = min(ns, j0 + per) - j0;
+  constexpr int NQ = C ? 2 : 1;
+  const R* p0 = tab + 4 * size_t(j0);
+  const double* e0 = eq + NQ * size_t(j0);
+  const Sources<R, NQ, 4, NQ, const R*, const double*> vec(p0, e0);
+  const Sources<R, NQ, 4, NQ, CR, CD> uni((CR)(p0), (CD)(e0));
+  // the surface never touches the targets
+  if (T.split) sum_split<KIND, R, RSQ_SEP>(n, T, vec, T.tx, T.ty, T.tz, kr, ki, acc, comp, R(0));
+  else sum_uniform<KIND, R, RSQ_SEP>(n, uni, T.tx, T.ty, T.tz, kr, ki, acc, comp, R(0));
+  put_tile<NA, W>(t, T, acc, comp, t.near_add);
+}
+
+// M2P (fmm_base.h:97-124): the sources are the upward equivalent surfaces (alpha
+// 1.05) of the nodes of the M2P list.  Few leaves have such lists and their
+// nodes lie all over memory, so what counts is latency: the W waves stage a
+// node's points (relative to the target leaf's centre, formed in FP64) and
+// densities in LDS at once and share them.  16 Plummer problems (2007 leaves
+// with 1..16 nodes, 74 M pairs): a wave per leaf, 64 points staged at a time
+// 225 us; four waves 88.
+template <int KIND, typename R, int W>
+__global__ __launch_bounds__(64 * W) void k_m2p(DevTree t, Wavek wk, const int* __restrict__ work) {
+  constexpr int NA = nval<KIND>();
+  constexpr bool C = kcplx<KIND>();
+  constexpr int NP = npack<KIND>(), NB = 256;  // points per LDS block
+  __shared__ R sp[NB * NP];
+  const Tile<R> T(t, work);
+  const R kr = R(wk.re), ki = R(wk.im);
+  const int ns = t.nsurf;
+  R acc[NA], comp[NA];
+#pragma unroll
+  for (int a = 0; a < NA; a++) { acc[a] = 0; comp[a] = 0; }
+  for (int g = t.m2p_off[T.leaf]; g < t.m2p_off[T.leaf + 1]; g++) {
+    const int snode = t.m2p_src[g];
+    const double b = 1.05 * t.r0 * ldexp(1.0, -t.level[snode]);
+    const double ox = t.center[3 * snode] - T.cx, oy = t.center[3 * snode + 1] - T.cy,
+                 oz = t.center[3 * snode + 2] - T.cz;
+    const double* eq = t.up + size_t(snode) * ns * (C ? 2 : 1);
+    for (int s0 = 0; s0 < ns; s0 += NB) {
+      const int m = min(NB, ns - s0);
+      __syncthreads();
+      for (int i = threadIdx.x; i < m; i += 64 * W) {
+        const int si = s0 + i;
+        R* p = sp + NP * i;
+        p[0] = R(ox + t.unit_surf[3 * si] * b);
+        p[1] = R(oy + t.unit_surf[3 * si + 1] * b);
+        p[2] = R(oz + t.unit_surf[3 * si + 2] * b);
+        p[3] = R(eq[C ? 2 * si : si]);
+        if (C) p[NP - 1] = R(eq[2 * si + 1]);
+      }
+      __syncthreads();
+      const int per = ((m + W - 1) / W + 3) / 4 * 4, j0 = min(m, T.wave * per), n = min(m, j0 + per) - j0;
+      const Sources<R, NP - 3, NP, 0, const R*, int> src(sp + NP * j0, 0);
+      if (T.split) sum_split<KIND, R, RSQ_SEP>(n, T, src, T.tx, T.ty, T.tz, kr, ki, acc, comp, R(0));
+      else sum_uniform<KIND, R, RSQ_SEP>(n, src, T.tx, T.ty, T.tz, kr, ki, acc, comp, R(0));
+    }
+  }
+  put_tile<NA, W>(t, T, acc, comp, nullptr);
 }
 
 template <int KIND, typename R, int MODE>
@@ -510,7 +487,7 @@ __global__ __launch_bounds__(64) void k_eval_surface(DevTree t, Wavek wk, const 
   const int vw = t.vw;
   int g0 = 0, g1 = 1;
   if (MODE == MODE_P2L) { g0 = t.p2l_off[node]; g1 = t.p2l_off[node + 1]; }
-  for (int i0 = 0; i0 < t.nsurf; i0 += TILE) {
+  for (int i0 = TILE * blockIdx.y; i0 < t.nsurf; i0 += TILE * gridDim.y) {
     const int i = i0 + lane;
     const bool act = i < t.nsurf;
     R px = 0, py = 0, pz = 0;
@@ -674,15 +651,14 @@ void launch_close_find(const DevTree& t, const int* work, int nwork, int* out, i
 // The correction of each listed pair per unit charge, once per tree: one
 // thread per pair, coef[k][a] = FP64 minus FP32 value of the pair with q = 1
 // (real kernels: a = potential, gradient; Helmholtz: their (re, im) parts).
-// The FP32 operands are formed as the near-field kernel forms them: PACKED
-// (real kernels, k_p2p_smem) the source relative to its leaf centre as
-// k_pack_sources rounds it and the target moved into the source leaf's frame,
-// else (k_eval_targets) both relative to the target leaf centre.  A pair is
+// The FP32 operands are formed as the near-field kernel forms them: the source
+// relative to its leaf centre as k_pack_sources rounds it and the target moved
+// into the source leaf's frame.  A pair is
 // linear in its charge, so per evaluation its correction is q coef (complex
 // product for Helmholtz); the FP32 value of a charged pair differs from q
 // times that of a unit charge by the rounding of the products, ~1e-7 of the
 // pair's value.
-template <int KIND, bool PACKED>
+template <int KIND>
 __global__ __launch_bounds__(256) void k_close_coef(DevTree t, Wavek wk, int npairs, double* __restrict__ coef) {
   constexpr bool C = kcplx<KIND>();
   constexpr int NA = C ? 8 : 4;
@@ -703,16 +679,10 @@ __global__ __launch_bounds__(256) void k_close_coef(DevTree t, Wavek wk, int npa
     a64[a] = 0.0;
   }
   float dx, dy, dz;
-  if constexpr (PACKED) {
-    const double* rel = t.src_rel + 3 * size_t(is);
-    dx = float(rel[0]) - (tx - float(t.center[3 * sl] - cx));
-    dy = float(rel[1]) - (ty - float(t.center[3 * sl + 1] - cy));
-    dz = float(rel[2]) - (tz - float(t.center[3 * sl + 2] - cz));
-  } else {
-    dx = float(y[0] - cx) - tx;
-    dy = float(y[1] - cy) - ty;
-    dz = float(y[2] - cz) - tz;
-  }
+  const double* rel = t.src_rel + 3 * size_t(is);
+  dx = float(rel[0]) - (tx - float(t.center[3 * sl] - cx));
+  dy = float(rel[1]) - (ty - float(t.center[3 * sl + 1] - cy));
+  dz = float(rel[2]) - (tz - float(t.center[3 * sl + 2] - cz));
   // a leaf with itself: the near-field kernel left out the pairs with FP32
   // r^2 <= rmin2 (their FP32 value is 0 here too)
   if (tl == sl) pair_grad<KIND, float, RSQ_MASK>(dx, dy, dz, 1.f, 0.f, kr, ki, a32, close_rmin2<float>(t, tl));
@@ -725,9 +695,9 @@ __global__ __launch_bounds__(256) void k_close_coef(DevTree t, Wavek wk, int npa
 void launch_close_coef(int kind, const DevTree& t, Wavek k, int npairs, double* coef, hipStream_t s) {
   if (npairs <= 0) return;
   const dim3 g((npairs + 255) / 256), b(256);
-  if (kind == LAPLACE) hipLaunchKernelGGL((k_close_coef<LAPLACE, true>), g, b, 0, s, t, k, npairs, coef);
-  else if (kind == YUKAWA) hipLaunchKernelGGL((k_close_coef<YUKAWA, true>), g, b, 0, s, t, k, npairs, coef);
-  else hipLaunchKernelGGL((k_close_coef<HELMHOLTZ, false>), g, b, 0, s, t, k, npairs, coef);
+  if (kind == LAPLACE) hipLaunchKernelGGL(k_close_coef<LAPLACE>, g, b, 0, s, t, k, npairs, coef);
+  else if (kind == YUKAWA) hipLaunchKernelGGL(k_close_coef<YUKAWA>, g, b, 0, s, t, k, npairs, coef);
+  else hipLaunchKernelGGL(k_close_coef<HELMHOLTZ>, g, b, 0, s, t, k, npairs, coef);
 }
 
 // One thread per target with listed pairs, its pairs in list order (so the
@@ -765,20 +735,43 @@ __global__ __launch_bounds__(256) void k_close_fix(DevTree t) {
 
 // ---------------------------------------------------------------- launchers
 
+// Waves per tile: up to 4 while the tiles are fewer than 4 waves on each of the
+// chip's 1024 SIMDs (Helmholtz, whose pairs cost more: 16; near field of 4700 FP32
+// tiles with 1, 2, 4 waves 391, 349, 326 us), up to 16 for the few tiles of a
+// tiny tree.  More waves per tile than that only take slots from the
+// transforms beside the near field (Laplace FP64, 4096 tiles: the evaluation 917
+// us with a wave, 960 with four).  The kernels with FP64 exp or sin / cos stop
+// at 4: larger workgroups leave them too few registers (L2P of 512 Helmholtz
+// tiles 55, 81, 165 us with 4, 8, 16 waves).
+template <int KIND>
+static int particle_waves(int ntiles) {
+  int w = 1;
+  while (w < 4 && ntiles * w < (kcplx<KIND>() ? 16384 : 4096)) w *= 2;
+  while (KIND == LAPLACE && w < 16 && ntiles * w < 2048) w *= 2;
+  return w;
+}
+
 template <int KIND, typename R>
-static void eval_targets_t(int mode, const DevTree& t, Wavek k, const int* work, int nwork, const int* tiles,
-                           int ntiles, hipStream_t s) {
-  if (nwork <= 0) return;
-  const bool real = !kcplx<KIND>() && tiles && ntiles > 0;
-  if (mode == MODE_P2P && real && t.src_pack && t.src_rel) {
-    if (t.nsrcs > 0)
-      hipLaunchKernelGGL(k_pack_sources<R>, dim3((t.nsrcs + 255) / 256), dim3(256), 0, s, t.nsrcs, t.src_rel, t.q,
-                         static_cast<typename P4<R>::t*>(t.src_pack));
-    hipLaunchKernelGGL((k_p2p_smem<KIND, R>), dim3(ntiles), dim3(64), 0, s, t, k, tiles);
-  } else if (mode == MODE_P2P) hipLaunchKernelGGL((k_eval_targets<KIND, R, MODE_P2P>), dim3(nwork), dim3(64), 0, s, t, k, work);
-  else if (mode == MODE_M2P) hipLaunchKernelGGL((k_eval_targets<KIND, R, MODE_M2P>), dim3(nwork), dim3(64), 0, s, t, k, work);
-  else if (real && t.surf_tab) hipLaunchKernelGGL((k_l2p_smem<KIND, R>), dim3(ntiles), dim3(64), 0, s, t, k, tiles);
-  else hipLaunchKernelGGL((k_eval_targets<KIND, R, MODE_L2P>), dim3(nwork), dim3(64), 0, s, t, k, work);
+static void eval_targets_t(int mode, const DevTree& t, Wavek k, const int* tiles, int ntiles, hipStream_t s) {
+  if (ntiles <= 0) return;
+  if (mode == MODE_P2P && t.nsrcs > 0)
+    hipLaunchKernelGGL((k_pack_sources<R, npack<KIND>()>), dim3((t.nsrcs + 255) / 256), dim3(256), 0, s, t.nsrcs,
+                       t.src_rel, t.q, static_cast<R*>(t.src_pack));
+  auto go = [&](auto W) {
+    constexpr int w = decltype(W)::value;
+    const dim3 g(ntiles), b(64 * w);
+    if (mode == MODE_P2P) hipLaunchKernelGGL((k_p2p_smem<KIND, R, w>), g, b, 0, s, t, k, tiles);
+    else if (mode == MODE_M2P) hipLaunchKernelGGL((k_m2p<KIND, R, (w < 4 ? 4 : w)>), g, dim3(64 * (w < 4 ? 4 : w)), 0, s, t, k, tiles);
+    else hipLaunchKernelGGL((k_l2p_smem<KIND, R, w>), g, b, 0, s, t, k, tiles);
+  };
+  const int w = particle_waves<KIND>(ntiles);
+  if (w == 1) go(std::integral_constant<int, 1>());
+  else if (w == 2) go(std::integral_constant<int, 2>());
+  else if (w == 4 || KIND != LAPLACE) go(std::integral_constant<int, 4>());
+  else if constexpr (KIND == LAPLACE) {
+    if (w == 8) go(std::integral_constant<int, 8>());
+    else go(std::integral_constant<int, 16>());
+  }
   // FP32 near field: the near-coincident pairs in FP64 (same stream, after it)
   if constexpr (sizeof(R) == 4) {
     if (mode == MODE_P2P && t.nclose > 0 && t.close && t.close_off && t.close_coef)
@@ -787,18 +780,18 @@ static void eval_targets_t(int mode, const DevTree& t, Wavek k, const int* work,
   }
 }
 
-void launch_eval_targets(int kind, bool f32, int mode, const DevTree& t, Wavek k, const int* work, int nwork,
-                         const int* tiles, int ntiles, hipStream_t s) {
+void launch_eval_targets(int kind, bool f32, int mode, const DevTree& t, Wavek k, const int* tiles, int ntiles,
+                         hipStream_t s) {
   switch (kind) {
-    case LAPLACE: f32 ? eval_targets_t<LAPLACE, float>(mode, t, k, work, nwork, tiles, ntiles, s)
-                      : eval_targets_t<LAPLACE, double>(mode, t, k, work, nwork, tiles, ntiles, s); break;
-    case YUKAWA: f32 ? eval_targets_t<YUKAWA, float>(mode, t, k, work, nwork, tiles, ntiles, s)
-                     : eval_targets_t<YUKAWA, double>(mode, t, k, work, nwork, tiles, ntiles, s); break;
+    case LAPLACE: f32 ? eval_targets_t<LAPLACE, float>(mode, t, k, tiles, ntiles, s)
+                      : eval_targets_t<LAPLACE, double>(mode, t, k, tiles, ntiles, s); break;
+    case YUKAWA: f32 ? eval_targets_t<YUKAWA, float>(mode, t, k, tiles, ntiles, s)
+                     : eval_targets_t<YUKAWA, double>(mode, t, k, tiles, ntiles, s); break;
     default:
-      if (k.im == 0.0) f32 ? eval_targets_t<HELMHOLTZ_REAL, float>(mode, t, k, work, nwork, tiles, ntiles, s)
-                           : eval_targets_t<HELMHOLTZ_REAL, double>(mode, t, k, work, nwork, tiles, ntiles, s);
-      else f32 ? eval_targets_t<HELMHOLTZ, float>(mode, t, k, work, nwork, tiles, ntiles, s)
-               : eval_targets_t<HELMHOLTZ, double>(mode, t, k, work, nwork, tiles, ntiles, s);
+      if (k.im == 0.0) f32 ? eval_targets_t<HELMHOLTZ_REAL, float>(mode, t, k, tiles, ntiles, s)
+                           : eval_targets_t<HELMHOLTZ_REAL, double>(mode, t, k, tiles, ntiles, s);
+      else f32 ? eval_targets_t<HELMHOLTZ, float>(mode, t, k, tiles, ntiles, s)
+               : eval_targets_t<HELMHOLTZ, double>(mode, t, k, tiles, ntiles, s);
       break;
   }
 }
@@ -807,8 +800,13 @@ template <int KIND, typename R>
 static void eval_surface_t(int mode, const DevTree& t, Wavek k, const int* work, int nwork, double* check,
                            hipStream_t s) {
   if (nwork <= 0) return;
-  if (mode == MODE_P2M) hipLaunchKernelGGL((k_eval_surface<KIND, R, MODE_P2M>), dim3(nwork), dim3(64), 0, s, t, k, work, check);
-  else hipLaunchKernelGGL((k_eval_surface<KIND, R, MODE_P2L>), dim3(nwork), dim3(64), 0, s, t, k, work, check);
+  // the surface's chunks of 64 points over several waves while the nodes do not
+  // fill the chip (Helmholtz FP64 P2M of 512 leaves 67 -> 37 us, Laplace P2L of
+  // 2106 nodes 92 -> 40)
+  const int nchunk = (t.nsurf + TILE - 1) / TILE;
+  const dim3 g(nwork, std::max(1, std::min(nchunk, 16384 / nwork)));
+  if (mode == MODE_P2M) hipLaunchKernelGGL((k_eval_surface<KIND, R, MODE_P2M>), g, dim3(64), 0, s, t, k, work, check);
+  else hipLaunchKernelGGL((k_eval_surface<KIND, R, MODE_P2L>), g, dim3(64), 0, s, t, k, work, check);
 }
 
 void launch_eval_surface(int kind, bool f32, int mode, const DevTree& t, Wavek k, const int* work, int nwork,

@@ -1,0 +1,59 @@
+"""P2P and M2P against the oracle where the number of waves that share a tile of targets changes: trees of one
+to thousands of tiles, full tiles, tails just below and above the source split, more than one tile per leaf, the
+three kernels.  FP64 within 1e-12 of the values' norm (the operators are applied to the same inputs; sums of at most
+some 1e4 terms in another order), FP32 within 1e-5."""
+import numpy as np
+import pytest
+
+import oracle as O
+from exafmm import abi
+from fmm_cases import make_problem, rel_err
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # kernel, n, ncrit, dist: tiles and their sizes
+    ("laplace", 40, 64, "cube"),              # one leaf, one tail tile
+    ("laplace", 500, 200, "cube"),            # leaves of about 62: one tile, above and below 64
+    ("laplace", 1600, 300, "cube"),           # leaves of about 200: several tiles with tails
+    ("laplace", 9000, 30, "clusters"),        # thousands of tiles, M2P lists
+    ("modified_helmholtz", 1100, 150, "cube"),
+    ("modified_helmholtz", 7000, 12, "clusters"),
+    ("helmholtz", 70, 100, "cube"),
+    ("helmholtz", 2000, 260, "cube"),
+    ("helmholtz", 9000, 20, "clusters"),
+]
+
+
+@pytest.mark.parametrize("kernel,n,ncrit,dist", CASES)
+@pytest.mark.parametrize("precision,split", [(abi.FP64, 32), (abi.FP64, 0), (abi.FLOAT, 32)])
+def test_particle_targets(require_gpu, kernel, n, ncrit, dist, precision, split):
+    pr = make_problem(kernel, n, 4, ncrit, dist, seed=5)
+    eng = abi.Engine(pr["kid"], 4, pr["wavek"], precision)
+    eng.set_operators(pr["ops"])
+    eng.set_tree(pr["flat"])
+    eng.set_charges(pr["qs"])
+    eng.set_tuning(abi.TUNE_P2P_SPLIT, split)
+    orc = O.Oracle(pr["kid"], 4, pr["flat"], pr["ops"], pr["wavek"])
+    orc.set_charges(pr["qs"])
+    rng = np.random.default_rng(1)
+    up = rng.normal(size=(eng.nnodes, eng.nsurf))
+    if eng.cplx:
+        up = up + 1j * rng.normal(size=up.shape)
+    tol = 1e-12 if precision == abi.FP64 else 1e-5
+
+    def check(v, r):
+        if np.linalg.norm(r) == 0:
+            assert np.linalg.norm(v) == 0
+            return
+        assert rel_err(v[:, 0], r[:, 0]) < tol
+        assert rel_err(v[:, 1:], r[:, 1:]) < tol
+
+    for op in ("P2P", "M2P"):
+        eng.clear()
+        orc.clear()
+        eng.set_equiv(up=up)
+        orc.up[:] = up
+        eng.op(op)
+        orc.run(O.STAGES[op])
+        check(eng.values(), orc.val)
+    eng.close()
