@@ -235,8 +235,6 @@ struct xfmm_context {
     m.inv_dn = inv_dn.ptr;
     m.fft_in = fft_in.ptr;
     m.fft_out = fft_out.ptr;
-    m.nsrc = n_m2l_src;
-    m.ntrg = n_m2l_trg;
     m.amax = f16_had ? reinterpret_cast<unsigned*>(m2l_amax.ptr) : nullptr;
     return m;
   }
@@ -1137,7 +1135,7 @@ int xfmm_set_tree(xfmm_context* c, const xfmm_tree* t) {
     c->m2l_trg_node.upload(trgs, st);
     c->m2l_scale.upload(scale, st);
     const size_t rb = c->f32_m2l ? 4 : 8;
-    const size_t per = size_t((c->nfreq + SPEC_K - 1) / SPEC_K * SPEC_K) * NCHILD * 2 * rb;
+    const size_t per = size_t(c->nfreq) * NCHILD * 2 * rb;
     c->fft_in.alloc(per * std::max(1, c->n_m2l_src));
     c->fft_out.alloc(per * std::max(1, c->n_m2l_trg));
 

@@ -119,22 +119,10 @@ struct M2LDev {
   const int* map_up = nullptr;       // [nsurf] local index x + p (y + p z) in the [0,p)^3 input cube
   const int* map_dn = nullptr;       // [nsurf] local index in the [p,2p)^3 output cube (offset p removed)
   const int* inv_dn = nullptr;       // [p^3] inverse of map_dn: surface index of a cube point, or -1
-  // Spectra: [frequency / SPEC_K][slot][SPEC_K][8 children] complex.  The
-  // Hadamard product walks frequencies with a few hundred slots at a time:
-  // in this order those lie in one region of a few MB (with a slot's whole
-  // spectrum contiguous, 280 KB at p = 10, every slot is another page and DRAM
-  // row).
-  void* fft_in = nullptr;            // nsrc slots
-  void* fft_out = nullptr;           // ntrg slots
-  int nsrc = 0, ntrg = 0;
+  void* fft_in = nullptr;            // [nsrc_slots][nfreq][8] complex
+  void* fft_out = nullptr;           // [ntrg_slots][nfreq][8] complex
   unsigned* amax = nullptr;          // split-FP16 Hadamard: largest |spectrum value| (float bits), else null
 };
-
-constexpr int SPEC_K = 16;
-// spectrum values (of 8 children each) before frequency k of a slot
-__host__ __device__ __forceinline__ size_t spec_off(int nslots, int slot, int k) {
-  return (size_t(k / SPEC_K) * nslots + slot) * SPEC_K + k % SPEC_K;
-}
 
 // fft_up_equiv: one (source slot, child) per work item; src_node[slot] gives
 // the node whose 8 children are transformed.

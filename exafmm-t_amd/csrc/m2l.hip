@@ -118,13 +118,13 @@ __global__ __launch_bounds__(256) void k_fft_up(M2LDev m, DevTree t, const int* 
   }
   __syncthreads();
   // z pass straight to global: f = kx + nh*(ky + n1*kz)
-  C2<R>* out = reinterpret_cast<C2<R>*>(m.fft_in);
+  C2<R>* out = reinterpret_cast<C2<R>*>(m.fft_in) + size_t(slot) * m.nfreq * NCHILD;
   float mx = 0.f;
   for (int f = threadIdx.x; f < m.nfreq; f += blockDim.x) {
     const int kx = f % nh, ky = (f / nh) % n1, kz = f / (nh * n1);
     C2<R> acc{0, 0};
     for (int z = 0; z < p; z++) cfma(acc, B[(z * n1 + ky) * nh + kx], w[(kz * z) % n1]);
-    out[spec_off(m.nsrc, slot, f) * NCHILD + c] = acc;
+    out[size_t(f) * NCHILD + c] = acc;
     mx = fmaxf(mx, fmaxf(fabsf(float(acc.x)), fabsf(float(acc.y))));
   }
   if (m.amax) wave_amax(mx, m.amax);
@@ -145,14 +145,14 @@ __global__ __launch_bounds__(256) void k_ifft_dn(M2LDev m, DevTree t, const int*
   R* g = reinterpret_cast<R*>(Bp);                 // p^3 output cube (x2 complex), reuses Bp
   make_twiddles(w, n1, +1);
   __syncthreads();
-  const C2<R>* in = reinterpret_cast<const C2<R>*>(m.fft_out);
+  const C2<R>* in = reinterpret_cast<const C2<R>*>(m.fft_out) + size_t(slot) * m.nfreq * NCHILD;
   // inverse z pass for z' = p + zz
   for (int e = threadIdx.x; e < p * n1 * nh; e += blockDim.x) {
     const int kx = e % nh, ky = (e / nh) % n1, zz = e / (nh * n1);
     const int z = p + zz;
     C2<R> acc{0, 0};
     for (int kz = 0; kz < n1; kz++)
-      cfma(acc, in[spec_off(m.ntrg, slot, kx + nh * (ky + n1 * kz)) * NCHILD + c], w[(kz * z) % n1]);
+      cfma(acc, in[size_t(kx + nh * (ky + n1 * kz)) * NCHILD + c], w[(kz * z) % n1]);
     Bp[e] = acc;
   }
   __syncthreads();
@@ -491,7 +491,7 @@ __global__ __launch_bounds__(64 * NW) void k_hadamard(M2LDev m, const R* __restr
 #pragma unroll
     for (int q = 0; q < NU_Q; q++)
       if (usrc[q] >= 0) {
-        const C2<R>* f = fin + spec_off(m.nsrc, usrc[q], k) * NCHILD;
+        const C2<R>* f = fin + (size_t(usrc[q]) * m.nfreq + k) * NCHILD;
         ra[q] = f[gp];
         rb[q] = f[gp + 4];
       }
@@ -539,7 +539,7 @@ __global__ __launch_bounds__(64 * NW) void k_hadamard(M2LDev m, const R* __restr
 #pragma unroll
     for (int t = 0; t < TPW; t++)
       if (trg[t] >= 0) {
-        C2<R>* o = fout + spec_off(m.ntrg, trg[t], k) * NCHILD;
+        C2<R>* o = fout + (size_t(trg[t]) * m.nfreq + k) * NCHILD;
         o[HadRow<R>::child(MfmaT<R>::row(g, 0))] = C2<R>{acc[t][0], acc[t][1]};
         o[HadRow<R>::child(MfmaT<R>::row(g, 2))] = C2<R>{acc[t][2], acc[t][3]};
       }
@@ -640,7 +640,7 @@ __global__ __launch_bounds__(64 * NW) void k_hadamard_h(M2LDev m, const h8* __re
 #pragma unroll
     for (int q = 0; q < NU_Q; q++)
       if (usrc[q] >= 0) {
-        const f4* f = fin + spec_off(m.nsrc, usrc[q], k) * 4 + qq;
+        const f4* f = fin + (size_t(usrc[q]) * m.nfreq + k) * 4 + qq;
         ru[0][q] = f[0];
         ru[1][q] = f[4];
       }
@@ -776,8 +776,8 @@ __global__ __launch_bounds__(64 * NW) void k_hadamard_h(M2LDev m, const h8* __re
       }
       const int tx = j < 8 ? trg[t] : other, ty = j < 8 ? other : trg[t];
       const int kk = k + (j >> 3);
-      if (tx >= 0) *reinterpret_cast<v4*>(fout + spec_off(m.ntrg, tx, kk) * NCHILD + 2 * g) = x;
-      if (ty >= 0) *reinterpret_cast<v4*>(fout + spec_off(m.ntrg, ty, kk) * NCHILD + 2 * g) = y;
+      if (tx >= 0) *reinterpret_cast<v4*>(fout + (size_t(tx) * m.nfreq + kk) * NCHILD + 2 * g) = x;
+      if (ty >= 0) *reinterpret_cast<v4*>(fout + (size_t(ty) * m.nfreq + kk) * NCHILD + 2 * g) = y;
     }
     if (!early) next();
     __syncthreads();
@@ -906,7 +906,7 @@ __global__ __launch_bounds__(256) void k_fft_up_mfma(M2LDev m, DevTree t, const 
       wf[mt][ks] = (f < n1 && k < KK) ? R(dft_entry(f * v, n1, -1, RowMap<R>::ra(j), k & 1)) : R(0);
     }
   __syncthreads();
-  C2<RS>* out = reinterpret_cast<C2<RS>*>(m.fft_in);
+  C2<RS>* out = reinterpret_cast<C2<RS>*>(m.fft_in) + size_t(slot) * m.nfreq * NCHILD;
   float mx = 0.f;
   for (int kx = 0; kx < NKX; kx++) {
     // x: Ay[(y, re/im)][(z, c)] = sum_x gx[c][z][y][x] exp(-2 pi i kx x / n1),
@@ -986,7 +986,7 @@ __global__ __launch_bounds__(256) void k_fft_up_mfma(M2LDev m, DevTree t, const 
           const int kz = mt * 8 + RowMap<R>::fd(g, 2 * h);
           if (kz < n1) {
             const C2<RS> v{RS(acc[2 * h]), RS(acc[2 * h + 1])};
-            out[spec_off(m.nsrc, slot, kx * n1 * n1 + ky + n1 * kz) * NCHILD + c] = v;
+            out[size_t(kx * n1 * n1 + ky + n1 * kz) * NCHILD + c] = v;
             mx = fmaxf(mx, fmaxf(fabsf(float(v.x)), fabsf(float(v.y))));
           }
         }
@@ -1058,7 +1058,7 @@ __global__ __launch_bounds__(256) void k_ifft_dn_mfma(M2LDev m, DevTree t, const
     for (int x = 0; x < 2; x++)
 #pragma unroll
       for (int v = 0; v < VW; v++) gs[r][x][v] = R(0);
-  const C2<RS>* in = reinterpret_cast<const C2<RS>*>(m.fft_out);
+  const C2<RS>* in = reinterpret_cast<const C2<RS>*>(m.fft_out) + size_t(slot) * m.nfreq * NCHILD;
   // z-pass input fragments of this wave's tiles, loaded one slab ahead
   RS bz[NTZW][KS];
   auto fetch = [&](int kx) {
@@ -1069,7 +1069,7 @@ __global__ __launch_bounds__(256) void k_ifft_dn_mfma(M2LDev m, DevTree t, const
 #pragma unroll
       for (int kp = 0; kp < KS / 2; kp++) {
         C2<RS> v{RS(0), RS(0)};
-        if (nt < NTZ && kp * 4 + g < n1) v = in[spec_off(m.ntrg, slot, kx * n1 * n1 + ky + n1 * (kp * 4 + g)) * NCHILD + c];
+        if (nt < NTZ && kp * 4 + g < n1) v = in[size_t(kx * n1 * n1 + ky + n1 * (kp * 4 + g)) * NCHILD + c];
         bz[s][2 * kp] = v.x;
         bz[s][2 * kp + 1] = v.y;
       }
