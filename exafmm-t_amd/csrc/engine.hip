@@ -83,9 +83,12 @@ struct xfmm_context {
   bool net_heavy = false;
   bool trans32() const { return f32_trans && !net_heavy; }
   bool fft32() const { return f32_m2l_fft && !net_heavy; }
-  // dn and trg_value are zero (cleared by the last upward pass or clear_values
-  // and not written since), so the downward pass need not clear them itself
-  bool down_clean = false;
+  // dn / trg_value stand for zeros that are not written: an upward pass leaves
+  // them zero, and the downward pass that follows stores instead of adding, so
+  // they are cleared only when anything else reads or adds to them first
+  // (materialize)
+  bool dn_lazy = false, val_lazy = false;
+  bool values_out = false;  // the caller holds the address of trg_value: cleared at once
   double wk_re = 0, wk_im = 0;
   int nsurf = 0, nconv = 0, nfreq = 0, n1 = 0, vw = 1;
   bool cplx = false;
@@ -142,6 +145,12 @@ struct xfmm_context {
   DevBuf<long> leaf_slot_rows, leaf_node_rows;            // i*nsurf, node*nsurf
   std::vector<int> nl_level_off;                          // [depth+2] ranges of the non-leaf list
   DevBuf<long> nl_rows, nl_child_rows;                    // node*nsurf, child0*nsurf
+  // rows that no operator of a pass stores: up of leaves without bodies, dn of
+  // nodes whose parent is no M2L target
+  DevBuf<long> up_zero_rows, dn_zero_rows;
+  int n_up_zero = 0, n_dn_zero = 0;
+  int l2l_first = 0;                                      // first level with a dn that M2L or P2L wrote
+  bool p2p_all = false, l2p_all = false;                  // the P2P / L2P tiles hold every target exactly once
   // M2L
   int n_m2l_src = 0, n_m2l_trg = 0, n_m2l_blk = 0;
   DevBuf<int> m2l_src_node, m2l_trg_node, m2l_blk_trg, m2l_blk_uni, m2l_blk_nu, m2l_blk_lev;
@@ -325,12 +334,12 @@ void drop_graph(xfmm_context* c) {
 // ---------------------------------------------------------------- operators
 
 void op_P2M(xfmm_context* c);
-void op_M2M(xfmm_context* c);
+void op_M2M(xfmm_context* c, bool add = true);
 void op_P2L(xfmm_context* c);
 void op_M2P(xfmm_context* c);
 void op_P2P(xfmm_context* c);
-void op_L2L(xfmm_context* c);
-void op_L2P(xfmm_context* c, const double* near_add = nullptr, bool wait_near = false);
+void op_L2L(xfmm_context* c, int first = 0);
+void op_L2P(xfmm_context* c, const double* near_add = nullptr, bool wait_near = false, bool set = false);
 
 void check_ready(xfmm_context* c) {
   if (!c->have_tree) throw ArgError{"xfmm: tree not set (call xfmm_set_tree)"};
@@ -411,31 +420,34 @@ GemmGroup level_group(const xfmm_context* c, int l, int n, int k, size_t stride)
   return G;
 }
 
-void op_M2M(xfmm_context* c) {
+// add: onto the parents' densities (else they are stored)
+void op_M2M(xfmm_context* c, bool add) {
   const bool f32 = c->trans32();
   // parent row = [child_0 .. child_7] (contiguous, K = 8 nsurf) x M2Mcat
   for (int l = c->depth - 1; l >= 0; l--)
     launch_gemm_rows(f32, level_group(c, l, c->nsurf, 8 * c->nsurf, m2m_stride(c, f32)), c->up.ptr,
-                     c->nl_child_rows.ptr, gemm_op(f32, c->m2mcat, c->m2mcat32), c->up.ptr, c->nl_rows.ptr, 1,
+                     c->nl_child_rows.ptr, gemm_op(f32, c->m2mcat, c->m2mcat32), c->up.ptr, c->nl_rows.ptr, add,
                      c->stream);
 }
 
-void op_L2L(xfmm_context* c) {
+// from level `first` on
+void op_L2L(xfmm_context* c, int first) {
   const bool f32 = c->trans32();
-  for (int l = 0; l < c->depth; l++)
+  for (int l = first; l < c->depth; l++)
     launch_gemm_rows(f32, level_group(c, l, 8 * c->nsurf, c->nsurf, l2l_stride(c, f32)), c->dn.ptr, c->nl_rows.ptr,
                      gemm_op(f32, c->l2lcat, c->l2lcat32), c->dn.ptr, c->nl_child_rows.ptr, 1, c->stream);
 }
 
 // near_add (may be null): per-target values added to the L2P result (the
 // near field of a full evaluation); wait_near: they come from the second
-// stream, joined before the L2P kernel.
-void op_L2P(xfmm_context* c, const double* near_add, bool wait_near) {
+// stream, joined before the L2P kernel; set: store the values (else add to them).
+void op_L2P(xfmm_context* c, const double* near_add, bool wait_near, bool set) {
   pinv_products(c, c->r_dn, c->dn.ptr, c->leaf_node_rows.ptr, c->f32_pinv, gemm_op(c->f32_pinv, c->dc2e_uT, c->dc2e_uT32),
                 gemm_op(c->f32_pinv, c->dc2e_vT, c->dc2e_vT32), c->dn.ptr);
   DevTree t = c->dev_tree();
   if (wait_near) HIPCHK(hipStreamWaitEvent(c->stream, c->ev[20], 0));
   t.near_add = near_add;
+  t.set_values = set;
   launch_eval_targets(c->kind, c->f32_far, MODE_L2P, t, c->wavek(), c->t_l2p.ptr, c->nt_l2p, c->stream);
 }
 
@@ -506,17 +518,23 @@ void record(xfmm_context* c, int i) {
   if (c->ev_ok && !c->capturing) HIPCHK(hipEventRecord(c->ev[i], c->stream));
 }
 
+// The near-field P2P of the current charges, stored in `near`.
+void run_near(xfmm_context* c, hipStream_t s) {
+  DevTree t = c->dev_tree();
+  t.trg_value = c->near.ptr;
+  t.set_values = c->p2p_all;
+  if (!c->p2p_all) launch_zero(c->near.ptr, c->near.n, s);
+  launch_eval_targets(c->kind, c->f32_p2p, MODE_P2P, t, c->wavek(), c->t_p2p.ptr, c->nt_p2p, s);
+}
+
 // Queue the near-field P2P of the current charges on the second stream, after
 // everything already queued on the main stream.
 void launch_near(xfmm_context* c) {
   if (!c->ev_ok || c->near_pending) return;
   HIPCHK(hipEventRecord(c->ev[23], c->stream));
   HIPCHK(hipStreamWaitEvent(c->stream2, c->ev[23], 0));
-  launch_zero(c->near.ptr, c->near.n, c->stream2);
   if (!c->capturing) HIPCHK(hipEventRecord(c->ev[21], c->stream2));
-  DevTree t = c->dev_tree();
-  t.trg_value = c->near.ptr;
-  launch_eval_targets(c->kind, c->f32_p2p, MODE_P2P, t, c->wavek(), c->t_p2p.ptr, c->nt_p2p, c->stream2);
+  run_near(c, c->stream2);
   if (!c->capturing) HIPCHK(hipEventRecord(c->ev[22], c->stream2));
   HIPCHK(hipEventRecord(c->ev[20], c->stream2));
   c->near_pending = true;
@@ -649,9 +667,11 @@ void run_hadamards(xfmm_context* c, const M2LDev& m) {
   launch_hadamard(m, ops, c->f16_had ? c->m2l_hscale.ptr : nullptr, hb, c->tune_kch, had_tiles(c), c->stream);
 }
 
-void op_M2L(xfmm_context* c, bool timed) {
+// add: onto the check potentials of the targets' children (else they are stored)
+void op_M2L(xfmm_context* c, bool timed, bool add) {
   if (c->n_m2l_trg == 0) return;
   M2LDev m = c->m2l_dev();
+  m.dn_add = add;
   DevTree t = c->dev_tree();
   if (timed) record(c, 16);
   if (m.amax) launch_zero(c->m2l_amax.ptr, 1, c->stream);
@@ -661,6 +681,13 @@ void op_M2L(xfmm_context* c, bool timed) {
   if (timed) record(c, 18);
   launch_ifft_dn(m, t, c->m2l_trg_node.ptr, c->m2l_scale.ptr, c->n_m2l_trg, c->stream);
   if (timed) record(c, 19);
+}
+
+// Write the zeros that dn and trg_value stand for.
+void materialize(xfmm_context* c) {
+  if (c->dn_lazy) launch_zero(c->dn.ptr, c->dn.n, c->stream);
+  if (c->val_lazy) launch_zero(c->trg_value.ptr, c->trg_value.n, c->stream);
+  c->dn_lazy = c->val_lazy = false;
 }
 
 }  // namespace
@@ -1115,6 +1142,39 @@ int xfmm_set_tree(xfmm_context* c, const xfmm_tree* t) {
         src_slot[i] = int(srcs.size());
         srcs.push_back(i);
       }
+    {
+      const long len = long(c->nsurf) * c->vw;
+      std::vector<long> uz, dz;
+      std::vector<char> reached(nn, 0);  // dn written by M2L
+      for (int i : trgs)
+        for (int o = 0; o < 8; o++) reached[ch[i] + o] = 1;
+      c->l2l_first = D;
+      for (int i = 0; i < nn; i++) {
+        if (ch[i] < 0 && t->src_count[i] == 0 && t->trg_count[i] == 0) uz.push_back(i * len);
+        if (!reached[i]) dz.push_back(i * len);
+        if (ch[i] >= 0 && (reached[i] || t->p2l_offset[i + 1] > t->p2l_offset[i]))
+          c->l2l_first = std::min(c->l2l_first, lev[i]);
+      }
+      // a density below a level that no M2L or P2L reaches is zero, and stays so
+      c->up_zero_rows.upload(uz, st);
+      c->dn_zero_rows.upload(dz, st);
+      c->n_up_zero = int(uz.size());
+      c->n_dn_zero = int(dz.size());
+      auto all_once = [&](const std::vector<int>& w) {
+        std::vector<char> seen(t->ntrgs, 0);
+        long n = 0;
+        for (int i : w)
+          for (int k = t->trg_begin[i]; k < t->trg_begin[i] + t->trg_count[i]; k++) {
+            if (seen[k]) return false;
+            seen[k] = 1;
+            n++;
+          }
+        return n == t->ntrgs;
+      };
+      c->l2p_all = all_once(wl2p);
+      c->p2p_all = wp2p.size() == wl2p.size() && c->l2p_all;
+      HIPCHK(hipStreamSynchronize(st));  // uz, dz are temporaries
+    }
     c->h_lat.resize(size_t(nn) * 3);
     for (int i = 0; i < nn; i++) {
       const double h = 2.0 * t->r0 / double(1 << lev[i]);
@@ -1155,7 +1215,7 @@ int xfmm_set_tree(xfmm_context* c, const xfmm_tree* t) {
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
     c->have_tree = true;
-    c->down_clean = false;
+    c->dn_lazy = c->val_lazy = c->values_out = false;
     c->net_heavy = false;  // zero charges
   });
 }
@@ -1202,7 +1262,7 @@ int xfmm_set_charges_device(xfmm_context* c, const void* q) {
     if (c->prec == XFMM_MIXED) {
       double sums[3] = {0, 0, 0};
       if (c->nsrcs) {
-        c->charge_sums.alloc(3 * (CHARGE_SUM_BLOCKS + 1));
+        if (!c->charge_sums.ptr) c->charge_sums.alloc(3 * (CHARGE_SUM_BLOCKS + 1));
         launch_charge_sums(c->q.ptr, c->nsrcs, c->vw == 2, c->charge_sums.ptr, c->stream);
         HIPCHK(hipMemcpyAsync(sums, c->charge_sums.ptr + 3 * CHARGE_SUM_BLOCKS, sizeof(sums), hipMemcpyDeviceToHost,
                               c->stream));
@@ -1219,7 +1279,7 @@ int xfmm_clear_values(xfmm_context* c) {
     launch_zero(c->up.ptr, c->up.n, c->stream);
     launch_zero(c->dn.ptr, c->dn.n, c->stream);
     launch_zero(c->trg_value.ptr, c->trg_value.n, c->stream);
-    c->down_clean = true;
+    c->dn_lazy = c->val_lazy = false;
     HIPCHK(hipGetLastError());
   });
 }
@@ -1227,16 +1287,15 @@ int xfmm_clear_values(xfmm_context* c) {
 int xfmm_upward_pass(xfmm_context* c) {
   return guarded(c, [&] {
     check_ready(c);
-    // clear the accumulators of both passes (the near field of the previous
-    // evaluation has been consumed by then)
-    launch_zero(c->up.ptr, c->up.n, c->stream);
-    launch_zero(c->dn.ptr, c->dn.n, c->stream);
-    launch_zero(c->trg_value.ptr, c->trg_value.n, c->stream);
-    c->down_clean = true;
+    // P2M and M2M store every density but those of leaves without bodies
+    launch_zero_rows(c->up.ptr, c->up_zero_rows.ptr, c->n_up_zero, c->nsurf * c->vw, c->stream);
+    c->dn_lazy = true;
+    c->val_lazy = !c->values_out;
+    if (c->values_out) launch_zero(c->trg_value.ptr, c->trg_value.n, c->stream);
     record(c, 0);
     op_P2M(c);
     record(c, 1);
-    op_M2M(c);
+    op_M2M(c, false);
     record(c, 2);
     // the near field goes on the second stream here, so that it overlaps
     // the downward pass (measured: starting it with the upward pass, where it
@@ -1249,35 +1308,30 @@ int xfmm_upward_pass(xfmm_context* c) {
 int xfmm_downward_pass(xfmm_context* c) {
   return guarded(c, [&] {
     check_ready(c);
-    if (!c->down_clean) {
-      launch_zero(c->dn.ptr, c->dn.n, c->stream);
-      launch_zero(c->trg_value.ptr, c->trg_value.n, c->stream);
-    }
-    c->down_clean = false;
+    // every value and check potential is stored by the first operator that
+    // reaches it: L2P (M2P where leaves have such lists), M2L and, for what M2L
+    // does not reach, the zero rows; the rest adds
+    const bool m2p = c->nt_m2p > 0, set = c->l2p_all && !m2p;
+    if (!set) launch_zero(c->trg_value.ptr, c->trg_value.n, c->stream);
     record(c, 3);
-    op_P2L(c);
-    record(c, 4);
     op_M2P(c);
     record(c, 5);
     // near field: taken from the second stream when the upward pass started
     // it, else computed here; either way it is added last, so both give
     // identical values
     const bool pend = c->near_pending;
-    if (!pend) {
-      DevTree t = c->dev_tree();
-      t.trg_value = c->near.ptr;
-      launch_zero(c->near.ptr, c->near.n, c->stream);
-      launch_eval_targets(c->kind, c->f32_p2p, MODE_P2P, t, c->wavek(), c->t_p2p.ptr, c->nt_p2p, c->stream);
-    }
+    if (!pend) run_near(c, c->stream);
     record(c, 6);
-    op_M2L(c, true);
+    launch_zero_rows(c->dn.ptr, c->dn_zero_rows.ptr, c->n_dn_zero, c->nsurf * c->vw, c->stream);
+    op_M2L(c, true, false);
     record(c, 7);
-    op_L2L(c);
+    op_P2L(c);
+    record(c, 11);
+    op_L2L(c, c->l2l_first);
     record(c, 8);
-    // every leaf with targets has an L2P work item, so the L2P kernel adds
-    // the near field to each target's result exactly once
-    op_L2P(c, c->near.ptr, pend);
+    op_L2P(c, c->near.ptr, pend, set);
     record(c, 9);
+    c->dn_lazy = c->val_lazy = false;
     if (c->vscale.ptr) launch_scale_values(c->trg_value.ptr, c->vscale.ptr, c->ntrgs, c->vw, c->stream);
     c->near_pending = false;
     c->near_overlapped = pend;
@@ -1292,6 +1346,8 @@ int xfmm_graph_capture(xfmm_context* c) {
     HIPCHK(hipStreamSynchronize(c->stream));
     HIPCHK(hipStreamSynchronize(c->stream2));
     c->near_pending = false;
+    materialize(c);  // what is captured does not run now
+    HIPCHK(hipStreamSynchronize(c->stream));
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     c->capturing = true;
     int rc = xfmm_upward_pass(c);
@@ -1307,7 +1363,6 @@ int xfmm_graph_capture(xfmm_context* c) {
     c->graph = g;
     HIPCHK(hipGraphInstantiate(&c->graph_exec, c->graph, nullptr, nullptr, 0));
     c->near_pending = false;
-    c->down_clean = false;
   });
 }
 
@@ -1319,7 +1374,7 @@ int xfmm_graph_launch(xfmm_context* c) {
     // afterwards is that of a completed evaluation
     HIPCHK(hipGraphLaunch(c->graph_exec, c->stream));
     c->near_pending = false;
-    c->down_clean = false;
+    c->dn_lazy = c->val_lazy = false;
   });
 }
 
@@ -1327,7 +1382,7 @@ int xfmm_graph_launch(xfmm_context* c) {
   int xfmm_##NAME(xfmm_context* c) {                    \
     return guarded(c, [&] {                             \
       check_ready(c);                                   \
-      c->down_clean = false;                            \
+      materialize(c);                                   \
       op_##NAME(c);                                     \
       HIPCHK(hipGetLastError());                        \
     });                                                 \
@@ -1342,8 +1397,8 @@ XFMM_OP(L2P)
 int xfmm_M2L(xfmm_context* c) {
   return guarded(c, [&] {
     check_ready(c);
-    c->down_clean = false;
-    op_M2L(c, false);
+    materialize(c);
+    op_M2L(c, false, true);
     HIPCHK(hipGetLastError());
   });
 }
@@ -1352,6 +1407,7 @@ int xfmm_get_values(xfmm_context* c, double* v) {
   return guarded(c, [&] {
     require(c->have_tree, "xfmm_get_values: tree not set");
     require(v || c->ntrgs == 0, "xfmm_get_values: null output");
+    materialize(c);
     if (c->ntrgs)
       HIPCHK(hipMemcpyAsync(v, c->trg_value.ptr, size_t(c->ntrgs) * 4 * c->vw * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -1361,6 +1417,7 @@ int xfmm_get_values(xfmm_context* c, double* v) {
 int xfmm_get_equiv(xfmm_context* c, double* up, double* dn) {
   return guarded(c, [&] {
     require(c->have_tree, "xfmm_get_equiv: tree not set");
+    materialize(c);
     const size_t n = size_t(c->nnodes) * c->nsurf * c->vw * sizeof(double);
     if (up) HIPCHK(hipMemcpyAsync(up, c->up.ptr, n, hipMemcpyDeviceToHost, c->stream));
     if (dn) HIPCHK(hipMemcpyAsync(dn, c->dn.ptr, n, hipMemcpyDeviceToHost, c->stream));
@@ -1371,10 +1428,10 @@ int xfmm_get_equiv(xfmm_context* c, double* up, double* dn) {
 int xfmm_set_equiv(xfmm_context* c, const double* up, const double* dn) {
   return guarded(c, [&] {
     require(c->have_tree, "xfmm_set_equiv: tree not set");
+    materialize(c);
     const size_t n = size_t(c->nnodes) * c->nsurf * c->vw * sizeof(double);
     if (up) HIPCHK(hipMemcpyAsync(c->up.ptr, up, n, hipMemcpyHostToDevice, c->stream));
     if (dn) HIPCHK(hipMemcpyAsync(c->dn.ptr, dn, n, hipMemcpyHostToDevice, c->stream));
-    if (dn) c->down_clean = false;
     HIPCHK(hipStreamSynchronize(c->stream));
   });
 }
@@ -1383,7 +1440,8 @@ int xfmm_values_device(xfmm_context* c, void** ptr) {
   return guarded(c, [&] {
     require(c->have_tree && ptr, "xfmm_values_device: tree not set or null output");
     *ptr = c->trg_value.ptr;
-    c->down_clean = false;  // the caller may write through the pointer
+    materialize(c);
+    c->values_out = true;
   });
 }
 
@@ -1402,7 +1460,7 @@ int xfmm_timings(const xfmm_context* cc, double* ms, int cap) {
   // P2M M2M P2L M2P P2P M2L L2L L2P FFT HAD IFFT; P2P from the second stream
   // when it ran there (overlapped with the other operators)
   const bool ov = c->near_overlapped;
-  const int pairs[11][2] = {{0, 1}, {1, 2}, {3, 4}, {4, 5}, {ov ? 21 : 5, ov ? 22 : 6}, {6, 7}, {7, 8}, {8, 9},
+  const int pairs[11][2] = {{0, 1}, {1, 2}, {7, 11}, {3, 5}, {ov ? 21 : 5, ov ? 22 : 6}, {6, 7}, {11, 8}, {8, 9},
                             {16, 17}, {17, 18}, {18, 19}};
   int n = 0;
   for (int i = 0; i < 11 && n < cap; i++) {
@@ -1468,7 +1526,7 @@ int xfmm_autotune(xfmm_context* c, int reps, double* best_ms) {
     HIPCHK(hipStreamSynchronize(c->stream));
     HIPCHK(hipStreamSynchronize(c->stream2));
     c->near_pending = false;
-    c->down_clean = false;
+    materialize(c);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     HIPCHK(hipEventCreate(&e0));
     struct EvGuard {

@@ -350,6 +350,15 @@ void launch_zero(double* p, size_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_zero, dim3(unsigned(blocks)), dim3(256), 0, s, p, n);
 }
 
+__global__ __launch_bounds__(256) void k_zero_rows(double* __restrict__ p, const long* __restrict__ rows, int len) {
+  double* r = p + rows[blockIdx.x];
+  for (int i = threadIdx.x; i < len; i += 256) r[i] = 0.0;
+}
+
+void launch_zero_rows(double* p, const long* rows, int n, int len, hipStream_t s) {
+  if (n > 0) hipLaunchKernelGGL(k_zero_rows, dim3(n), dim3(256), 0, s, p, rows, len);
+}
+
 __global__ __launch_bounds__(256) void k_charge_sums(const double* __restrict__ q, int n, bool cplx,
                                                      double* __restrict__ out) {
   __shared__ double red[3][256];
@@ -372,16 +381,20 @@ __global__ __launch_bounds__(256) void k_charge_sums(const double* __restrict__ 
   if (threadIdx.x < 3) out[3 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
 }
 
-__global__ void k_charge_sums_total(double* __restrict__ out) {
-  if (threadIdx.x >= 3) return;
+// One wave per sum: the block sums of a lane, then the lanes, in a fixed order
+// (a thread per sum over all 256 blocks: 7 us of load latency, this 3).
+__global__ __launch_bounds__(192) void k_charge_sums_total(double* __restrict__ out) {
+  const int k = threadIdx.x >> 6, lane = threadIdx.x & 63;
   double t = 0;
-  for (int b = 0; b < CHARGE_SUM_BLOCKS; b++) t += out[3 * b + threadIdx.x];
-  out[3 * CHARGE_SUM_BLOCKS + threadIdx.x] = t;
+#pragma unroll
+  for (int b = 0; b < CHARGE_SUM_BLOCKS / 64; b++) t += out[3 * (lane + 64 * b) + k];
+  for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o, 64);
+  if (lane == 0) out[3 * CHARGE_SUM_BLOCKS + k] = t;
 }
 
 void launch_charge_sums(const double* q, int n, bool cplx, double* out, hipStream_t s) {
   hipLaunchKernelGGL(k_charge_sums, dim3(CHARGE_SUM_BLOCKS), dim3(256), 0, s, q, n, cplx, out);
-  hipLaunchKernelGGL(k_charge_sums_total, dim3(1), dim3(64), 0, s, out);
+  hipLaunchKernelGGL(k_charge_sums_total, dim3(1), dim3(192), 0, s, out);
 }
 
 __global__ void k_scale_values(double* __restrict__ val, const double* __restrict__ scale, int n, int vw) {

@@ -38,6 +38,7 @@ struct DevTree {
   double* trg_value = nullptr;        // T[ntrgs][4]
   const double* near_add = nullptr;   // L2P only (may be null): [ntrgs][4] values that the L2P kernels add to
                                       // each target's result after their own sum (the evaluation's near field)
+  bool set_values = false;            // P2P / M2P / L2P store their values (else they add to trg_value)
   int p2p_split = 32;                 // P2P / M2P / L2P: tail tiles of <= p2p_split targets (<= 32) split their sources over lanes
   const int* close = nullptr;         // near-coincident P2P pairs, [4] ints (target, source, target leaf, source leaf), sorted by target
   const int* close_off = nullptr;     // [nclose + 1]: pairs of the k-th target with any are close[close_off[k] .. close_off[k + 1])
@@ -119,6 +120,7 @@ struct M2LDev {
   const int* map_up = nullptr;       // [nsurf] local index x + p (y + p z) in the [0,p)^3 input cube
   const int* map_dn = nullptr;       // [nsurf] local index in the [p,2p)^3 output cube (offset p removed)
   const int* inv_dn = nullptr;       // [p^3] inverse of map_dn: surface index of a cube point, or -1
+  bool dn_add = true;                // inverse transform: add to dn (else store)
   void* fft_in = nullptr;            // [nsrc_slots][nfreq][8] complex
   void* fft_out = nullptr;           // [ntrg_slots][nfreq][8] complex
   unsigned* amax = nullptr;          // split-FP16 Hadamard: largest |spectrum value| (float bits), else null
@@ -166,8 +168,8 @@ void launch_hadamard(const M2LDev& m, const void* m2l_opsx, const float* hscale,
 // With hscale != null (mixed only) the split-FP16 form of k_hadamard_h
 // instead (same size), and hscale[L][k] receives the operator scales.
 void launch_m2l_expand(const M2LDev& m, int nlev, const void* M, void* X, float* hscale, hipStream_t s);
-// ifft_dn_check: one (target slot, child) per work item, adds
-// scale[slot] * result to the child's dn vector.
+// ifft_dn_check: one (target slot, child) per work item, adds (m.dn_add, else
+// stores) scale[slot] * result to the child's dn vector.
 void launch_ifft_dn(const M2LDev& m, const DevTree& t, const int* trg_node, const double* scale, int nslots,
                     hipStream_t s);
 
@@ -175,6 +177,8 @@ void launch_ifft_dn(const M2LDev& m, const DevTree& t, const int* trg_node, cons
 size_t m2l_lds_bytes(const M2LDev& m);
 
 void launch_zero(double* p, size_t n, hipStream_t s);
+// p[rows[i] .. rows[i] + len) = 0 for i < n
+void launch_zero_rows(double* p, const long* rows, int n, int len, hipStream_t s);
 // {Re sum q, Im sum q, sum |q|} of n charges (complex: interleaved pairs),
 // in a fixed order: per-block partial sums in out[0 .. 3 CHARGE_SUM_BLOCKS),
 // their total in out[3 CHARGE_SUM_BLOCKS .. + 3)

@@ -194,10 +194,10 @@ __global__ __launch_bounds__(256) void k_ifft_dn(M2LDev m, DevTree t, const int*
   for (int i = threadIdx.x; i < m.nsurf; i += blockDim.x) {
     const int l = m.map_dn[i];
     if (CPLX) {
-      dn[2 * i] += sc * double(g[2 * l]);
-      dn[2 * i + 1] += sc * double(g[2 * l + 1]);
+      dn[2 * i] = (m.dn_add ? dn[2 * i] : 0.0) + sc * double(g[2 * l]);
+      dn[2 * i + 1] = (m.dn_add ? dn[2 * i + 1] : 0.0) + sc * double(g[2 * l + 1]);
     } else {
-      dn[i] += sc * double(g[l]);
+      dn[i] = (m.dn_add ? dn[i] : 0.0) + sc * double(g[l]);
     }
   }
 }
@@ -998,7 +998,7 @@ __global__ __launch_bounds__(256) void k_fft_up_mfma(M2LDev m, DevTree t, const 
   if (m.amax) wave_amax(mx, m.amax);
 }
 
-// ifft_dn_check for one node: dn[c][i] += scale * sum over (kx, ky, kz) of
+// ifft_dn_check for one node: dn[c][i] (+)= scale * sum over (kx, ky, kz) of
 // w(kx) Re(in(kx,ky,kz)[c] exp(+2 pi i (kx x + ky y + kz z) / n1)) at the
 // child's check-surface points (x,y,z) in [p,2p)^3, w = 1 for kx = 0 and the
 // Nyquist plane, else 2 (c2r of the half spectrum; reference
@@ -1170,7 +1170,10 @@ __global__ __launch_bounds__(256) void k_ifft_dn_mfma(M2LDev m, DevTree t, const
     const int i = m.inv_dn[(z * P + y) * P + x];
     if (i >= 0) {
 #pragma unroll
-      for (int v = 0; v < VW; v++) dn[(size_t(c) * ns + i) * VW + v] += sc * double(gv[v]);
+      for (int v = 0; v < VW; v++) {
+        double* d = dn + (size_t(c) * ns + i) * VW + v;
+        *d = (m.dn_add ? *d : 0.0) + sc * double(gv[v]);
+      }
     }
   };
 #pragma unroll

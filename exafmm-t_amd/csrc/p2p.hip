@@ -214,8 +214,8 @@ struct Tile {
   }
 };
 
-// trg_value (+ near_add) of the tile's targets += the sums of its lanes and
-// waves / 4 pi.
+// trg_value of the tile's targets = (with t.set_values) or += the sums of its
+// lanes and waves / 4 pi (+ near_add).
 template <int NA, int W, typename R>
 __device__ __forceinline__ void put_tile(const DevTree& t, const Tile<R>& T, const R* acc, const R* comp,
                                          const double* near_add) {
@@ -223,7 +223,10 @@ __device__ __forceinline__ void put_tile(const DevTree& t, const Tile<R>& T, con
     double* o = t.trg_value + size_t(T.tb + i) * NA;
     const double* n = near_add ? near_add + size_t(T.tb + i) * NA : nullptr;
 #pragma unroll
-    for (int a = 0; a < NA; a++) o[a] = n ? (o[a] + v[a] * FOUR_PI_INV) + n[a] : o[a] + v[a] * FOUR_PI_INV;
+    for (int a = 0; a < NA; a++) {
+      const double r = (t.set_values ? 0.0 : o[a]) + v[a] * FOUR_PI_INV;
+      o[a] = n ? r + n[a] : r;
+    }
   };
   if (W == 1 && !T.split) {
     if (T.act) {

@@ -57,3 +57,49 @@ def test_particle_targets(require_gpu, kernel, n, ncrit, dist, precision, split)
         orc.run(O.STAGES[op])
         check(eng.values(), orc.val)
     eng.close()
+
+
+@pytest.mark.parametrize("kernel,n,ncrit,dist", [("laplace", 9000, 30, "clusters"), ("helmholtz", 2000, 260, "cube")])
+def test_passes_read_as_zeroed(require_gpu, kernel, n, ncrit, dist):
+    """After an upward pass the target values and dn read as zero, single operators add to zeros, and a pass after
+    foreign values, in another order or repeated gives the values of a fresh one bit for bit."""
+    pr = make_problem(kernel, n, 4, ncrit, dist, seed=6)
+
+    def engine():
+        eng = abi.Engine(pr["kid"], 4, pr["wavek"], abi.FP64)
+        eng.set_operators(pr["ops"])
+        eng.set_tree(pr["flat"])
+        eng.set_charges(pr["qs"])
+        return eng
+
+    a = engine()
+    a.upward_pass()
+    a.downward_pass()
+    want, (up, dn) = a.values(), a.equiv()
+    a.upward_pass()
+    assert not np.any(a.values()) and not np.any(a.equiv()[1])
+    assert np.array_equal(a.equiv()[0], up)
+    a.op("P2P")
+    p2p = a.values()
+    a.op("P2P")
+    assert np.array_equal(a.values(), 2 * p2p)
+    a.downward_pass()
+    assert np.array_equal(a.values(), want) and np.array_equal(a.equiv()[1], dn)
+    b = engine()
+    b.values_device_ptr()
+    b.set_equiv(up=np.full(up.shape, 7.0), dn=np.full(dn.shape, 7.0))
+    b.op("P2P")
+    b.upward_pass()
+    assert not np.any(b.values())
+    b.upward_pass()
+    b.downward_pass()
+    assert np.array_equal(b.values(), want)
+    assert np.array_equal(b.equiv()[0], up) and np.array_equal(b.equiv()[1], dn)
+    b.graph_capture()
+    b.upward_pass()
+    assert not np.any(b.equiv()[1])
+    for _ in range(3):
+        b.graph_launch()
+        assert np.array_equal(b.values(), want) and np.array_equal(b.equiv()[1], dn)
+    a.close()
+    b.close()
