@@ -292,10 +292,11 @@ static void launch_tiles(GemmGroup G, const double* A, const long* arow, const C
 
 // Tile and K split by the number of 32 x 64 (w4) and 32 x 32 (w2) wave tiles
 // against the chip's 1024 SIMDs, and by the length of K (measured, us):
-//  w4 >= 768: 64 x 128 workgroups of four 32 x 64 tiles (FP64 4096 x 481 x
-//    488, w4 = 1024: 39, 32 x 64 with K over 4 waves 42, 32 x 32 over 4 42),
-//    but K over 4 waves when K is long (FP32 4096 x 488 x 3904, w4 = 1024:
-//    203 -> 157);
+//  w4 >= 2560: 64 x 128 workgroups of four 32 x 64 tiles (2.5 waves a SIMD hide
+//    their own loads; 16 Plummer problems, L2L of some 870 x 2368 x 296, w4 = 1036:
+//    the evaluation 3365 with them, 3260 with 32 x 32 tiles);
+//  w4 >= 768 and K long: 32 x 64 tiles with K over 4 waves (FP32 4096 x 488 x 3904,
+//    w4 = 1024: 157, four waves without a split 203);
 //  w2 >= 128: 32 x 32 tiles with K over 4 waves (FP64 4096 x 160 x 296, w2 =
 //    640: 12, four waves without a split 14, 32 x 64 23), over 8 or 16
 //    when K is long (FP64 512 x 296 x 2368, w2 = 160: 28 with 4, 26 with 8; FP32
@@ -315,7 +316,7 @@ static void launch_group(const GemmGroup& G, const double* A, const long* arow, 
     k = std::max(k, sg.k);
   }
   const bool klong = k >= 1024;
-  if (w4 >= 768) {
+  if (w4 >= (klong ? 768 : 2560)) {
     if (klong) launch_tiles<CT, 2, 4, 4, 1, 1>(G, A, arow, B, C, crow, beta, s);
     else launch_tiles<CT, 2, 4, 1, 2, 2>(G, A, arow, B, C, crow, beta, s);
   } else if (w2 >= 128) {
