@@ -9,8 +9,8 @@
 //   Helmholtz helmholtz.h:186-207:          phi += q e^{ikr}/r,    grad += (1/r^2 - ik/r) phi_ij d
 // Pairs with r = 0 contribute nothing (laplace.h:57, `invr &= r2 > zero`).
 //
-// Layout: particle targets in tiles of 64 per leaf, a target per lane, sources
-// read as wave-uniform vectors; surface targets with a wave per node, sources
+// Layout: particle targets in tiles of 64 per leaf (P2P and M2P: sources in LDS;
+// L2P: a target per lane, sources read as wave-uniform vectors); surface targets with a wave per node, sources
 // staged through LDS in tiles of 64.  Coordinates are made relative to a leaf
 // centre in FP64 before any FP32 conversion, so the mixed path keeps
 // |d| accuracy at the scale of the leaf.  In the FP32 path each tile of 64
@@ -166,7 +166,7 @@ __device__ __forceinline__ R close_rmin2(const DevTree& t, int leaf) {
 // ---------------------------------------------- particle targets: P2P, M2P, L2P
 //
 // One workgroup of W waves per (leaf, tile of TILE targets), work[2 b] = leaf,
-// work[2 b + 1] = tile.  A full tile has a target per lane and reads its
+// work[2 b + 1] = tile.  L2P and M2P: a full tile has a target per lane and reads its
 // sources as wave-uniform vectors (scalar loads from constant address space,
 // no LDS and no barriers); a tail tile of nt <= t.p2p_split (<= TILE / 2)
 // targets gives each target TILE / nt lanes (target lane % nt, phase lane /
@@ -340,9 +340,7 @@ __device__ __forceinline__ void sum_split(int n, const Tile<R>& T, SRC src, R ux
 }
 
 // Near field (fmm_base.h:82-94).  Each source is packed once per evaluation as
-// (x, y, z, q[, Im q]) relative to its leaf centre; a target is moved into the
-// frame of the source leaf with one subtraction per source leaf (the offset
-// of the two centres is formed in FP64).
+// (x, y, z, q[, Im q]) relative to its leaf centre.
 template <int KIND>
 constexpr int npack() { return kcplx<KIND>() ? 5 : 4; }
 
@@ -360,39 +358,147 @@ __global__ void k_pack_sources(int n, const double* __restrict__ rel, const doub
   for (int d = 0; d < NP; d++) out[size_t(i) * NP + d] = v[d];
 }
 
+// A workgroup of W waves per (leaf, tile of TILE targets).  A lane holds M targets
+// (target l + u L of the tile in lane l, L = ceil(nt / M)), so that k = 64 / L
+// lanes share a target's sources and few lanes are left over: leaves of 24
+// targets use 60 of 64 lanes (48 with one target in a lane).  The sources of
+// all leaves of the list are one sequence, moved into the target leaf's frame
+// (the offset of the centres formed in FP64) on their way to LDS, padded with
+// zero charges to whole trips of the loop; the W waves take a part of every
+// block each, the k lane groups every k-th source of it, two of them per trip,
+// and the sums are added in FP64 in a fixed order.  A tile of more than
+// t.p2p_split targets uses two lane groups at most.
+// Bound by the vector units: 17 instructions (Laplace) a pair, 1/sqrt at a
+// quarter rate.  Per source leaf and tile instead (full tiles with a target per
+// lane and scalar loads, others with the lane groups reading each leaf from the
+// vector cache) the small leaves paid for remainders and for 16 lanes' worth
+// of cache reads a pair.  Before -> after: FP32, 32768 leaves of 30 targets 519
+// -> 465 us, of 61 1214 -> 1190; 38841 Plummer leaves of 15 478 -> 371; Yukawa FP32,
+// 15074 leaves of 20 220 -> 178; FP64, 12069 leaves of 41 1228 -> 1115; Helmholtz
+// FP64, 512 leaves of 59 268 -> 225.  128 sources a wave: 256 and 512 cost 2 and 20
+// % (fewer workgroups on a CU); the next block loaded ahead gives nothing.
+// M = 1 for Helmholtz FP32, whose registers M = 2 halves the waves with (4096
+// leaves of 49: 312 and 327 us).
 template <int KIND, typename R, int W>
-__global__ __launch_bounds__(64 * W) void k_p2p_smem(DevTree t, Wavek wk, const int* __restrict__ work) {
-  constexpr int NA = nval<KIND>(), NP = npack<KIND>();
-  // constant address space: the packed sources are read-only for the whole
-  // launch, and wave-uniform loads from it become scalar loads
-  typedef const R __attribute__((address_space(4))) * CR;
-  const R* pack = static_cast<const R*>(t.src_pack);
-  const Tile<R> T(t, work);
-  const R kr = R(wk.re), ki = R(wk.im);
-  const R rmin2 = close_rmin2<R>(t, T.leaf);
-  R acc[NA], comp[NA];
+__global__ __launch_bounds__(64 * W) void k_p2p(DevTree t, Wavek wk, const int* __restrict__ work) {
+  constexpr int NA = nval<KIND>(), NP = npack<KIND>(), M = kcplx<KIND>() && sizeof(R) == 4 ? 1 : 2;
+  constexpr int CAP = 128 * W;  // sources in LDS
+  constexpr int NE = 64;        // source leaves listed at a time
+  constexpr int SZ = std::max(int(CAP * NP * sizeof(R)), int(W * NA * 64 * sizeof(double)));
+  __shared__ __attribute__((aligned(16))) char smem[SZ];
+  __shared__ int pre[NE + 1], first[NE], self;
+  __shared__ R off[3][NE];
+  R* sp = reinterpret_cast<R*>(smem);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int leaf = work[2 * blockIdx.x], t0 = TILE * work[2 * blockIdx.x + 1];
+  const int tb = t.trg_begin[leaf] + t0, nt = min(TILE, t.trg_count[leaf] - t0);
+  const int L = (nt + M - 1) / M, kmax = 64 / L, k = nt <= t.p2p_split ? kmax : min(kmax, 2);
+  const int l = lane % L, ph = lane / L < k ? lane / L : 0;
+  const double cx = t.center[3 * leaf], cy = t.center[3 * leaf + 1], cz = t.center[3 * leaf + 2];
+  const R far = R(4.0 * t.r0 * ldexp(1.0, -t.level[leaf]));
+  const R kr = R(wk.re), ki = R(wk.im), rmin2 = close_rmin2<R>(t, leaf);
+  R x[M][3], acc[M][NA], comp[M][NA];
 #pragma unroll
-  for (int a = 0; a < NA; a++) { acc[a] = 0; comp[a] = 0; }
-  for (int g = t.p2p_off[T.leaf] + T.wave; g < t.p2p_off[T.leaf + 1]; g += W) {
-    const int snode = t.p2p_src[g];
-    const int sb = t.src_begin[snode], ns = t.src_count[snode];
-    // target in the frame of the source leaf
-    const R ux = T.tx - R(t.center[3 * snode] - T.cx);
-    const R uy = T.ty - R(t.center[3 * snode + 1] - T.cy);
-    const R uz = T.tz - R(t.center[3 * snode + 2] - T.cz);
-    const R* S = pack + size_t(NP) * sb;
-    const Sources<R, NP - 3, NP, 0, const R*, int> vec(S, 0);
-    const Sources<R, NP - 3, NP, 0, CR, int> uni((CR)(S), 0);
-    // only a leaf with itself can pair coinciding points
-    if (snode == T.leaf) {
-      if (T.split) sum_split<KIND, R, RSQ_MASK>(ns, T, vec, ux, uy, uz, kr, ki, acc, comp, rmin2);
-      else sum_uniform<KIND, R, RSQ_MASK>(ns, uni, ux, uy, uz, kr, ki, acc, comp, rmin2);
-    } else {
-      if (T.split) sum_split<KIND, R, RSQ_SEP>(ns, T, vec, ux, uy, uz, kr, ki, acc, comp, R(0));
-      else sum_uniform<KIND, R, RSQ_SEP>(ns, uni, ux, uy, uz, kr, ki, acc, comp, R(0));
+  for (int u = 0; u < M; u++) {
+    const double* p = t.trg + 3 * size_t(tb + min(l + u * L, nt - 1));
+    x[u][0] = R(p[0] - cx);
+    x[u][1] = R(p[1] - cy);
+    x[u][2] = R(p[2] - cz);
+#pragma unroll
+    for (int a = 0; a < NA; a++) { acc[u][a] = 0; comp[u][a] = 0; }
+  }
+  const int unit = 2 * W * k, most = min(CAP / unit * unit, TILE * W * k);  // at most TILE sources a lane and block
+  const R* pack = static_cast<const R*>(t.src_pack);
+  // all pairs of total sources, source i read by load(i, v)
+  auto sums = [&](auto RM, int total, auto load) {
+    for (int s0 = 0; s0 < total; s0 += most) {
+      const int m = min(most, total - s0), n = (m + unit - 1) / unit * unit, steps = n / (W * k);
+      __syncthreads();
+      for (int i = tid; i < n; i += 64 * W) {
+        R v[NP] = {far};
+        if (i < m) load(s0 + i, v);
+#pragma unroll
+        for (int d = 0; d < NP; d++) sp[NP * i + d] = v[d];
+      }
+      __syncthreads();
+      const R* S = sp + NP * (wave * steps * k + ph);
+      R part[M][NA] = {};
+      for (int j = 0; j < steps; j += 2) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          const R w[5] = {S[0], S[1], S[2], S[3], NP > 4 ? S[NP - 1] : R(0)};
+          S += NP * k;
+#pragma unroll
+          for (int u = 0; u < M; u++)
+            pair_grad<KIND, R, decltype(RM)::value>(w[0] - x[u][0], w[1] - x[u][1], w[2] - x[u][2], w[3], w[4], kr, ki,
+                                                    part[u], rmin2);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < M; u++) fold_tile<R, NA>(acc[u], comp[u], part[u]);
+    }
+  };
+  if (tid == 0) self = 0;
+  const int g1 = t.p2p_off[leaf + 1];
+  for (int g0 = t.p2p_off[leaf]; g0 < g1; g0 += NE) {
+    __syncthreads();
+    if (tid < NE) {
+      int n = 0;
+      if (g0 + tid < g1) {
+        const int s = t.p2p_src[g0 + tid];
+        if (s == leaf) self = 1;
+        else n = t.src_count[s];
+        first[tid] = t.src_begin[s];
+        off[0][tid] = R(t.center[3 * s] - cx);
+        off[1][tid] = R(t.center[3 * s + 1] - cy);
+        off[2][tid] = R(t.center[3 * s + 2] - cz);
+      }
+#pragma unroll
+      for (int d = 1; d < 64; d *= 2) {
+        const int o = __shfl_up(n, d);
+        if (tid >= d) n += o;
+      }
+      pre[tid + 1] = n;
+      if (tid == 0) pre[0] = 0;
+    }
+    __syncthreads();
+    sums(std::integral_constant<int, RSQ_SEP>(), pre[NE], [&](int i, R* v) {
+      int e = 0;  // the last leaf with pre[e] <= i
+#pragma unroll
+      for (int d = NE / 2; d > 0; d /= 2)
+        if (pre[e + d] <= i) e += d;
+      const R* p = pack + size_t(NP) * (first[e] + i - pre[e]);
+#pragma unroll
+      for (int d = 0; d < NP; d++) v[d] = p[d];
+#pragma unroll
+      for (int d = 0; d < 3; d++) v[d] += off[d][e];
+    });
+  }
+  __syncthreads();
+  // only a leaf with itself can pair coinciding points
+  if (self)
+    sums(std::integral_constant<int, RSQ_MASK>(), t.src_count[leaf], [&](int i, R* v) {
+      const R* p = pack + size_t(NP) * (t.src_begin[leaf] + i);
+#pragma unroll
+      for (int d = 0; d < NP; d++) v[d] = p[d];
+    });
+  double* red = reinterpret_cast<double*>(smem);
+#pragma unroll
+  for (int u = 0; u < M; u++) {
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < NA; a++) red[(wave * NA + a) * 64 + lane] = double(acc[u][a]) - double(comp[u][a]);
+    __syncthreads();
+    const int n = min(L, nt - u * L);
+    for (int i = tid; i < n * NA; i += 64 * W) {
+      const int ti = i / NA, a = i % NA;
+      double v = 0;
+      for (int w = 0; w < W; w++)
+        for (int h = 0; h < k; h++) v += red[(w * NA + a) * 64 + ti + h * L];
+      double* o = t.trg_value + size_t(tb + u * L) * NA + i;
+      *o = (t.set_values ? 0.0 : *o) + v * FOUR_PI_INV;
     }
   }
-  put_tile<NA, W>(t, T, acc, comp, nullptr);
 }
 
 // L2P (fmm_scale_invariant.h:198-230, fmm.h:188-218).  The sources are the points
@@ -683,9 +789,9 @@ __global__ __launch_bounds__(256) void k_close_coef(DevTree t, Wavek wk, int npa
   }
   float dx, dy, dz;
   const double* rel = t.src_rel + 3 * size_t(is);
-  dx = float(rel[0]) - (tx - float(t.center[3 * sl] - cx));
-  dy = float(rel[1]) - (ty - float(t.center[3 * sl + 1] - cy));
-  dz = float(rel[2]) - (tz - float(t.center[3 * sl + 2] - cz));
+  dx = (float(rel[0]) + float(t.center[3 * sl] - cx)) - tx;
+  dy = (float(rel[1]) + float(t.center[3 * sl + 1] - cy)) - ty;
+  dz = (float(rel[2]) + float(t.center[3 * sl + 2] - cz)) - tz;
   // a leaf with itself: the near-field kernel left out the pairs with FP32
   // r^2 <= rmin2 (their FP32 value is 0 here too)
   if (tl == sl) pair_grad<KIND, float, RSQ_MASK>(dx, dy, dz, 1.f, 0.f, kr, ki, a32, close_rmin2<float>(t, tl));
@@ -763,7 +869,7 @@ static void eval_targets_t(int mode, const DevTree& t, Wavek k, const int* tiles
   auto go = [&](auto W) {
     constexpr int w = decltype(W)::value;
     const dim3 g(ntiles), b(64 * w);
-    if (mode == MODE_P2P) hipLaunchKernelGGL((k_p2p_smem<KIND, R, w>), g, b, 0, s, t, k, tiles);
+    if (mode == MODE_P2P) hipLaunchKernelGGL((k_p2p<KIND, R, w>), g, b, 0, s, t, k, tiles);
     else if (mode == MODE_M2P) hipLaunchKernelGGL((k_m2p<KIND, R, (w < 4 ? 4 : w)>), g, dim3(64 * (w < 4 ? 4 : w)), 0, s, t, k, tiles);
     else hipLaunchKernelGGL((k_l2p_smem<KIND, R, w>), g, b, 0, s, t, k, tiles);
   };

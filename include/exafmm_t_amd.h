@@ -179,10 +179,11 @@ int xfmm_set_value_scale(xfmm_context* ctx, const double* scale);
  *   XFMM_TUNE_HAD_KCH    frequencies per Hadamard workgroup, 1..256 (default:
  *                        chosen from the size of the problem, at most 16; the
  *                        split-FP16 kernel rounds it up to an even number)
- *   XFMM_TUNE_P2P_SPLIT  P2P / M2P / L2P tail tiles of at most this many targets
- *                        (0..32) split each target's sources over
- *                        several lanes (default 32; the partial sums then add
- *                        in another order)
+ *   XFMM_TUNE_P2P_SPLIT  M2P / L2P tail tiles of at most this many targets
+ *                        (0..32) split each target's sources over several
+ *                        lanes; P2P tiles of more targets use two lanes a
+ *                        target at most (default 32; the partial sums then
+ *                        add in another order)
  *   XFMM_TUNE_HAD_GROUPS split-FP16 Hadamard (mixed / FLOAT): 128-target groups
  *                        per workgroup, 1 or 2 (4 is taken as 2), which share
  *                        the operators and the union of sources staged in LDS

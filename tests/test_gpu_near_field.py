@@ -2,12 +2,14 @@
 to thousands of tiles, full tiles, tails just below and above the source split, more than one tile per leaf, the
 three kernels.  FP64 within 1e-12 of the values' norm (the operators are applied to the same inputs; sums of at most
 some 1e4 terms in another order), FP32 within 1e-5."""
+import os
+
 import numpy as np
 import pytest
 
 import oracle as O
 from exafmm import abi
-from fmm_cases import make_problem, rel_err
+from fmm_cases import CACHE, KERNELS, charges, make_problem, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -103,3 +105,37 @@ def test_passes_read_as_zeroed(require_gpu, kernel, n, ncrit, dist):
         assert np.array_equal(b.values(), want) and np.array_equal(b.equiv()[1], dn)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("kernel,ncrit", [("laplace", 70), ("modified_helmholtz", 40), ("helmholtz", 64)])
+@pytest.mark.parametrize("precision", [abi.FP64, abi.FLOAT])
+def test_long_source_lists(require_gpu, kernel, ncrit, precision):
+    """P2P lists of more than 64 leaves (a large leaf beside a dense layer), leaves of 1 to 58 targets.  Tolerances as
+    above."""
+    mod, cls, kid, wavek = KERNELS[kernel]
+    rng = np.random.default_rng(3)
+    x = np.concatenate([rng.random((9000, 3)) * [0.04, 1, 1] + [0.46, 0, 0],
+                        rng.random((ncrit - 3, 3)) * 0.5 + [0.5, 0, 0], [[0, 0, 0], [1, 1, 1]]])
+    q = charges("centered", len(x), rng, kid == 1)
+    name = os.path.join(CACHE, "%s_long_%d.dat" % (kernel, ncrit))
+    fmm = getattr(mod, cls)(4, ncrit, **({} if wavek is None else {"wavek": wavek}), filename=name)
+    tree = mod.setup(mod.init_sources(x, q), mod.init_targets(x), fmm)
+    flat = fmm.flat_tree(tree)
+    count = np.diff(flat["p2p_offset"])
+    assert np.any((count > 64) & (flat["trg_count"] > 0))
+    wk = 0.0 if wavek is None else wavek
+    eng = abi.Engine(kid, 4, wk, precision)
+    eng.set_operators(fmm.operators())
+    eng.set_tree(flat)
+    eng.set_charges(fmm.sorted_charges(tree))
+    orc = O.Oracle(kid, 4, flat, fmm.operators(), wk)
+    orc.set_charges(fmm.sorted_charges(tree))
+    eng.clear()
+    orc.clear()
+    eng.op("P2P")
+    orc.run(O.STAGES["P2P"])
+    v, r = eng.values(), orc.val
+    tol = 1e-12 if precision == abi.FP64 else 1e-5
+    assert rel_err(v[:, 0], r[:, 0]) < tol
+    assert rel_err(v[:, 1:], r[:, 1:]) < tol
+    eng.close()
