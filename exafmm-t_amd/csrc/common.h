@@ -36,6 +36,37 @@ __device__ __forceinline__ double rsqrt_sep(double r2) {
 __device__ __forceinline__ float rsqrt_sep(float r2) { return __builtin_amdgcn_rsqf(r2); }
 __device__ __forceinline__ double dexp(double x) { return exp(x); }
 __device__ __forceinline__ void dsincos(double x, double* s, double* c) { sincos(x, s, c); }
+// sin and cos for |x| < 2^30 in FP64.  x = n pi/2 + r with pi/2 as the sum of its
+// rounding P1 and the rest P2 (Cody and Waite): the first fma is exact, the
+// second leaves an error of n 2^-107 + 2^-54 |r|; the Taylor series of sin r (to
+// r^17) and cos r (to r^16) are truncated at 1e-19 and 2e-18 for |r| <= pi/4.
+// The library's sincos keeps a path for huge arguments beside it, a branch and
+// registers (189 against 128 in the Helmholtz near field: half the waves).
+__device__ __forceinline__ void sincos_near(double x, double* s, double* c) {
+  const double n = __builtin_rint(x * 0.63661977236758134308);
+  const double r = fma(-n, 6.123233995736766036e-17, fma(-n, 1.57079632679489661923, x));
+  const double z = r * r;
+  double u = 1.0 / 355687428096000.0, v = 1.0 / 20922789888000.0;
+  u = fma(u, z, -1.0 / 1307674368000.0);
+  v = fma(v, z, -1.0 / 87178291200.0);
+  u = fma(u, z, 1.0 / 6227020800.0);
+  v = fma(v, z, 1.0 / 479001600.0);
+  u = fma(u, z, -1.0 / 39916800.0);
+  v = fma(v, z, -1.0 / 3628800.0);
+  u = fma(u, z, 1.0 / 362880.0);
+  v = fma(v, z, 1.0 / 40320.0);
+  u = fma(u, z, -1.0 / 5040.0);
+  v = fma(v, z, -1.0 / 720.0);
+  u = fma(u, z, 1.0 / 120.0);
+  v = fma(v, z, 1.0 / 24.0);
+  u = fma(u, z, -1.0 / 6.0);
+  v = fma(v, z, -0.5);
+  const double sn = fma(u * z, r, r), cs = fma(v, z, 1.0);
+  const int q = int(n);
+  const double a = q & 1 ? cs : sn, b = q & 1 ? sn : cs;
+  *s = q & 2 ? -a : a;
+  *c = (q + 1) & 2 ? -b : b;
+}
 // FP32 (mixed / FLOAT near field and surface evaluations): exp through the
 // hardware 2^x, sine and cosine on the hardware units, whose argument is in
 // revolutions, after reducing x / (2 pi) to [-1/2, 1/2].  The reductions

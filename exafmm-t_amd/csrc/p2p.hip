@@ -17,20 +17,27 @@
 // sources is summed in plain FP32 and tiles are combined with compensated
 // (Kahan) summation.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "kernels.h"
 
 namespace xfmm {
 
-// Helmholtz with a real wave number (Im k = 0): the evaluation kernels are
-// instantiated without the damping factor e^{-Im(k) r}, which is then exactly
-// 1 (the values are bit-identical to the general instantiation).  Internal to
-// the launchers of this file.
+// Helmholtz with a real wave number (Im k = 0) and phases k r < 2^30 in the
+// tree's box (real_phases): the evaluation kernels are instantiated without
+// the damping factor e^{-Im(k) r}, which is then exactly 1, and in FP64 with
+// sincos_near.  Internal to the launchers of this file.
 constexpr int HELMHOLTZ_REAL = 3;
 
 template <int KIND>
 constexpr bool kcplx() { return KIND == HELMHOLTZ || KIND == HELMHOLTZ_REAL; }
+
+template <int KIND, typename R>
+__device__ __forceinline__ void phase(R x, R* s, R* c) {
+  if constexpr (KIND == HELMHOLTZ_REAL && sizeof(R) == 8) sincos_near(x, s, c);
+  else dsincos(x, s, c);
+}
 
 // 1/r of a pair.  RSQ_LIB: library rsqrt, r = 0 gives 0 (the direct sum used as
 // accuracy check).  RSQ_MASK: hardware estimate refined to full precision
@@ -71,7 +78,7 @@ __device__ __forceinline__ void pair_grad(R dx, R dy, R dz, R qr, R qi, R kr, R 
     const R r = r2 * invr;
     const R e = KIND == HELMHOLTZ_REAL ? invr : dexp(-ki * r) * invr;
     R sn, cs;
-    dsincos(kr * r, &sn, &cs);
+    phase<KIND>(kr * r, &sn, &cs);
     const R gr = e * cs, gi = e * sn;
     const R pr = qr * gr - qi * gi;
     const R pim = qr * gi + qi * gr;
@@ -103,7 +110,7 @@ __device__ __forceinline__ void pair_pot(R dx, R dy, R dz, R qr, R qi, R kr, R k
     const R r = r2 * invr;
     const R e = KIND == HELMHOLTZ_REAL ? invr : dexp(-ki * r) * invr;
     R sn, cs;
-    dsincos(kr * r, &sn, &cs);
+    phase<KIND>(kr * r, &sn, &cs);
     const R gr = e * cs, gi = e * sn;
     a[0] += qr * gr - qi * gi;
     a[1] += qr * gi + qi * gr;
@@ -375,7 +382,7 @@ __global__ void k_pack_sources(int n, const double* __restrict__ rel, const doub
 // of cache reads a pair.  Before -> after: FP32, 32768 leaves of 30 targets 519
 // -> 465 us, of 61 1214 -> 1190; 38841 Plummer leaves of 15 478 -> 371; Yukawa FP32,
 // 15074 leaves of 20 220 -> 178; FP64, 12069 leaves of 41 1228 -> 1115; Helmholtz
-// FP64, 512 leaves of 59 268 -> 225.  128 sources a wave: 256 and 512 cost 2 and 20
+// FP64, 512 leaves of 59 268 -> 175 (225 with the library's sincos).  128 sources a wave: 256 and 512 cost 2 and 20
 // % (fewer workgroups on a CU); the next block loaded ahead gives nothing.
 // M = 1 for Helmholtz FP32, whose registers M = 2 halves the waves with (4096
 // leaves of 49: 312 and 327 us).
@@ -844,6 +851,11 @@ __global__ __launch_bounds__(256) void k_close_fix(DevTree t) {
 
 // ---------------------------------------------------------------- launchers
 
+// Points and surfaces of a tree are within 6 r0 of each other in a coordinate.
+static bool real_phases(Wavek k, const DevTree& t) {
+  return k.im == 0.0 && std::fabs(k.re) * 16.0 * t.r0 < 1073741824.0;
+}
+
 // Waves per tile: up to 4 while the tiles are fewer than 4 waves on each of the
 // chip's 1024 SIMDs (Helmholtz, whose pairs cost more: 16; near field of 4700 FP32
 // tiles with 1, 2, 4 waves 391, 349, 326 us), up to 16 for the few tiles of a
@@ -874,7 +886,15 @@ static void eval_targets_t(int mode, const DevTree& t, Wavek k, const int* tiles
     else hipLaunchKernelGGL((k_l2p_smem<KIND, R, w>), g, b, 0, s, t, k, tiles);
   };
   const int w = particle_waves<KIND>(ntiles);
-  if (w == 1) go(std::integral_constant<int, 1>());
+  // the FP64 near field of fewer than 1024 Helmholtz tiles, without the library's
+  // sincos: 8 waves (512 tiles: 193 us with 4, 175 with 8)
+  bool wide = false;
+  if constexpr (KIND == HELMHOLTZ_REAL && sizeof(R) == 8) {
+    wide = mode == MODE_P2P && ntiles < 1024;
+    if (wide) go(std::integral_constant<int, 8>());
+  }
+  if (wide) {
+  } else if (w == 1) go(std::integral_constant<int, 1>());
   else if (w == 2) go(std::integral_constant<int, 2>());
   else if (w == 4 || KIND != LAPLACE) go(std::integral_constant<int, 4>());
   else if constexpr (KIND == LAPLACE) {
@@ -897,7 +917,7 @@ void launch_eval_targets(int kind, bool f32, int mode, const DevTree& t, Wavek k
     case YUKAWA: f32 ? eval_targets_t<YUKAWA, float>(mode, t, k, tiles, ntiles, s)
                      : eval_targets_t<YUKAWA, double>(mode, t, k, tiles, ntiles, s); break;
     default:
-      if (k.im == 0.0) f32 ? eval_targets_t<HELMHOLTZ_REAL, float>(mode, t, k, tiles, ntiles, s)
+      if (real_phases(k, t)) f32 ? eval_targets_t<HELMHOLTZ_REAL, float>(mode, t, k, tiles, ntiles, s)
                            : eval_targets_t<HELMHOLTZ_REAL, double>(mode, t, k, tiles, ntiles, s);
       else f32 ? eval_targets_t<HELMHOLTZ, float>(mode, t, k, tiles, ntiles, s)
                : eval_targets_t<HELMHOLTZ, double>(mode, t, k, tiles, ntiles, s);
@@ -926,7 +946,7 @@ void launch_eval_surface(int kind, bool f32, int mode, const DevTree& t, Wavek k
     case YUKAWA: f32 ? eval_surface_t<YUKAWA, float>(mode, t, k, work, nwork, check, s)
                      : eval_surface_t<YUKAWA, double>(mode, t, k, work, nwork, check, s); break;
     default:
-      if (k.im == 0.0) f32 ? eval_surface_t<HELMHOLTZ_REAL, float>(mode, t, k, work, nwork, check, s)
+      if (real_phases(k, t)) f32 ? eval_surface_t<HELMHOLTZ_REAL, float>(mode, t, k, work, nwork, check, s)
                            : eval_surface_t<HELMHOLTZ_REAL, double>(mode, t, k, work, nwork, check, s);
       else f32 ? eval_surface_t<HELMHOLTZ, float>(mode, t, k, work, nwork, check, s)
                : eval_surface_t<HELMHOLTZ, double>(mode, t, k, work, nwork, check, s);

@@ -139,3 +139,26 @@ def test_long_source_lists(require_gpu, kernel, ncrit, precision):
     assert rel_err(v[:, 0], r[:, 0]) < tol
     assert rel_err(v[:, 1:], r[:, 1:]) < tol
     eng.close()
+
+
+@pytest.mark.parametrize("wavek", [0.5, 50.0, 3.0e4, 1.0e7, 1.0e10])
+def test_helmholtz_phases(require_gpu, wavek):
+    """Near field with phases k r from below 1 to beyond 2^30 (the library's reduction).  k r is rounded to 53 bits and
+    r to about 3 ulp on both sides: 8 k r 2^-53 rad a pair, times 8 for the cancellation of sums of 400 charges of
+    both signs."""
+    pr = make_problem("helmholtz", 400, 3, 64, "cube", seed=8, wavek=wavek)
+    eng = abi.Engine(pr["kid"], 3, wavek, abi.FP64)
+    eng.set_operators(pr["ops"])
+    eng.set_tree(pr["flat"])
+    eng.set_charges(pr["qs"])
+    orc = O.Oracle(pr["kid"], 3, pr["flat"], pr["ops"], wavek)
+    orc.set_charges(pr["qs"])
+    eng.clear()
+    orc.clear()
+    eng.op("P2P")
+    orc.run(O.STAGES["P2P"])
+    v, r = eng.values(), orc.val
+    tol = 1e-13 + 64 * wavek * np.sqrt(3.0) * 2.0 ** -53
+    assert rel_err(v[:, 0], r[:, 0]) < tol
+    assert rel_err(v[:, 1:], r[:, 1:]) < tol
+    eng.close()
