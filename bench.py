@@ -445,7 +445,7 @@ def roofline(dom, ms, mixed, h16, npairs, m2l_pairs, nfreq, nsrc, ntrg):
     rb = 4 if mixed else 8
     if dom == "P2P":
         flops = P2P_FLOP_PER_PAIR * npairs
-        roof = {"kernel": "P2P near field (k_p2p_smem, %s)" % ("FP32" if mixed else "FP64"),
+        roof = {"kernel": "P2P near field (k_p2p, %s)" % ("FP32" if mixed else "FP64"),
                 "bound": "valu", "achieved": flops / t / 1e12,
                 "peak": (PEAK["fp32_vector"] if mixed else PEAK["fp64_vector"]) / 1e12, "unit": "TFLOP/s",
                 "traffic": None, "algorithmic": "%d pairs x %d flop" % (npairs, P2P_FLOP_PER_PAIR)}

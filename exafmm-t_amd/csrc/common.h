@@ -42,7 +42,7 @@ __device__ __forceinline__ void dsincos(double x, double* s, double* c) { sincos
 // (to r^16) are truncated at 1e-19 and 2e-18 for |r| <= pi/4, and what rounds r
 // and 1 - r^2/2 is added back (largest error over phases up to 1e9: 8.4e-17, the library's 8.7e-17).
 // The library's sincos keeps a path for huge arguments beside it, a branch and
-// registers (189 against 128 in the Helmholtz near field: half the waves).
+// registers (189 against 122 in the Helmholtz near field: half the waves).
 __device__ __forceinline__ void sincos_near(double x, double* s, double* c) {
   const double n = __builtin_rint(x * 0.63661977236758134308);
   const double h = fma(-n, 1.57079632679489661923, x);

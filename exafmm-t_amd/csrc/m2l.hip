@@ -12,14 +12,14 @@
 //     (unnormalised; 1/n^3 is folded into M) and gather through surf2conv_dn
 //     into the children's downward check potentials, times ifft_scale.
 //
-// GPU structure.  Transforms: one workgroup per (node, child); the input is
-// nonzero only on the [0,p)^3 corner and only the [p,2p)^3 corner of the
-// output is needed, so each 1-D pass is a small dense DFT restricted to those
-// index ranges, evaluated from LDS with a twiddle table.  Hadamard: a
-// workgroup owns 64 target parents (consecutive in Hilbert order, so their
-// sources overlap in L2) and 16 frequencies; each wave takes 4 frequencies,
-// lanes are targets, the 8x8 matrix M[r][k] is wave-uniform (scalar loads)
-// and the 26 relative positions are accumulated in registers.
+// GPU structure.  Transforms: the input is nonzero only on the [0,p)^3 corner
+// and only the [p,2p)^3 corner of the output is needed, so each 1-D pass is a
+// small dense DFT restricted to those index ranges: one workgroup per node, y
+// and z on the matrix units, x on the vector units (per child with a twiddle
+// table where a node's grid does not fit the LDS).  Hadamard: a workgroup owns
+// 64 (FP64) or 128 / 256 (split FP16) target parents, consecutive in Hilbert
+// order, and a chunk of frequencies; per frequency the union of their sources
+// and the 26 operators are staged in LDS and multiplied as real 16 x 16 tiles.
 #include <type_traits>
 
 #include "kernels.h"

@@ -375,20 +375,25 @@ __global__ void k_pack_sources(int n, const double* __restrict__ rel, const doub
 // block each, the k lane groups every k-th source of it, two of them per trip,
 // and the sums are added in FP64 in a fixed order.  A tile of more than
 // t.p2p_split targets uses two lane groups at most.
-// Bound by the vector units: 17 instructions (Laplace) a pair, 1/sqrt at a
-// quarter rate.  Per source leaf and tile instead (full tiles with a target per
+// Bound by the vector units: 14 instructions a pair (Laplace FP32).  Per source
+// leaf and tile instead (full tiles with a target per
 // lane and scalar loads, others with the lane groups reading each leaf from the
 // vector cache) the small leaves paid for remainders and for 16 lanes' worth
 // of cache reads a pair.  Before -> after: FP32, 32768 leaves of 30 targets 519
 // -> 465 us, of 61 1214 -> 1190; 38841 Plummer leaves of 15 478 -> 371; Yukawa FP32,
 // 15074 leaves of 20 220 -> 178; FP64, 12069 leaves of 41 1228 -> 1115; Helmholtz
-// FP64, 512 leaves of 59 268 -> 175 (225 with the library's sincos).  128 sources a wave: 256 and 512 cost 2 and 20
+// FP64, 512 leaves of 59 268 -> 196 (223 with the library's sincos).  128 sources a wave: 256 and 512 cost 2 and 20
 // % (fewer workgroups on a CU); the next block loaded ahead gives nothing.
-// M = 1 for Helmholtz FP32, whose registers M = 2 halves the waves with (4096
-// leaves of 49: 312 and 327 us).
+// M = 1 for Helmholtz where M = 2 costs waves by its registers (FP32, 4096 leaves
+// of 49: 312 and 327 us; FP64 with sincos_near, 122 and 138 registers: 196 and 207),
+// but not in FP64 with the library's sincos, whose branch wants pairs to overlap
+// (425 and 223).
+template <int KIND, typename R>
+constexpr int points_per_lane() { return kcplx<KIND>() && (sizeof(R) == 4 || KIND == HELMHOLTZ_REAL) ? 1 : 2; }
+
 template <int KIND, typename R, int W>
 __global__ __launch_bounds__(64 * W) void k_p2p(DevTree t, Wavek wk, const int* __restrict__ work) {
-  constexpr int NA = nval<KIND>(), NP = npack<KIND>(), M = kcplx<KIND>() && sizeof(R) == 4 ? 1 : 2;
+  constexpr int NA = nval<KIND>(), NP = npack<KIND>(), M = points_per_lane<KIND, R>();
   constexpr int CAP = 128 * W;  // sources in LDS
   constexpr int NE = 64;        // source leaves listed at a time
   constexpr int SZ = std::max(int(CAP * NP * sizeof(R)), int(W * NA * 64 * sizeof(double)));
@@ -887,7 +892,7 @@ static void eval_targets_t(int mode, const DevTree& t, Wavek k, const int* tiles
   };
   const int w = particle_waves<KIND>(ntiles);
   // the FP64 near field of fewer than 1024 Helmholtz tiles, without the library's
-  // sincos: 8 waves (512 tiles: 193 us with 4, 175 with 8)
+  // sincos: 8 waves (512 tiles, before the error terms of sincos_near: 193 us with 4, 175 with 8)
   bool wide = false;
   if constexpr (KIND == HELMHOLTZ_REAL && sizeof(R) == 8) {
     wide = mode == MODE_P2P && ntiles < 1024;
