@@ -153,7 +153,8 @@ struct xfmm_context {
   bool p2p_all = false, l2p_all = false;                  // the P2P / L2P tiles hold every target exactly once
   // M2L
   int n_m2l_src = 0, n_m2l_trg = 0, n_m2l_blk = 0;
-  DevBuf<int> m2l_src_node, m2l_trg_node, m2l_blk_trg, m2l_blk_uni, m2l_blk_nu, m2l_blk_lev;
+  DevBuf<int> m2l_src_node, m2l_trg_node, m2l_blk_trg, m2l_blk_uni, m2l_blk_nu, m2l_blk_lev,
+      m2l_blk_lev0;
   DevBuf<short> m2l_blk_loc;
   DevBuf<double> m2l_scale;
   // host side of the Hadamard blocks, rebuilt when their size changes
@@ -648,6 +649,8 @@ void build_had_blocks(xfmm_context* c) {
   c->m2l_blk_uni.upload(buni, c->stream);
   c->m2l_blk_nu.upload(bnu, c->stream);
   c->m2l_blk_lev.upload(blev, c->stream);
+  const std::vector<int> lev0(blev.size(), 0);
+  c->m2l_blk_lev0.upload(lev0, c->stream);
   c->m2l_blk_loc.upload(bloc, c->stream);
   HIPCHK(hipStreamSynchronize(c->stream));
   c->had_ntrg = T;
@@ -661,7 +664,8 @@ void run_hadamards(xfmm_context* c, const M2LDev& m) {
   hb.trg = c->m2l_blk_trg.ptr;
   hb.uni = c->m2l_blk_uni.ptr;
   hb.nunion = c->m2l_blk_nu.ptr;
-  hb.oplev = c->m2l_blk_lev.ptr;
+  // one operator set serves every level (as op_level for the translations)
+  hb.oplev = c->nm2l == 1 ? c->m2l_blk_lev0.ptr : c->m2l_blk_lev.ptr;
   hb.loc = c->m2l_blk_loc.ptr;
   const void* ops = c->f32_m2l ? static_cast<const void*>(c->m2l32.ptr) : static_cast<const void*>(c->m2l64.ptr);
   launch_hadamard(m, ops, c->f16_had ? c->m2l_hscale.ptr : nullptr, hb, c->tune_kch, had_tiles(c), c->stream);

@@ -118,7 +118,10 @@ int xfmm_sizes(const xfmm_context* ctx, int* nsurf, int* nconv, int* nfreq);
  *   m2m, l2l                       : T[nlevels][8][nsurf][nsurf]
  *   m2l                            : double[nm2l][26][nfreq][8*8][2]
  *     (layout of matrix_M2L, fmm_scale_invariant.h:545-552); nm2l = 1 for
- *     Laplace, depth for the others (slot l serves target level l). */
+ *     Laplace, depth for the others (slot l serves target level l).
+ * A single slot (nlevels = 1, nm2l = 1) serves every level; any other count
+ * below depth + 1 (nlevels) or depth (nm2l) is refused by the passes and
+ * operators (XFMM_ERR_ARG). */
 int xfmm_set_operators(xfmm_context* ctx, int nlevels, const double* uc2e_u, const double* uc2e_v,
                        const double* dc2e_u, const double* dc2e_v, const double* m2m, const double* l2l,
                        int nm2l, const double* m2l);
