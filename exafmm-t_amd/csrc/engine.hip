@@ -170,8 +170,8 @@ struct xfmm_context {
   DevBuf<double> close_coef;
   DevBuf<double> charge_sums;  // partial sums of the charge balance rule (device charges)
   int nclose = 0;  // targets with near-coincident pairs
-  DevBuf<double> src_rel, src_pack, surf_tab;
-  DevBuf<float> surf_tab32;  // P2P sources relative to their leaf centre; packed (x, y, z, q)
+  DevBuf<double> surf_tab;
+  DevBuf<float> surf_tab32;
 
   // per-target output factors (phi, gradient) applied at the end of each
   // downward pass (xfmm_set_value_scale); empty = none
@@ -216,11 +216,8 @@ struct xfmm_context {
     t.p2l_off = p2l_off.ptr;
     t.p2l_src = p2l_src.ptr;
     t.unit_surf = unit_surf.ptr;
-    t.nsrcs = nsrcs;
-    t.src_rel = src_rel.ptr;
     t.surf_tab = surf_tab.ptr;
     t.surf_tab32 = surf_tab32.ptr;
-    t.src_pack = src_pack.ptr;
     t.up = up.ptr;
     t.dn = dn.ptr;
     t.trg_value = trg_value.ptr;
@@ -1029,14 +1026,6 @@ int xfmm_set_tree(xfmm_context* c, const xfmm_tree* t) {
     c->trg_count.upload(t->trg_count, nn, st);
     c->src.upload(t->src_coord, size_t(t->nsrcs) * 3, st);
     {
-      std::vector<double> rel(size_t(t->nsrcs) * 3);
-      for (int i = 0; i < nn; i++) {
-        if (ch[i] >= 0) continue;
-        for (int k = t->src_begin[i]; k < t->src_begin[i] + t->src_count[i]; k++)
-          for (int d = 0; d < 3; d++) rel[3 * size_t(k) + d] = t->src_coord[3 * size_t(k) + d] - t->center[3 * i + d];
-      }
-      c->src_rel.upload(rel, st);
-      c->src_pack.alloc(std::max<size_t>(1, size_t(t->nsrcs) * (c->cplx ? 5 : 4)));
       // L2P equivalent surface per level, relative to the box centre
       const std::vector<double> us = unit_surface(c->p);
       std::vector<double> tab(size_t(D + 1) * c->nsurf * 4, 0.0);

@@ -10,7 +10,7 @@ namespace xfmm {
 // kind T are doubles (real kernels) or interleaved (re, im) doubles
 // (Helmholtz); `vw` is the number of doubles per value (1 or 2).
 struct DevTree {
-  int nnodes = 0, depth = 0, p = 0, nsurf = 0, vw = 1, nsrcs = 0;
+  int nnodes = 0, depth = 0, p = 0, nsurf = 0, vw = 1;
   double r0 = 0;
   const double* center = nullptr;  // [nnodes][3]
   const int* level = nullptr;      // [nnodes]
@@ -29,10 +29,8 @@ struct DevTree {
   const int* p2l_off = nullptr;
   const int* p2l_src = nullptr;
   const double* unit_surf = nullptr;  // [nsurf][3] unit-cube surface (reference point order)
-  const double* src_rel = nullptr;    // [nsrcs][3] source positions relative to their leaf centre
   const double* surf_tab = nullptr;   // [depth + 1][nsurf][4] L2P equivalent surface (radius 2.95 r_l), (x, y, z, 0) relative to the centre
   const float* surf_tab32 = nullptr;  // the same in FP32 (FP32 L2P)
-  void* src_pack = nullptr;           // [nsrcs] (x, y, z, q[, Im q]) relative to the leaf centre, in the P2P type
   double* up = nullptr;               // T[nnodes][nsurf]
   double* dn = nullptr;               // T[nnodes][nsurf]
   double* trg_value = nullptr;        // T[ntrgs][4]

@@ -346,35 +346,23 @@ __device__ __forceinline__ void sum_split(int n, const Tile<R>& T, SRC src, R ux
   }
 }
 
-// Near field (fmm_base.h:82-94).  Each source is packed once per evaluation as
-// (x, y, z, q[, Im q]) relative to its leaf centre.
+// Values of a source in LDS: position, charge.
 template <int KIND>
 constexpr int npack() { return kcplx<KIND>() ? 5 : 4; }
-
-template <typename R, int NP>
-__global__ void k_pack_sources(int n, const double* __restrict__ rel, const double* __restrict__ q,
-                               R* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  R v[NP];
-#pragma unroll
-  for (int d = 0; d < 3; d++) v[d] = R(rel[3 * size_t(i) + d]);
-#pragma unroll
-  for (int d = 3; d < NP; d++) v[d] = R(q[size_t(i) * (NP - 3) + d - 3]);
-#pragma unroll
-  for (int d = 0; d < NP; d++) out[size_t(i) * NP + d] = v[d];
-}
 
 // A workgroup of W waves per (leaf, tile of TILE targets).  A lane holds M targets
 // (target l + u L of the tile in lane l, L = ceil(nt / M)), so that k = 64 / L
 // lanes share a target's sources and few lanes are left over: leaves of 24
 // targets use 60 of 64 lanes (48 with one target in a lane).  The sources of
 // all leaves of the list are one sequence, moved into the target leaf's frame
-// (the offset of the centres formed in FP64) on their way to LDS, padded with
-// zero charges to whole trips of the loop; the W waves take a part of every
-// block each, the k lane groups every k-th source of it, two of them per trip,
+// on their way to LDS (subtracted in FP64, rounded once), padded with zero
+// charges to whole trips of the loop; the W waves take a part of every block each, the k lane groups every k-th source of it, two of them per trip,
 // and the sums are added in FP64 in a fixed order.  A tile of more than
 // t.p2p_split targets uses two lane groups at most.
+// Sources packed beforehand relative to their own leaf (half the bytes in FP32)
+// and shifted here cost FP32 two more roundings per coordinate, 5 to 7 times the
+// error of a pair across a leaf plane, and were no faster (2M points 1.18 ms
+// either way; Helmholtz FP32, 4096 leaves of 49, 312 and 305 us).
 // Bound by the vector units: 14 instructions a pair (Laplace FP32).  Per source
 // leaf and tile instead (full tiles with a target per
 // lane and scalar loads, others with the lane groups reading each leaf from the
@@ -399,7 +387,6 @@ __global__ __launch_bounds__(64 * W) void k_p2p(DevTree t, Wavek wk, const int* 
   constexpr int SZ = std::max(int(CAP * NP * sizeof(R)), int(W * NA * 64 * sizeof(double)));
   __shared__ __attribute__((aligned(16))) char smem[SZ];
   __shared__ int pre[NE + 1], first[NE], self;
-  __shared__ R off[3][NE];
   R* sp = reinterpret_cast<R*>(smem);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int leaf = work[2 * blockIdx.x], t0 = TILE * work[2 * blockIdx.x + 1];
@@ -420,7 +407,16 @@ __global__ __launch_bounds__(64 * W) void k_p2p(DevTree t, Wavek wk, const int* 
     for (int a = 0; a < NA; a++) { acc[u][a] = 0; comp[u][a] = 0; }
   }
   const int unit = 2 * W * k, most = min(CAP / unit * unit, TILE * W * k);  // at most TILE sources a lane and block
-  const R* pack = static_cast<const R*>(t.src_pack);
+  // source i of the tree in the target leaf's frame
+  auto get = [&](int i, R* v) {
+    const double* p = t.src + 3 * size_t(i);
+    const double* q = t.q + size_t(i) * (NP - 3);
+    v[0] = R(p[0] - cx);
+    v[1] = R(p[1] - cy);
+    v[2] = R(p[2] - cz);
+#pragma unroll
+    for (int d = 3; d < NP; d++) v[d] = R(q[d - 3]);
+  };
   // all pairs of total sources, source i read by load(i, v)
   auto sums = [&](auto RM, int total, auto load) {
     for (int s0 = 0; s0 < total; s0 += most) {
@@ -461,9 +457,6 @@ __global__ __launch_bounds__(64 * W) void k_p2p(DevTree t, Wavek wk, const int* 
         if (s == leaf) self = 1;
         else n = t.src_count[s];
         first[tid] = t.src_begin[s];
-        off[0][tid] = R(t.center[3 * s] - cx);
-        off[1][tid] = R(t.center[3 * s + 1] - cy);
-        off[2][tid] = R(t.center[3 * s + 2] - cz);
       }
 #pragma unroll
       for (int d = 1; d < 64; d *= 2) {
@@ -479,21 +472,14 @@ __global__ __launch_bounds__(64 * W) void k_p2p(DevTree t, Wavek wk, const int* 
 #pragma unroll
       for (int d = NE / 2; d > 0; d /= 2)
         if (pre[e + d] <= i) e += d;
-      const R* p = pack + size_t(NP) * (first[e] + i - pre[e]);
-#pragma unroll
-      for (int d = 0; d < NP; d++) v[d] = p[d];
-#pragma unroll
-      for (int d = 0; d < 3; d++) v[d] += off[d][e];
+      get(first[e] + i - pre[e], v);
     });
   }
   __syncthreads();
   // only a leaf with itself can pair coinciding points
   if (self)
-    sums(std::integral_constant<int, RSQ_MASK>(), t.src_count[leaf], [&](int i, R* v) {
-      const R* p = pack + size_t(NP) * (t.src_begin[leaf] + i);
-#pragma unroll
-      for (int d = 0; d < NP; d++) v[d] = p[d];
-    });
+    sums(std::integral_constant<int, RSQ_MASK>(), t.src_count[leaf],
+         [&](int i, R* v) { get(t.src_begin[leaf] + i, v); });
   double* red = reinterpret_cast<double*>(smem);
 #pragma unroll
   for (int u = 0; u < M; u++) {
@@ -772,9 +758,8 @@ void launch_close_find(const DevTree& t, const int* work, int nwork, int* out, i
 // The correction of each listed pair per unit charge, once per tree: one
 // thread per pair, coef[k][a] = FP64 minus FP32 value of the pair with q = 1
 // (real kernels: a = potential, gradient; Helmholtz: their (re, im) parts).
-// The FP32 operands are formed as the near-field kernel forms them: the source
-// relative to its leaf centre as k_pack_sources rounds it and the target moved
-// into the source leaf's frame.  A pair is
+// The FP32 operands are formed as the near-field kernel forms them: source and
+// target relative to the target leaf's centre, each rounded once.  A pair is
 // linear in its charge, so per evaluation its correction is q coef (complex
 // product for Helmholtz); the FP32 value of a charged pair differs from q
 // times that of a unit charge by the rounding of the products, ~1e-7 of the
@@ -799,11 +784,7 @@ __global__ __launch_bounds__(256) void k_close_coef(DevTree t, Wavek wk, int npa
     a32[a] = 0.f;
     a64[a] = 0.0;
   }
-  float dx, dy, dz;
-  const double* rel = t.src_rel + 3 * size_t(is);
-  dx = (float(rel[0]) + float(t.center[3 * sl] - cx)) - tx;
-  dy = (float(rel[1]) + float(t.center[3 * sl + 1] - cy)) - ty;
-  dz = (float(rel[2]) + float(t.center[3 * sl + 2] - cz)) - tz;
+  const float dx = float(y[0] - cx) - tx, dy = float(y[1] - cy) - ty, dz = float(y[2] - cz) - tz;
   // a leaf with itself: the near-field kernel left out the pairs with FP32
   // r^2 <= rmin2 (their FP32 value is 0 here too)
   if (tl == sl) pair_grad<KIND, float, RSQ_MASK>(dx, dy, dz, 1.f, 0.f, kr, ki, a32, close_rmin2<float>(t, tl));
@@ -880,9 +861,6 @@ static int particle_waves(int ntiles) {
 template <int KIND, typename R>
 static void eval_targets_t(int mode, const DevTree& t, Wavek k, const int* tiles, int ntiles, hipStream_t s) {
   if (ntiles <= 0) return;
-  if (mode == MODE_P2P && t.nsrcs > 0)
-    hipLaunchKernelGGL((k_pack_sources<R, npack<KIND>()>), dim3((t.nsrcs + 255) / 256), dim3(256), 0, s, t.nsrcs,
-                       t.src_rel, t.q, static_cast<R*>(t.src_pack));
   auto go = [&](auto W) {
     constexpr int w = decltype(W)::value;
     const dim3 g(ntiles), b(64 * w);
