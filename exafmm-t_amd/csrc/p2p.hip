@@ -44,9 +44,16 @@ __device__ __forceinline__ void phase(R x, R* s, R* c) {
 // (rsqrt_sep), r^2 <= rmin2 gives 0 (a leaf with itself, where a target may
 // coincide with a source; the FP32 near field also leaves out the
 // near-coincident pairs that k_close_fix adds in FP64).  RSQ_SEP: rsqrt_sep
-// without the test (pairs that cannot coincide: distinct leaves own distinct
-// points, and surfaces never touch particles).
-enum RsqMode { RSQ_LIB = 0, RSQ_MASK = 1, RSQ_SEP = 2 };
+// without the test (surfaces never touch particles).  RSQ_SOFT: rsqrt_sep(r^2 +
+// rmin2) for two leaves, whose points are distinct but can be rounded to the same
+// numbers in the target leaf's frame (soft_r2; the sum starts from rmin2, so
+// it costs no instruction).
+enum RsqMode { RSQ_LIB = 0, RSQ_MASK = 1, RSQ_SEP = 2, RSQ_SOFT = 3 };
+template <int RM, typename R>
+__device__ __forceinline__ R dist2(R dx, R dy, R dz, R rmin2) {
+  if constexpr (RM == RSQ_SOFT) return fma(dz, dz, fma(dx, dx, fma(dy, dy, rmin2)));
+  else return dx * dx + dy * dy + dz * dz;
+}
 template <int RM, typename R>
 __device__ __forceinline__ R inv_r(R r2, R rmin2) {
   if constexpr (RM == RSQ_LIB) return rsqrt_pos(r2);
@@ -57,7 +64,7 @@ __device__ __forceinline__ R inv_r(R r2, R rmin2) {
 // potential + gradient of one pair, accumulated into a[] (4 or 8 values)
 template <int KIND, typename R, int RM>
 __device__ __forceinline__ void pair_grad(R dx, R dy, R dz, R qr, R qi, R kr, R ki, R* a, R rmin2 = R(0)) {
-  const R r2 = dx * dx + dy * dy + dz * dz;
+  const R r2 = dist2<RM>(dx, dy, dz, rmin2);
   const R invr = inv_r<RM>(r2, rmin2);
   if constexpr (KIND == LAPLACE) {
     const R qinv = qr * invr;
@@ -168,6 +175,23 @@ __device__ __forceinline__ R close_rmin2(const DevTree& t, int leaf) {
     }
   }
   return R(0);
+}
+
+// RSQ_SOFT's term for a target leaf.  Two points of different leaves closer than
+// a rounding of the leaf's size can get the same position in its frame: r^2 = 0,
+// 1/r infinite and a gradient of infinity times zero.  FP32: (2^-18 side)^2 keeps
+// their FP32 value finite, below their true value and, since such pairs are listed
+// (k_close_find), corrected to it in FP64; it changes 1/r of an unlisted pair (r >=
+// side / 16) by less than 2^-29.  FP64: (2^-54 side)^2, of the size of the
+// distances that the frame resolves.
+template <typename R>
+__device__ __forceinline__ R soft_r2(const DevTree& t, int leaf) {
+  const double e = 2.0 * t.r0 * ldexp(1.0, -t.level[leaf] - (sizeof(R) == 4 ? 18 : 54)), e2 = e * e;
+  if constexpr (sizeof(R) == 4) return R(e2);
+  // one value for all lanes: FP64 keeps it in scalar registers (W = 16 would take
+  // 122 vector registers, with them 120)
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(e2)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(e2)));
 }
 
 // ---------------------------------------------- particle targets: P2P, M2P, L2P
@@ -395,7 +419,7 @@ __global__ __launch_bounds__(64 * W) void k_p2p(DevTree t, Wavek wk, const int* 
   const int l = lane % L, ph = lane / L < k ? lane / L : 0;
   const double cx = t.center[3 * leaf], cy = t.center[3 * leaf + 1], cz = t.center[3 * leaf + 2];
   const R far = R(4.0 * t.r0 * ldexp(1.0, -t.level[leaf]));
-  const R kr = R(wk.re), ki = R(wk.im), rmin2 = close_rmin2<R>(t, leaf);
+  const R kr = R(wk.re), ki = R(wk.im), rmin2 = close_rmin2<R>(t, leaf), soft = soft_r2<R>(t, leaf);
   R x[M][3], acc[M][NA], comp[M][NA];
 #pragma unroll
   for (int u = 0; u < M; u++) {
@@ -439,7 +463,7 @@ __global__ __launch_bounds__(64 * W) void k_p2p(DevTree t, Wavek wk, const int* 
 #pragma unroll
           for (int u = 0; u < M; u++)
             pair_grad<KIND, R, decltype(RM)::value>(w[0] - x[u][0], w[1] - x[u][1], w[2] - x[u][2], w[3], w[4], kr, ki,
-                                                    part[u], rmin2);
+                                                    part[u], RM == RSQ_MASK ? rmin2 : soft);
         }
       }
 #pragma unroll
@@ -467,7 +491,7 @@ __global__ __launch_bounds__(64 * W) void k_p2p(DevTree t, Wavek wk, const int* 
       if (tid == 0) pre[0] = 0;
     }
     __syncthreads();
-    sums(std::integral_constant<int, RSQ_SEP>(), pre[NE], [&](int i, R* v) {
+    sums(std::integral_constant<int, RSQ_SOFT>(), pre[NE], [&](int i, R* v) {
       int e = 0;  // the last leaf with pre[e] <= i
 #pragma unroll
       for (int d = NE / 2; d > 0; d /= 2)
@@ -788,7 +812,7 @@ __global__ __launch_bounds__(256) void k_close_coef(DevTree t, Wavek wk, int npa
   // a leaf with itself: the near-field kernel left out the pairs with FP32
   // r^2 <= rmin2 (their FP32 value is 0 here too)
   if (tl == sl) pair_grad<KIND, float, RSQ_MASK>(dx, dy, dz, 1.f, 0.f, kr, ki, a32, close_rmin2<float>(t, tl));
-  else pair_grad<KIND, float, RSQ_SEP>(dx, dy, dz, 1.f, 0.f, kr, ki, a32);
+  else pair_grad<KIND, float, RSQ_SOFT>(dx, dy, dz, 1.f, 0.f, kr, ki, a32, soft_r2<float>(t, tl));
   pair_grad<KIND, double, RSQ_MASK>(y[0] - x[0], y[1] - x[1], y[2] - x[2], 1.0, 0.0, wk.re, wk.im, a64);
 #pragma unroll
   for (int a = 0; a < NA; a++) coef[size_t(k) * NA + a] = a64[a] - double(a32[a]);
