@@ -20,8 +20,11 @@ namespace {
 
 thread_local std::string g_thread_error;
 
+// A failed HIP call.  Its code stays behind as the thread's last error, which the
+// next call that asks for it would report as its own: taken back here.
 struct HipError {
   std::string msg;
+  explicit HipError(std::string m) : msg(std::move(m)) { (void)hipGetLastError(); }
 };
 
 #define HIPCHK(expr)                                                                 \
@@ -345,6 +348,7 @@ void check_ready(xfmm_context* c) {
   if (c->nlevels != 1 && c->nlevels < c->depth + 1)
     throw ArgError{"xfmm: level-dependent operators cover fewer levels than the tree depth"};
   if (c->nm2l != 1 && c->nm2l < c->depth) throw ArgError{"xfmm: M2L operators cover fewer levels than the tree depth"};
+  if (c->had_ntrg == 0) throw ArgError{"xfmm: M2L blocks not built (an allocation failed; set the tree or the tuning again)"};
 }
 
 // Entries between the packed operators of two levels: pseudo-inverse factors
@@ -563,6 +567,7 @@ int had_block_targets(const xfmm_context* c) { return c->f16_had ? 128 * had_gro
 void build_had_blocks(xfmm_context* c) {
   const int T = had_block_targets(c), ucap = had_ucap(T), urows = had_urows(T);
   if (c->had_ntrg == T) return;
+  c->had_ntrg = 0;  // until all of the new blocks are there
   const int ntrg = int(c->h_m2l_trg.size());
   std::vector<int> btrg, buni, bnu, blev;
   std::vector<short> bloc;
@@ -861,6 +866,7 @@ int xfmm_set_operators(xfmm_context* c, int nlevels, const double* uc2e_u, const
     drop_graph(c);
     require(uc2e_u && uc2e_v && dc2e_u && dc2e_v && m2m && l2l && m2l, "xfmm_set_operators: null operator");
     if (c->kind == XFMM_LAPLACE) require(nlevels == 1 && nm2l == 1, "xfmm_set_operators: Laplace operators are scale invariant (nlevels = nm2l = 1)");
+    c->have_ops = false;  // until all of them are there: a call that fails leaves none to run on
     const int ns = c->nsurf, vw = c->vw;
     const size_t ns2 = size_t(ns) * ns;
     // Rank of C2E_V = V S^+ per level: 1 + its last column that is not
@@ -1490,6 +1496,7 @@ int xfmm_set_tuning(xfmm_context* c, int param, int value) {
     } else if (param == XFMM_TUNE_HAD_GROUPS) {
       require(value == 1 || value == 2 || value == 4, "xfmm_set_tuning: Hadamard groups must be 1, 2 or 4");
       c->tune_groups = value;
+      drop_graph(c);
       if (c->have_tree) build_had_blocks(c);
     } else if (param == XFMM_TUNE_HAD_TILES) {
       require(value == 1 || value == 2, "xfmm_set_tuning: Hadamard tiles per wave must be 1 or 2");

@@ -59,3 +59,26 @@ def test_too_few_levels_refused(require_gpu, kernel):
         with pytest.raises(abi.XfmmError, match="fewer levels"):
             eng.op("M2L")
     eng.close()
+
+
+@pytest.mark.parametrize("precision", [abi.FP64, abi.MIXED])
+def test_failed_upload_leaves_no_operators(require_gpu, precision):
+    """A set of operators whose upload fails part of the way (an M2L of more bytes than there is memory) replaces
+    some of the earlier ones: the passes refuse to run on the mixture until a whole set is there."""
+    pr = make_problem("modified_helmholtz", 6000, 4, 40, "cube", seed=15)
+    eng = abi.Engine(pr["kid"], 4, pr["wavek"], precision)
+    eng.set_operators(pr["ops"])
+    eng.set_tree(pr["flat"])
+    eng.set_charges(pr["qs"])
+    eng.upward_pass()
+    eng.downward_pass()
+    want = eng.values()
+    with pytest.raises(abi.XfmmError):
+        eng.set_operators(dict(pr["ops"], nm2l=2 ** 30))
+    with pytest.raises(abi.XfmmError, match="operators not set"):
+        eng.upward_pass()
+    eng.set_operators(pr["ops"])
+    eng.upward_pass()
+    eng.downward_pass()
+    assert np.array_equal(eng.values(), want)
+    eng.close()
