@@ -181,7 +181,7 @@ struct xfmm_context {
   DevBuf<double> vscale;
   // tuning (xfmm_set_tuning / xfmm_autotune)
   int tune_kch = 0;        // Hadamard frequencies per workgroup (0: chosen from the grid)
-  // split-FP16 Hadamard: 128-target groups per workgroup (1 or 2) and 16-target
+  // split-FP16 Hadamard: 64-target groups per workgroup (1, 2 or 4) and 16-target
   // tiles per wave; 0: chosen from the number of targets
   int tune_groups = 0, tune_tiles = 0;
   int tune_split = 32;     // P2P / M2P / L2P: largest tail tile whose sources are split over lanes
@@ -550,15 +550,15 @@ void launch_near(xfmm_context* c) {
 // targets, two tiles per wave from 1024 targets on (1720 targets at p = 10
 // 1.73 ms, one tile 1.96; 584 targets at p = 8 451 and 384 us).
 int had_groups(const xfmm_context* c) {
-  if (c->tune_groups > 0) return std::min(c->tune_groups, 2);
-  return c->h_m2l_trg.size() >= 1024 ? 2 : 1;
+  if (c->tune_groups > 0) return c->tune_groups;
+  return c->h_m2l_trg.size() >= 1024 ? 4 : 2;
 }
 int had_tiles(const xfmm_context* c) {
   if (c->tune_tiles > 0) return c->tune_tiles;
-  if (c->f16_had) return had_groups(c) == 2 ? 2 : 1;
+  if (c->f16_had) return had_groups(c) == 4 ? 2 : 1;
   return c->h_m2l_trg.size() >= 1024 ? 2 : 1;
 }
-int had_block_targets(const xfmm_context* c) { return c->f16_had ? 128 * had_groups(c) : 64; }
+int had_block_targets(const xfmm_context* c) { return c->f16_had ? 64 * had_groups(c) : 64; }
 
 // Hadamard blocks of the uploaded tree (layout at HadBlocks): consecutive
 // targets of one operator level (all levels of a scale-invariant kernel), in
@@ -1510,7 +1510,9 @@ int xfmm_set_tuning(xfmm_context* c, int param, int value) {
 
 int xfmm_get_tuning(const xfmm_context* c, int param, int* value) {
   if (!c || !value) return fail(nullptr, XFMM_ERR_ARG, "xfmm_get_tuning: null argument");
-  if (param == XFMM_TUNE_HAD_KCH) *value = c->tune_kch > 0 ? c->tune_kch : HAD_KCH;
+  if (param == XFMM_TUNE_HAD_KCH)
+    *value = c->have_tree ? had_frequencies(c->nfreq, c->n_m2l_blk, c->tune_kch, c->f16_had)
+                          : c->tune_kch > 0 ? c->tune_kch : HAD_KCH;
   else if (param == XFMM_TUNE_P2P_SPLIT) *value = c->tune_split;
   else if (param == XFMM_TUNE_HAD_GROUPS) *value = had_groups(c);
   else if (param == XFMM_TUNE_HAD_TILES) *value = had_tiles(c);
@@ -1584,15 +1586,16 @@ int xfmm_autotune(xfmm_context* c, int reps, double* best_ms) {
       if (m.amax) launch_zero(c->m2l_amax.ptr, 1, c->stream);
       launch_fft_up(m, t, c->m2l_src_node.ptr, c->n_m2l_src, c->stream);
       const int cand[] = {4, 8, 16, 32, 64};
-      // groups and tiles per wave matter only for the split-FP16 kernel
-      const int ngr = (c->f16_had && m.amax) ? 4 : 1;
+      // groups and tiles per wave matter only for the split-FP16 kernel: the
+      // two sizes of block around the default (had_groups)
+      const int ngr = (c->f16_had && m.amax) ? 4 : 1, most = c->h_m2l_trg.size() >= 1024 ? 4 : 2;
       int best = c->tune_kch, bestg = c->tune_groups, bestt = c->tune_tiles;
       double bt = 1e30;
       for (int gi = 0; gi < ngr; gi++)
         for (int v : cand) {
           c->tune_kch = v;
           if (ngr > 1) {
-            c->tune_groups = (gi & 1) ? 2 : 1;
+            c->tune_groups = (gi & 1) ? most : most / 2;
             c->tune_tiles = (gi & 2) ? 2 : 1;
             build_had_blocks(c);
           }

@@ -144,6 +144,8 @@ void launch_fft_up(const M2LDev& m, const DevTree& t, const int* src_node, int n
 constexpr int had_urows(int ntrg) { return ntrg <= 64 ? 18 : ntrg <= 128 ? 26 : 40; }
 constexpr int had_ucap(int ntrg) { return 16 * had_urows(ntrg); }
 constexpr int HAD_KCH = 16;    // largest default of the frequencies per workgroup (tunable per context)
+// Frequencies per workgroup of a launch over nblk blocks (kch <= 0: chosen).
+int had_frequencies(int nfreq, int nblk, int kch, bool split);
 struct HadBlocks {
   int nblk = 0, ntrg = 64;
   const int* trg = nullptr;

@@ -1301,15 +1301,16 @@ void launch_ifft_dn(const M2LDev& m, const DevTree& t, const int* trg_node, cons
 }
 
 // Frequencies per workgroup when not tuned: an even number up to HAD_KCH, such
-// that the workgroups fill the chip's slots (`resident` per CU) with the least
+// that the workgroups fill the chip's slots with the least
 // waste; a workgroup's start (index loads, first staging) costs about as
 // much as two frequencies.
-static int had_kch(const M2LDev& m, const HadBlocks& hb, int kch, int resident) {
+int had_frequencies(int nfreq, int nblk, int kch, bool split) {
   if (kch >= 1) return kch;
+  const int slots = 256 * (split ? 1 : 3);  // workgroups resident on the chip
   int best = 2;
   long cost = -1;
   for (int k = 2; k <= HAD_KCH; k += 2) {
-    const long wgs = long((m.nfreq + k - 1) / k) * hb.nblk, rounds = (wgs + 256 * resident - 1) / (256 * resident);
+    const long wgs = long((nfreq + k - 1) / k) * nblk, rounds = (wgs + slots - 1) / slots;
     const long c = rounds * (k + 2);
     if (cost < 0 || c <= cost) {
       cost = c;
@@ -1323,7 +1324,7 @@ void launch_hadamard(const M2LDev& m, const void* m2l_opsx, const float* hscale,
                      int tiles, hipStream_t s) {
   if (hb.nblk <= 0) return;
   const bool split = m.mixed && hscale && m.amax;
-  kch = had_kch(m, hb, kch, split ? 1 : 3);
+  kch = had_frequencies(m.nfreq, hb.nblk, kch, split);
   if (split) kch = (kch + 1) / 2 * 2;  // whole pairs of frequencies (nfreq is even)
   const int nchunk = (m.nfreq + kch - 1) / kch;
   dim3 grid(unsigned((nchunk + 7) / 8 * 8) * unsigned(hb.nblk));
@@ -1334,7 +1335,10 @@ void launch_hadamard(const M2LDev& m, const void* m2l_opsx, const float* hscale,
       hipLaunchKernelGGL(kern, grid, dim3(64 * nw), lds, s, m, static_cast<const h8*>(m2l_opsx), hscale, hb, nchunk,
                          kch);
     };
-    if (hb.ntrg == 128) {
+    if (hb.ntrg == 64) {
+      if (tiles >= 2) go(k_hadamard_h<2, 2>, 2);
+      else go(k_hadamard_h<4, 1>, 4);
+    } else if (hb.ntrg == 128) {
       if (tiles >= 2) go(k_hadamard_h<4, 2>, 4);
       else go(k_hadamard_h<8, 1>, 8);
     } else {

@@ -382,7 +382,8 @@ constexpr int npack() { return kcplx<KIND>() ? 5 : 4; }
 // on their way to LDS (subtracted in FP64, rounded once), padded with zero
 // charges to whole trips of the loop; the W waves take a part of every block each, the k lane groups every k-th source of it, two of them per trip,
 // and the sums are added in FP64 in a fixed order.  A tile of more than
-// t.p2p_split targets uses two lane groups at most.
+// t.p2p_split targets uses two lane groups at most; with t.p2p_split = 0 a single
+// wave sums a target's sources in one lane (W = M = 1).
 // Sources packed beforehand relative to their own leaf (half the bytes in FP32)
 // and shifted here cost FP32 two more roundings per coordinate, 5 to 7 times the
 // error of a pair across a leaf plane, and were no faster (2M points 1.18 ms
@@ -403,9 +404,9 @@ constexpr int npack() { return kcplx<KIND>() ? 5 : 4; }
 template <int KIND, typename R>
 constexpr int points_per_lane() { return kcplx<KIND>() && (sizeof(R) == 4 || KIND == HELMHOLTZ_REAL) ? 1 : 2; }
 
-template <int KIND, typename R, int W>
+template <int KIND, typename R, int W, int M = points_per_lane<KIND, R>()>
 __global__ __launch_bounds__(64 * W) void k_p2p(DevTree t, Wavek wk, const int* __restrict__ work) {
-  constexpr int NA = nval<KIND>(), NP = npack<KIND>(), M = points_per_lane<KIND, R>();
+  constexpr int NA = nval<KIND>(), NP = npack<KIND>();
   constexpr int CAP = 128 * W;  // sources in LDS
   constexpr int NE = 64;        // source leaves listed at a time
   constexpr int SZ = std::max(int(CAP * NP * sizeof(R)), int(W * NA * 64 * sizeof(double)));
@@ -415,7 +416,7 @@ __global__ __launch_bounds__(64 * W) void k_p2p(DevTree t, Wavek wk, const int* 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int leaf = work[2 * blockIdx.x], t0 = TILE * work[2 * blockIdx.x + 1];
   const int tb = t.trg_begin[leaf] + t0, nt = min(TILE, t.trg_count[leaf] - t0);
-  const int L = (nt + M - 1) / M, kmax = 64 / L, k = nt <= t.p2p_split ? kmax : min(kmax, 2);
+  const int L = (nt + M - 1) / M, kmax = 64 / L, k = nt <= t.p2p_split ? kmax : t.p2p_split > 0 ? min(kmax, 2) : 1;
   const int l = lane % L, ph = lane / L < k ? lane / L : 0;
   const double cx = t.center[3 * leaf], cy = t.center[3 * leaf + 1], cz = t.center[3 * leaf + 2];
   const R far = R(4.0 * t.r0 * ldexp(1.0, -t.level[leaf]));
@@ -892,15 +893,19 @@ static void eval_targets_t(int mode, const DevTree& t, Wavek k, const int* tiles
     else if (mode == MODE_M2P) hipLaunchKernelGGL((k_m2p<KIND, R, (w < 4 ? 4 : w)>), g, dim3(64 * (w < 4 ? 4 : w)), 0, s, t, k, tiles);
     else hipLaunchKernelGGL((k_l2p_smem<KIND, R, w>), g, b, 0, s, t, k, tiles);
   };
-  const int w = particle_waves<KIND>(ntiles);
+  // t.p2p_split = 0: nothing is split over lanes, of one wave or of several
+  const bool whole = t.p2p_split == 0 && mode != MODE_M2P;
+  const int w = whole ? 1 : particle_waves<KIND>(ntiles);
   // the FP64 near field of fewer than 1024 Helmholtz tiles, without the library's
   // sincos: 8 waves (512 tiles, before the error terms of sincos_near: 193 us with 4, 175 with 8)
   bool wide = false;
   if constexpr (KIND == HELMHOLTZ_REAL && sizeof(R) == 8) {
-    wide = mode == MODE_P2P && ntiles < 1024;
+    wide = mode == MODE_P2P && ntiles < 1024 && !whole;
     if (wide) go(std::integral_constant<int, 8>());
   }
   if (wide) {
+  } else if (whole && mode == MODE_P2P) {
+    hipLaunchKernelGGL((k_p2p<KIND, R, 1, 1>), dim3(ntiles), dim3(64), 0, s, t, k, tiles);
   } else if (w == 1) go(std::integral_constant<int, 1>());
   else if (w == 2) go(std::integral_constant<int, 2>());
   else if (w == 4 || KIND != LAPLACE) go(std::integral_constant<int, 4>());

@@ -182,18 +182,21 @@ int xfmm_set_value_scale(xfmm_context* ctx, const double* scale);
  *   XFMM_TUNE_HAD_KCH    frequencies per Hadamard workgroup, 1..256 (default:
  *                        chosen from the size of the problem, at most 16; the
  *                        split-FP16 kernel rounds it up to an even number)
- *   XFMM_TUNE_P2P_SPLIT  M2P / L2P tail tiles of at most this many targets
+ *   XFMM_TUNE_P2P_SPLIT  P2P / M2P / L2P tail tiles of at most this many targets
  *                        (0..32) split each target's sources over several
  *                        lanes; P2P tiles of more targets use two lanes a
- *                        target at most (default 32; the partial sums then
- *                        add in another order)
- *   XFMM_TUNE_HAD_GROUPS split-FP16 Hadamard (mixed / FLOAT): 128-target groups
- *                        per workgroup, 1 or 2 (4 is taken as 2), which share
- *                        the operators and the union of sources staged in LDS
- *                        for a frequency (default: 2 from 1024 targets on)
+ *                        target at most, and the waves of a tile share its
+ *                        sources (default 32; the partial sums then add in
+ *                        another order).  0: P2P and L2P sum all sources of a
+ *                        target in one lane, in the order of the lists
+ *   XFMM_TUNE_HAD_GROUPS split-FP16 Hadamard (mixed / FLOAT): 64-target groups
+ *                        per workgroup, 1, 2 or 4, which share the operators
+ *                        and the union of sources staged in LDS for a
+ *                        frequency (default: 4 from 1024 targets on, else 2)
  *   XFMM_TUNE_HAD_TILES  16-target tiles per wave, 1 or 2; a wave applies each
  *                        operator operand it reads to all of its tiles
  *                        (default: from the number of targets)
+ * xfmm_get_tuning gives what was set, else what the uploaded tree is run with.
  * Setting one drops a captured graph. */
 enum { XFMM_TUNE_HAD_KCH = 0, XFMM_TUNE_P2P_SPLIT = 1, XFMM_TUNE_HAD_GROUPS = 2, XFMM_TUNE_HAD_TILES = 3 };
 int xfmm_set_tuning(xfmm_context* ctx, int param, int value);
@@ -201,8 +204,8 @@ int xfmm_get_tuning(const xfmm_context* ctx, int param, int* value);
 
 /* Autotuner: on the uploaded tree and operators, times every candidate of
  * each tuning parameter (P2P split 0, 8, 16, 32 over the P2P + L2P kernels;
- * Hadamard chunk 4, 8, 16, 32, 64 times groups 1, 2 times tiles per wave 1, 2
- * over the Hadamard launches), fastest of `reps` runs each (1..100), and keeps the fastest.
+ * Hadamard chunk 4, 8, 16, 32, 64 times groups 1, 2 (2, 4 from 1024 targets on)
+ * times tiles per wave 1, 2 over the Hadamard launches), fastest of `reps` runs each (1..100), and keeps the fastest.
  * best_ms (may be NULL) receives the two best times.  Leaves no evaluation result behind (call the
  * passes again); drops a captured graph, so capture after tuning. */
 int xfmm_autotune(xfmm_context* ctx, int reps, double* best_ms);
