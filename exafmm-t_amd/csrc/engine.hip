@@ -595,7 +595,7 @@ void build_had_blocks(xfmm_context* c) {
     for (size_t jt = 0; jt < cur_t.size(); jt++) {
       const int node = c->h_m2l_trg[cur_t[jt]];
       const int* q = &c->h_lat[3 * size_t(node)];
-      // the cube's key: its position (10 bits of each coordinate tell the cubes of a block apart) and level
+      // the cube's key: its position (9 bits of each coordinate tell the cubes of a block apart) and level
       const int key = ((q[0] >> 2) & 511) | ((q[1] >> 2) & 511) << 9 | ((q[2] >> 2) & 511) << 18 | (c->h_level[node] & 15) << 27;
       size_t k = std::find(cubes.begin(), cubes.end(), key) - cubes.begin();
       if (k == cubes.size()) cubes.push_back(key);
@@ -1308,8 +1308,9 @@ int xfmm_downward_pass(xfmm_context* c) {
   return guarded(c, [&] {
     check_ready(c);
     // every value and check potential is stored by the first operator that
-    // reaches it: L2P (M2P where leaves have such lists), M2L and, for what M2L
-    // does not reach, the zero rows; the rest adds
+    // reaches it: values by L2P (cleared first where leaves have M2P lists, whose
+    // sums L2P then adds to), check potentials by M2L and, for what M2L does not
+    // reach, the zero rows; the rest adds
     const bool m2p = c->nt_m2p > 0, set = c->l2p_all && !m2p;
     if (!set) launch_zero(c->trg_value.ptr, c->trg_value.n, c->stream);
     record(c, 3);

@@ -137,30 +137,22 @@ __device__ __forceinline__ void fold_tile(R* acc, R* comp, const R* part) {
 
 constexpr int TILE = 64;
 
-// Sum the m (<= TILE) staged sources of a tile into part[], in source order,
-// four pairs per loop trip so that the LDS reads of a trip are issued together.
-template <int KIND, typename R, int RM, bool GRAD>
+// Sum the potentials of the m (<= TILE) staged sources of a tile into part[], in
+// source order, four pairs per loop trip so that the LDS reads of a trip are
+// issued together.
+template <int KIND, typename R, int RM>
 __device__ __forceinline__ void tile_sum(int m, const R* sx, const R* sy, const R* sz, const R* sq, const R* sqi, R tx,
-                                         R ty, R tz, R kr, R ki, R* part, R rmin2 = R(0)) {
+                                         R ty, R tz, R kr, R ki, R* part) {
   constexpr bool C = kcplx<KIND>();
   int j = 0;
   for (; j + 4 <= m; j += 4) {
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      if constexpr (GRAD)
-        pair_grad<KIND, R, RM>(sx[j + u] - tx, sy[j + u] - ty, sz[j + u] - tz, sq[j + u], C ? sqi[j + u] : R(0), kr, ki,
-                               part, rmin2);
-      else
-        pair_pot<KIND, R, RM>(sx[j + u] - tx, sy[j + u] - ty, sz[j + u] - tz, sq[j + u], C ? sqi[j + u] : R(0), kr, ki,
-                              part);
-    }
+    for (int u = 0; u < 4; u++)
+      pair_pot<KIND, R, RM>(sx[j + u] - tx, sy[j + u] - ty, sz[j + u] - tz, sq[j + u], C ? sqi[j + u] : R(0), kr, ki,
+                            part);
   }
-  for (; j < m; j++) {
-    if constexpr (GRAD)
-      pair_grad<KIND, R, RM>(sx[j] - tx, sy[j] - ty, sz[j] - tz, sq[j], C ? sqi[j] : R(0), kr, ki, part, rmin2);
-    else
-      pair_pot<KIND, R, RM>(sx[j] - tx, sy[j] - ty, sz[j] - tz, sq[j], C ? sqi[j] : R(0), kr, ki, part);
-  }
+  for (; j < m; j++)
+    pair_pot<KIND, R, RM>(sx[j] - tx, sy[j] - ty, sz[j] - tz, sq[j], C ? sqi[j] : R(0), kr, ki, part);
 }
 
 // Squared distance below which the FP32 near field of a leaf with itself
@@ -651,7 +643,7 @@ __global__ __launch_bounds__(64) void k_eval_surface(DevTree t, Wavek wk, const 
 #pragma unroll
         for (int a = 0; a < NA; a++) part[a] = 0;
         // check surfaces are well separated from the source particles
-        tile_sum<KIND, R, RSQ_SEP, false>(m, sx, sy, sz, sq, sqi, px, py, pz, kr, ki, part);
+        tile_sum<KIND, R, RSQ_SEP>(m, sx, sy, sz, sq, sqi, px, py, pz, kr, ki, part);
         fold_tile<R, NA>(acc, comp, part);
       }
     }
