@@ -189,19 +189,16 @@ __device__ __forceinline__ R soft_r2(const DevTree& t, int leaf) {
 // ---------------------------------------------- particle targets: P2P, M2P, L2P
 //
 // One workgroup of W waves per (leaf, tile of TILE targets), work[2 b] = leaf,
-// work[2 b + 1] = tile.  L2P and M2P: a full tile has a target per lane and reads its
-// sources as wave-uniform vectors (scalar loads from constant address space,
-// no LDS and no barriers); a tail tile of nt <= t.p2p_split (<= TILE / 2)
-// targets gives each target TILE / nt lanes (target lane % nt, phase lane /
-// nt) that take every (TILE / nt)-th source.  The W waves share the sources;
-// the partial sums of a target are added in FP64 through LDS in a fixed order.
-// Pairs are summed in chunks of 64 sources (plain sums, FP32 chunks combined
-// with Kahan summation).
+// work[2 b + 1] = tile.  In L2P and M2P a full tile has a target per lane; a tail
+// tile of nt <= t.p2p_split (<= TILE / 2) targets gives each target TILE / nt lanes
+// (target lane % nt, phase lane / nt) that take every (TILE / nt)-th source.  L2P
+// reads its sources as wave-uniform vectors (scalar loads from constant address
+// space, no LDS and no barriers), M2P and P2P stage theirs in LDS.  The W waves
+// share the sources; the partial sums of a target are added in FP64 through LDS in
+// a fixed order.  Pairs are summed in chunks of 64 sources (plain sums, FP32 chunks
+// combined with Kahan summation).
 // W (particle_waves): a wave per tile leaves a small tree's chip idle and its
-// longest tile is the time.  Near field, a wave per tile and W waves: Laplace
-// FP64, 64 leaves of 47 targets 119 and 29 us (16); Yukawa FP64, 1300
-// leaves of 15 193 and 73 (4); Helmholtz FP64, 512 leaves of 59 881 (a wave per
-// leaf) and 276 (4).
+// longest tile is the time.
 template <int KIND>
 constexpr int nval() { return kcplx<KIND>() ? 8 : 4; }  // values per target
 
@@ -372,27 +369,28 @@ constexpr int npack() { return kcplx<KIND>() ? 5 : 4; }
 // targets use 60 of 64 lanes (48 with one target in a lane).  The sources of
 // all leaves of the list are one sequence, moved into the target leaf's frame
 // on their way to LDS (subtracted in FP64, rounded once), padded with zero
-// charges to whole trips of the loop; the W waves take a part of every block each, the k lane groups every k-th source of it, two of them per trip,
-// and the sums are added in FP64 in a fixed order.  A tile of more than
-// t.p2p_split targets uses two lane groups at most; with t.p2p_split = 0 a single
-// wave sums a target's sources in one lane (W = M = 1).
+// charges to whole trips of the loop; the W waves take a part of every block
+// each, the k lane groups every k-th source of it, two of them per trip, and the
+// sums are added in FP64 in a fixed order.  A tile of more than t.p2p_split
+// targets uses two lane groups at most; with t.p2p_split = 0 a single wave sums a
+// target's sources in one lane (W = M = 1).
 // Sources packed beforehand relative to their own leaf (half the bytes in FP32)
 // and shifted here cost FP32 two more roundings per coordinate, 5 to 7 times the
 // error of a pair across a leaf plane, and were no faster (2M points 1.18 ms
 // either way; Helmholtz FP32, 4096 leaves of 49, 312 and 305 us).
 // Bound by the vector units: 14 instructions a pair (Laplace FP32).  Per source
-// leaf and tile instead (full tiles with a target per
-// lane and scalar loads, others with the lane groups reading each leaf from the
-// vector cache) the small leaves paid for remainders and for 16 lanes' worth
-// of cache reads a pair.  Before -> after: FP32, 32768 leaves of 30 targets 519
-// -> 465 us, of 61 1214 -> 1190; 38841 Plummer leaves of 15 478 -> 371; Yukawa FP32,
-// 15074 leaves of 20 220 -> 178; FP64, 12069 leaves of 41 1228 -> 1115; Helmholtz
-// FP64, 512 leaves of 59 268 -> 196 (223 with the library's sincos).  128 sources a wave: 256 and 512 cost 2 and 20
-// % (fewer workgroups on a CU); the next block loaded ahead gives nothing.
+// leaf and tile instead (full tiles with a target per lane and scalar loads,
+// others with the lane groups reading each leaf from the vector cache) the small
+// leaves paid for remainders and for 16 lanes' worth of cache reads a pair.  That
+// and this, us: FP32, 32768 leaves of 30 targets 519 and 475, of 61 1214 and 1200; 38841
+// Plummer leaves of 15 478 and 377; Yukawa FP32, 15074 leaves of 20 220 and 180; FP64,
+// 12069 leaves of 41 1228 and 1105; Helmholtz FP64, 512 leaves of 59 268 and 191.
+// 128 sources a wave: 256 cost up to 7 %, 512 up to 40 % (fewer workgroups on a
+// CU); the next block loaded ahead gives nothing.
 // M = 1 for Helmholtz where M = 2 costs waves by its registers (FP32, 4096 leaves
-// of 49: 312 and 327 us; FP64 with sincos_near, 122 and 138 registers: 196 and 207),
-// but not in FP64 with the library's sincos, whose branch wants pairs to overlap
-// (425 and 223).
+// of 49: 284 and 303 us; FP64 with sincos_near, 512 leaves of 59: 186 and 195), but
+// not in FP64 with the library's sincos, whose branch wants pairs to overlap (460
+// and 268).
 template <int KIND, typename R>
 constexpr int points_per_lane() { return kcplx<KIND>() && (sizeof(R) == 4 || KIND == HELMHOLTZ_REAL) ? 1 : 2; }
 
@@ -859,19 +857,23 @@ static bool real_phases(Wavek k, const DevTree& t) {
   return k.im == 0.0 && std::fabs(k.re) * 16.0 * t.r0 < 1073741824.0;
 }
 
-// Waves per tile: up to 4 while the tiles are fewer than 4 waves on each of the
-// chip's 1024 SIMDs (Helmholtz, whose pairs cost more: 16; near field of 4700 FP32
-// tiles with 1, 2, 4 waves 391, 349, 326 us), up to 16 for the few tiles of a
-// tiny tree.  More waves per tile than that only take slots from the
-// transforms beside the near field (Laplace FP64, 4096 tiles: the evaluation 917
-// us with a wave, 960 with four).  The kernels with FP64 exp or sin / cos stop
-// at 4: larger workgroups leave them too few registers (L2P of 512 Helmholtz
-// tiles 55, 81, 165 us with 4, 8, 16 waves).
+// Waves per tile: doubled up to 4 while the tiles times waves are fewer than 4096
+// (Helmholtz, whose pairs cost more: 16384).  Near field with 1, 2, 4 waves, us:
+//   Laplace FP64, 64 tiles of 47 targets 80, 45, 28 (8 and 16 waves: 26, 27, the same
+//     evaluation); 519 tiles of 46 85, 71, 43 (42, 59); FP32 75, 47, 32 (31, 49);
+//     64 tiles of 16: 4, 8, 16 waves 12, 14, 20;
+//   Yukawa FP64, 1015 tiles of 20 157, 83, 56; 3570 of 17 143, 101, 86;
+//   Helmholtz FP64, 64 tiles of 47 251, 134, 70; 623 of 59 324, 284, 205; 4161 of 49
+//     960, 857, 779; FP32, 4161 of 49 390, 314, 277.
+// Above the line more waves only take slots from the transforms beside the near
+// field.  The evaluation with 1, 2, 4 waves: Laplace, 4551 tiles, FP64 709, 713, 746
+// (FP32 478, 476, 453), 32768 tiles, FP32 1027, 1050, 1110; Yukawa, 15074 tiles, FP32
+// 1226, 1239, 1248; Helmholtz, 4161 tiles, FP64 1473, 1416, 1375, FP32 720, 680, 663,
+// 32891 tiles, FP32 2668, 2636, 2716.
 template <int KIND>
 static int particle_waves(int ntiles) {
   int w = 1;
   while (w < 4 && ntiles * w < (kcplx<KIND>() ? 16384 : 4096)) w *= 2;
-  while (KIND == LAPLACE && w < 16 && ntiles * w < 2048) w *= 2;
   return w;
 }
 
@@ -882,29 +884,23 @@ static void eval_targets_t(int mode, const DevTree& t, Wavek k, const int* tiles
     constexpr int w = decltype(W)::value;
     const dim3 g(ntiles), b(64 * w);
     if (mode == MODE_P2P) hipLaunchKernelGGL((k_p2p<KIND, R, w>), g, b, 0, s, t, k, tiles);
-    else if (mode == MODE_M2P) hipLaunchKernelGGL((k_m2p<KIND, R, (w < 4 ? 4 : w)>), g, dim3(64 * (w < 4 ? 4 : w)), 0, s, t, k, tiles);
+    else if (mode == MODE_M2P) hipLaunchKernelGGL((k_m2p<KIND, R, 4>), g, dim3(256), 0, s, t, k, tiles);
     else hipLaunchKernelGGL((k_l2p_smem<KIND, R, w>), g, b, 0, s, t, k, tiles);
   };
+  // the near field of few tiles: 8 waves in FP64 Helmholtz without the library's
+  // sincos (4 and 8 waves: 64 tiles 70 and 63 us, 623 tiles 205 and 178, 1869 tiles 207 and
+  // 201, 4161 tiles 779 and 793), else the 4 that particle_waves gives below 1024
+  constexpr int FEW = KIND == HELMHOLTZ_REAL && sizeof(R) == 8 ? 8 : 4;
   // t.p2p_split = 0: nothing is split over lanes, of one wave or of several
   const bool whole = t.p2p_split == 0 && mode != MODE_M2P;
   const int w = whole ? 1 : particle_waves<KIND>(ntiles);
-  // the FP64 near field of fewer than 1024 Helmholtz tiles, without the library's
-  // sincos: 8 waves (512 tiles, before the error terms of sincos_near: 193 us with 4, 175 with 8)
-  bool wide = false;
-  if constexpr (KIND == HELMHOLTZ_REAL && sizeof(R) == 8) {
-    wide = mode == MODE_P2P && ntiles < 1024 && !whole;
-    if (wide) go(std::integral_constant<int, 8>());
-  }
-  if (wide) {
-  } else if (whole && mode == MODE_P2P) {
+  if (whole && mode == MODE_P2P) {
     hipLaunchKernelGGL((k_p2p<KIND, R, 1, 1>), dim3(ntiles), dim3(64), 0, s, t, k, tiles);
+  } else if (mode == MODE_P2P && ntiles < 1024) {
+    hipLaunchKernelGGL((k_p2p<KIND, R, FEW>), dim3(ntiles), dim3(64 * FEW), 0, s, t, k, tiles);
   } else if (w == 1) go(std::integral_constant<int, 1>());
   else if (w == 2) go(std::integral_constant<int, 2>());
-  else if (w == 4 || KIND != LAPLACE) go(std::integral_constant<int, 4>());
-  else if constexpr (KIND == LAPLACE) {
-    if (w == 8) go(std::integral_constant<int, 8>());
-    else go(std::integral_constant<int, 16>());
-  }
+  else go(std::integral_constant<int, 4>());
   // FP32 near field: the near-coincident pairs in FP64 (same stream, after it)
   if constexpr (sizeof(R) == 4) {
     if (mode == MODE_P2P && t.nclose > 0 && t.close && t.close_off && t.close_coef)
