@@ -543,12 +543,16 @@ void launch_near(xfmm_context* c) {
   c->near_launched = true;
 }
 
-// Launch shape of the Hadamard.  Split FP16: blocks of 256 targets for 8 waves
-// of two tiles once there are 1024 targets (4680 targets at p = 10 1.08 ms, 128
-// targets for 8 waves of one tile 1.33), below that 128 targets, whose
-// workgroups are twice as many (584 targets at p = 8: 103 us, 114 with 256).  FP64 / FP32: 64
-// targets, two tiles per wave from 1024 targets on (1720 targets at p = 10
-// 1.73 ms, one tile 1.96; 584 targets at p = 8 451 and 384 us).
+// Launch shape of the Hadamard (us with each shape).  Split FP16: 256 targets for 8
+// waves of two tiles from 1024 targets on (4680 targets at p = 10 1180, 128 targets for 8
+// waves of one tile 1450; 2322 at p = 8 299 and 348), below that 128 targets, whose
+// workgroups are twice as many (Helmholtz, 584 targets over three levels, each with
+// blocks of its own, p = 6 91, 256 targets 97, p = 8 the evaluation 1166 and 1191; 279
+// Yukawa targets at p = 8 68 and 74; 72 Laplace targets 20 and 26.  584 Laplace targets,
+// one operator level, would rather have 256: 91 and 83).  64 targets for 4 waves are
+// never better (4680: 2480, 584: 164, 72: 37).  FP64 / FP32: 64 targets, two tiles per
+// wave from 1024 targets on (1720 targets at p = 8 939, one tile 1018; 584 targets 426
+// and 356).
 int had_groups(const xfmm_context* c) {
   if (c->tune_groups > 0) return c->tune_groups;
   return c->h_m2l_trg.size() >= 1024 ? 4 : 2;

@@ -192,7 +192,7 @@ int xfmm_set_value_scale(xfmm_context* ctx, const double* scale);
  *   XFMM_TUNE_HAD_GROUPS split-FP16 Hadamard (mixed / FLOAT): 64-target groups
  *                        per workgroup, 1, 2 or 4, which share the operators
  *                        and the union of sources staged in LDS for a
- *                        frequency (default: 4 from 1024 targets on, else 2)
+ *                        frequency (default: 4 from 1024 M2L targets on, else 2)
  *   XFMM_TUNE_HAD_TILES  16-target tiles per wave, 1 or 2; a wave applies each
  *                        operator operand it reads to all of its tiles
  *                        (default: from the number of targets)
