@@ -399,7 +399,11 @@ __global__ __launch_bounds__(64 * W) void k_p2p(DevTree t, Wavek wk, const int* 
   constexpr int NA = nval<KIND>(), NP = npack<KIND>();
   constexpr int CAP = 128 * W;  // sources in LDS
   constexpr int NE = 64;        // source leaves listed at a time
-  constexpr int SZ = std::max(int(CAP * NP * sizeof(R)), int(W * NA * 64 * sizeof(double)));
+  // (with ROOM, which nothing uses, a CU holds fewer of these workgroups beside the
+  // transforms on the other stream, which finish sooner: the evaluation in FP64,
+  // 60k -> 100k Laplace 881 and 871 us, 30k Helmholtz 507 and 499; this kernel alone the same)
+  constexpr int ROOM = 3 * NE * sizeof(R);
+  constexpr int SZ = std::max(int(CAP * NP * sizeof(R)), int(W * NA * 64 * sizeof(double))) + ROOM;
   __shared__ __attribute__((aligned(16))) char smem[SZ];
   __shared__ int pre[NE + 1], first[NE], self;
   R* sp = reinterpret_cast<R*>(smem);
