@@ -37,7 +37,7 @@ struct DevTree {
   const double* near_add = nullptr;   // L2P only (may be null): [ntrgs][4] values that the L2P kernels add to
                                       // each target's result after their own sum (the evaluation's near field)
   bool set_values = false;            // P2P / M2P / L2P store their values (else they add to trg_value)
-  int p2p_split = 32;                 // P2P / M2P / L2P: tail tiles of <= p2p_split targets (<= 32) split their sources over lanes
+  int p2p_split = 32;                 // P2P / M2P / L2P: tail tiles of <= p2p_split targets (<= 32) split their sources over lanes (0: P2P and L2P in one lane a target)
   const int* close = nullptr;         // near-coincident P2P pairs, [4] ints (target, source, target leaf, source leaf), sorted by target
   const int* close_off = nullptr;     // [nclose + 1]: pairs of the k-th target with any are close[close_off[k] .. close_off[k + 1])
   const double* close_coef = nullptr; // [pairs][4 or 8]: FP64 minus FP32 value of each pair per unit charge
